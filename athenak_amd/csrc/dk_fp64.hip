@@ -15,6 +15,7 @@
 #include <utility>
 
 #include "dk_internal.hpp"
+#include "dk_stencil.hpp"
 #include "dk_smr.hpp"
 
 using dk::Geo;
@@ -22,6 +23,10 @@ using dk::DevBlock;
 using dk::Idx;
 using dk::Dir;
 using dk::kBlock;
+using dk::HaloOK;
+using dk::InPad;
+using dk::MakeStencil;
+using dk::Stencil;
 
 namespace dk {
 
@@ -65,29 +70,6 @@ inline int Grid(long long n) {
   long long b = (n + kBlock - 1)/kBlock;
   if (b < 1) b = 1;
   return static_cast<int>(std::min<long long>(b, 65536));
-}
-
-struct Stencil {
-  int ip, jp, kp;
-  double wx[3], wy[3], wz[3];
-};
-
-__device__ inline void MakeStencil(const Geo &g, const DevBlock &b, double x, double y,
-                                   double z, Stencil &w) {
-  dk::PMWeights(x, b.x1min, b.x1max, g.nx1, g.is, g.deposit, w.ip, w.wx);
-  dk::PMWeights(y, b.x2min, b.x2max, g.nx2, g.js, g.deposit, w.jp, w.wy);
-  dk::PMWeights(z, b.x3min, b.x3max, g.nx3, g.ks, g.deposit, w.kp, w.wz);
-}
-
-__device__ inline bool HaloOK(const Geo &g, const Stencil &w) {   // dust_pm.cpp:241-242
-  return !(w.ip < (g.is-1) || w.ip > (g.is+g.nx1) || w.jp < (g.js-1) || w.jp > (g.js+g.nx2) ||
-           w.kp < (g.ks-1) || w.kp > (g.ks+g.nx3));
-}
-
-// a stencil footprint must lie inside the padded block (guards every gather/deposit)
-__device__ inline bool InPad(const Geo &g, const Stencil &w) {
-  return w.ip >= 1 && w.ip <= g.n1 - 2 && w.jp >= 1 && w.jp <= g.n2 - 2 && w.kp >= 1 &&
-         w.kp <= g.n3 - 2;
 }
 
 __device__ inline void AtomicAdd(double *p, double v) { unsafeAtomicAdd(p, v); }
@@ -1074,9 +1056,13 @@ int ApplyOperatorTo(dk_ctx *c, double *field, double *out, double a_dt, double s
   int e;
   if ((e = FillGhosts(c, field, 3, true, t))) return e;
   if ((e = dk::Zero(c, out, 3*dk::NCells(c)))) return e;
-  {const int _pt = dk::ProfBegin(c, "applya_gtsg");
-  k_applya_gtsg<<<PGRID>>>(c->g, c->d_blocks, PARGS, field, out, a_dt, sh, c->d_err);
-   dk::ProfEnd(c, _pt);}
+  if (dk::T64Use(c)) {
+    if ((e = dk::T64Oper(c, field, out, a_dt, sh))) return e;
+  } else {
+    const int _pt = dk::ProfBegin(c, "applya_gtsg");
+    k_applya_gtsg<<<PGRID>>>(c->g, c->d_blocks, PARGS, field, out, a_dt, sh, c->d_err);
+    dk::ProfEnd(c, _pt);
+  }
   if ((e = Fold(c, out, 3, t))) return e;
   {const int _pt = dk::ProfBegin(c, "applya_cell");
   k_applya_cell<<<CGRID(ActiveCells(c))>>>(c->g, c->u0, c->qdep, field, out, correct ? 1 : 0);
@@ -1653,6 +1639,7 @@ int dk_destroy(dk_ctx *c) {
   if (c == nullptr) return DK_OK;
   (void)hipStreamSynchronize(c->stream);
   if (c->fast) dk::FastDestroy(c);
+  dk::T64Destroy(c);
   for (auto &x : c->gexec)
     if (x) {(void)hipGraphExecDestroy(x); x = nullptr;}
   dk::ProfDestroy(c);
@@ -1675,7 +1662,7 @@ int dk_bind_particles(dk_ctx *c, double *rdata, int32_t *idata, int64_t capacity
     return DK_EINVAL;
   c->rdata = rdata; c->idata = idata; c->cap = capacity; c->np = npart;
   if (c->form == DK_FORM_FP32) return dk::FastBind(c);
-  return DK_OK;
+  return dk::T64Reserve(c);
 }
 
 int dk_bind_gas(dk_ctx *c, double *u0, double *u1) {
@@ -1725,6 +1712,7 @@ int dk_explicit_push(dk_ctx *c, const dk_stage *st) {
       if ((e = dk::CloudAdvance(c, st->dt))) return e;
       return Launched(c);
     }
+    if (dk::T64Use(c)) return dk::T64Advance(c, st->dt);
     {const int _pt = dk::ProfBegin(c, "pc2_advance");
     k_pc2_advance<<<PGRID>>>(c->g, c->d_blocks, PARGS, c->ustar, c->dmom, st->dt,
                              c->P.back_reaction, sbox, strat, qs, om, c->d_err);
@@ -1774,6 +1762,7 @@ int dk_deposit_drag(dk_ctx *c, const dk_stage *st) {
       if ((e = dk::CloudPredictor(c, st->dt, dk::StiffnessActive(c->P)))) return e;
       return Launched(c);
     }
+    if (dk::T64Use(c)) return dk::T64Predictor(c, st->dt, dk::StiffnessActive(c->P) ? 1 : 0);
     {const int _pt = dk::ProfBegin(c, "pc2_predictor");
     k_pc2_predictor<<<PGRID>>>(c->g, c->d_blocks, PARGS, c->u1, c->qdep, st->dt,
                                dk::StiffnessActive(c->P) ? 1 : 0, c->d_err);
@@ -1781,6 +1770,7 @@ int dk_deposit_drag(dk_ctx *c, const dk_stage *st) {
     return Launched(c);
   }
   if ((e = dk::Zero(c, c->qdep, 5*dk::NCells(c)))) return e;
+  if (dk::T64Use(c)) return dk::T64Scatter(c, DragStep(c, st), ImplicitShearShift(c, st));
   {const int _pt = dk::ProfBegin(c, "scatter_imex");
   k_scatter_imex<<<PGRID>>>(c->g, c->d_blocks, PARGS, c->qdep, DragStep(c, st),
                             ImplicitShearShift(c, st), c->d_err);
@@ -1797,21 +1787,11 @@ int dk_fold_deposit_qp(dk_ctx *c, const dk_stage *st) {
   return Fold(c, c->qdep, 5, st->time);
 }
 
-// src/dust/dust_pm.cpp:372-442, src/dust/dust_solver.cpp:630-724
-int dk_gas_implicit_solve(dk_ctx *c, const dk_stage *st) {
-  int e = Ready(c);
-  if (e || !ActiveStage(c, st)) return e;
-  if (c->P.coupling == DK_PC2) {
-    if (st->stage == 1 && c->P.back_reaction) {
-      if (dk::StiffnessActive(c->P) && (e = dk::StiffnessRecord<double>(c, c->qdep, 5, 4, st->dt))) return e;
-      {const int _pt = dk::ProfBegin(c, "pc2_apply_predictor");
-      k_pc2_apply_predictor<<<CGRID(ActiveCells(c))>>>(c->g, c->u0, c->qdep, c->P.pc2_damping,
-                                                       st->dt);
-       dk::ProfEnd(c, _pt);}
-      return Launched(c);
-    }
-    return DK_OK;
-  }
+namespace {
+
+// the imex solve of a stage (dust_solver.cpp:630-724)
+int ImexSolve(dk_ctx *c, const dk_stage *st) {
+  int e;
   const int br = c->P.back_reaction;
   {const int _pt = dk::ProfBegin(c, "local_guess");
   k_local_guess<<<CGRID(ActiveCells(c))>>>(c->g, c->u0, c->qdep, c->ustar, br);
@@ -1834,6 +1814,31 @@ int dk_gas_implicit_solve(dk_ctx *c, const dk_stage *st) {
   return DK_OK;
 }
 
+}  // namespace
+
+// src/dust/dust_pm.cpp:372-442, src/dust/dust_solver.cpp:630-724
+int dk_gas_implicit_solve(dk_ctx *c, const dk_stage *st) {
+  int e = Ready(c);
+  if (e || !ActiveStage(c, st)) return e;
+  if (c->P.coupling == DK_PC2) {
+    if (st->stage == 1 && c->P.back_reaction) {
+      if (dk::StiffnessActive(c->P) && (e = dk::StiffnessRecord<double>(c, c->qdep, 5, 4, st->dt))) return e;
+      {const int _pt = dk::ProfBegin(c, "pc2_apply_predictor");
+      k_pc2_apply_predictor<<<CGRID(ActiveCells(c))>>>(c->g, c->u0, c->qdep, c->P.pc2_damping,
+                                                       st->dt);
+       dk::ProfEnd(c, _pt);}
+      return Launched(c);
+    }
+    return DK_OK;
+  }
+  // (every operator pass of the solve uses one set of bins)
+  const bool hold = c->P.back_reaction && c->P.solver != DK_LOCAL && !dk::T64Held(c);
+  if (hold && (e = dk::T64Hold(c, ImplicitShearShift(c, st)))) return e;
+  e = ImexSolve(c, st);
+  if (hold) dk::T64Release(c);
+  return e;
+}
+
 // src/dust/dust_tasks.cpp:265-312
 int dk_fill_ustar(dk_ctx *c, const dk_stage *st) {
   int e = Ready(c, false);
@@ -1846,6 +1851,7 @@ int dk_gather_kick_pmbr(dk_ctx *c, const dk_stage *st) {
   int e = Ready(c);
   if (e || !ActiveStage(c, st) || c->P.coupling == DK_PC2) return e;
   if (c->P.back_reaction && (e = dk::Zero(c, c->dmom, 3*dk::NCells(c)))) return e;
+  if (dk::T64Use(c)) return dk::T64Kick(c, DragStep(c, st), ImplicitShearShift(c, st));
   {const int _pt = dk::ProfBegin(c, "gather_kick");
   k_gather_kick<<<PGRID>>>(c->g, c->d_blocks, PARGS, c->ustar, c->dmom, DragStep(c, st),
                            ImplicitShearShift(c, st), c->P.back_reaction, c->d_err);
@@ -1919,6 +1925,16 @@ int dk_fill_gas_ghosts(dk_ctx *c, const dk_stage *st) {
 
 namespace {
 
+// the deposit, the solve and the kick of a stage
+int ImexPasses(dk_ctx *c, const dk_stage *st) {
+  int e;
+  if ((e = dk_deposit_drag(c, st))) return e;
+  if ((e = dk_fold_deposit_qp(c, st))) return e;
+  if ((e = dk_gas_implicit_solve(c, st))) return e;
+  if ((e = dk_fill_ustar(c, st))) return e;
+  return dk_gather_kick_pmbr(c, st);
+}
+
 int StageBody(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
   if (c->form == DK_FORM_FP32) return dk::FastStage(c, st, src);
   int e;
@@ -1927,11 +1943,12 @@ int StageBody(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
   if ((e = dk_add_drag_history_gas(c, st))) return e;
   if ((e = dk_explicit_push(c, st))) return e;
   if ((e = dk_update_particle_gids(c, st))) return e;
-  if ((e = dk_deposit_drag(c, st))) return e;
-  if ((e = dk_fold_deposit_qp(c, st))) return e;
-  if ((e = dk_gas_implicit_solve(c, st))) return e;
-  if ((e = dk_fill_ustar(c, st))) return e;
-  if ((e = dk_gather_kick_pmbr(c, st))) return e;
+  // (the imex passes of the stage share one set of bins: nothing moves a particle between them)
+  const bool hold = c->P.coupling == DK_IMEX && ActiveStage(c, st);
+  if (hold && (e = dk::T64Hold(c, ImplicitShearShift(c, st)))) return e;
+  e = ImexPasses(c, st);
+  if (hold) dk::T64Release(c);
+  if (e) return e;
   if ((e = dk_fold_pmbr(c, st))) return e;
   if ((e = dk_apply_pmbr(c, st))) return e;
   if (ActiveStage(c, st) && (e = dk_fill_gas_ghosts(c, st))) return e;

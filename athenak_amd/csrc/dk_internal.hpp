@@ -149,6 +149,8 @@ struct dk_ctx {
   long long *d_block_off = nullptr;   // uneven set-ups: particle offsets of the blocks
   // the FP32 form (dk_fp32.hip)
   struct Fast *fast = nullptr;
+  // the plain form's tile passes (dk_tile64.hip); null: the per-particle kernels
+  struct Tile64 *t64 = nullptr;
   int graphs = 0;
   long long graph_launches = 0;    // stage graphs launched (dk_graph_launches)
   // RemoveOutflowParticles run totals (x3_outflow_mass, x3_outflow_count, dust.hpp); the ledger
@@ -174,6 +176,23 @@ int ProfBegin(dk_ctx *c, const char *label);
 bool ProfOn(const dk_ctx *c);
 void ProfEnd(dk_ctx *c, int token);
 void ProfDestroy(dk_ctx *c);
+
+// dk_tile64.hip: the particle-mesh passes of the plain FP64 form tile by tile.  Reserve sizes the
+// workspaces for the bound particles (called where particles are bound); Use tells whether the
+// passes run on them, else the per-particle kernels run.  A pass bins the particles by tile itself,
+// unless the caller holds bins that it built for the same positions (Hold ... Release, within one
+// call of the library: the particle arrays are the caller's between calls).
+int T64Reserve(dk_ctx *c);
+void T64Destroy(dk_ctx *c);
+bool T64Use(const dk_ctx *c);
+int T64Hold(dk_ctx *c, double sh);
+bool T64Held(const dk_ctx *c);
+void T64Release(dk_ctx *c);
+int T64Scatter(dk_ctx *c, double a_dt, double sh);
+int T64Oper(dk_ctx *c, const double *field, double *out, double a_dt, double sh);
+int T64Kick(dk_ctx *c, double a_dt, double sh);
+int T64Predictor(dk_ctx *c, double dt, int rate_dep);
+int T64Advance(dk_ctx *c, double dt);
 
 // dk_fp32.hip
 int FastCreate(dk_ctx *c);

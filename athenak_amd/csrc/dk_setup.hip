@@ -266,6 +266,7 @@ int dk_setup_problem(dk_ctx *c, const dk_setup *su) {
   int e = dk::Check(hipGetLastError());
   if (e) return e;
   c->np = a.ntot;
+  if ((e = dk::T64Reserve(c))) return e;
   dk_stage st;
   std::memset(&st, 0, sizeof(st));
   st.stage = 1; st.nexp_stages = 3;
