@@ -28,7 +28,6 @@ using dk::HatCDF;
 using dk::HatMoment;
 using dk::MakeCloudGeo;
 using dk::MinImage;
-using dk::SmrCloudForEach;
 using dk::Sq;
 
 namespace {
@@ -304,34 +303,56 @@ __global__ void __launch_bounds__(kBlock) k_cloud_advance(Geo g, const DevBlock 
   }
 }
 
+// a group of lanes per cloud on a statically refined mesh (dk_cloudwalk.hpp): the group's linear
+// gather (GatherLinear) from the packed field
+constexpr int kCoop = dk::kCoop;
+__device__ inline void CoopGather(const Geo &g, const dk::CoopCloud &cl, const dk::CoopLeaf *lf,
+                                  const double *gp, const double x[3], int lane, double u[3]) {
+  double s[3] = {0.0, 0.0, 0.0};
+  dk::CoopCells<true>(cl, lf, x, lane,
+      [&](const dk::CoopLeaf &L, int k, int j, int i, double w, double m1x, double m1y, double m1z) {
+        double cf[3];
+        dk::CoopLinear(L, k, j, i, w, m1x, m1y, m1z, x, cf);
+        const double *q = gp + (((((long long)L.b*g.n3 + k + g.ks)*g.n2 + j + g.js)*g.n1 + i +
+                                 g.is)*12);
+        for (int c=0; c<3; ++c)
+          s[c] += w*q[c] + cf[0]*q[3 + c] + cf[1]*q[6 + c] + cf[2]*q[9 + c];
+      });
+  for (int c=0; c<3; ++c) u[c] = dk::CoopSum(s[c]);
+}
+
 // CloudPredictorT on a statically refined mesh: the gather and the deposit over the leaves of
-// every level (the deposit walks the cloud again without moments: the same cells and weights in
-// the same order), each leaf cell with its own volume
+// every level (the deposit forms the weights again), each leaf cell with its own volume
 __global__ void __launch_bounds__(kBlock) k_smr_cloud_predictor(
     Geo g, const DevBlock *B, dk::SmrTree t, CloudGeo cg, const double *r, const int32_t *iv,
     long long cap, long long np, const double *gp, double *qdep, double dt, int rate_dep,
     dk::ErrWord *err) {
-  GRID_STRIDE(p, np) {
+  __shared__ dk::CoopLeaf leaves[kBlock/kCoop][8];
+  const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
+  dk::CoopLeaf *lf = leaves[grp];
+  for (long long p = (long long)blockIdx.x*(kBlock/kCoop) + grp; p < np;
+       p += (long long)gridDim.x*(kBlock/kCoop)) {
     const double x[3] = {PR(DK_IPX,p), PR(DK_IPY,p), PR(DK_IPZ,p)};
-    const int lev = PI(DK_PLEV,p);
-    double ug[3] = {0.0, 0.0, 0.0};
-    const bool ok = SmrCloudForEach<true>(g, B, t, cg, x, lev,
-        [&](int b, int k, int j, int i, double w, double m1x, double m1y, double m1z) {
-          GatherLinear(g, B[b], cg, gp, b, k, j, i, w, m1x, m1y, m1z, x, ug);
-        });
-    if (!ok) {dk::RecordError(err, DK_EHALO, p); continue;}
+    const dk::CoopCloud cl = dk::CoopSpans(g, B, t, cg, x, PI(DK_PLEV,p), lane, lf);
+    if (cl.total < 0) {
+      if (lane == 0) dk::RecordError(err, DK_EHALO, p);
+      continue;
+    }
+    double ug[3];
+    CoopGather(g, cl, lf, gp, x, lane, ug);
     const double mass_rate = PR(DK_IPM,p)/PR(DK_IPTS,p);
     const double gx = -dt*mass_rate*(ug[0] - PR(DK_IPVX,p));
     const double gy = -dt*mass_rate*(ug[1] - PR(DK_IPVY,p));
     const double gz = -dt*mass_rate*(ug[2] - PR(DK_IPVZ,p));
-    SmrCloudForEach<false>(g, B, t, cg, x, lev, [&](int b, int k, int j, int i, double w) {
-      const DevBlock &bb = B[b];
-      const double inv_volume = 1.0/(bb.dx1*bb.dx2*bb.dx3);
-      unsafeAtomicAdd(&qdep[Idx(g,b,5,1,k,j,i)], inv_volume*w*gx);
-      unsafeAtomicAdd(&qdep[Idx(g,b,5,2,k,j,i)], inv_volume*w*gy);
-      unsafeAtomicAdd(&qdep[Idx(g,b,5,3,k,j,i)], inv_volume*w*gz);
-      if (rate_dep) unsafeAtomicAdd(&qdep[Idx(g,b,5,4,k,j,i)], inv_volume*w*mass_rate);
-    });
+    dk::CoopCells<false>(cl, lf, x, lane,
+        [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
+          const double inv_volume = 1.0/(L.d[0]*L.d[1]*L.d[2]);
+          const long long i0 = Idx(g, L.b, 5, 1, k + g.ks, j + g.js, i + g.is);
+          unsafeAtomicAdd(&qdep[i0], inv_volume*w*gx);
+          unsafeAtomicAdd(&qdep[i0 + g.ncb], inv_volume*w*gy);
+          unsafeAtomicAdd(&qdep[i0 + 2*g.ncb], inv_volume*w*gz);
+          if (rate_dep) unsafeAtomicAdd(&qdep[i0 + 3*g.ncb], inv_volume*w*mass_rate);
+        });
   }
 }
 
@@ -340,46 +361,49 @@ __global__ void __launch_bounds__(kBlock) k_smr_cloud_advance(
     Geo g, const DevBlock *B, dk::SmrTree t, CloudGeo cg, double *r, const int32_t *iv,
     long long cap, long long np, const double *gp, double *dmom, double dt, int br,
     dk::ErrWord *err) {
-  GRID_STRIDE(p, np) {
+  __shared__ dk::CoopLeaf leaves[kBlock/kCoop][8];
+  const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
+  dk::CoopLeaf *lf = leaves[grp];
+  for (long long p = (long long)blockIdx.x*(kBlock/kCoop) + grp; p < np;
+       p += (long long)gridDim.x*(kBlock/kCoop)) {
     const double x0[3] = {PR(DK_IPX1,p), PR(DK_IPY1,p), PR(DK_IPZ1,p)};
     const double v0[3] = {PR(DK_IPVX1,p), PR(DK_IPVY1,p), PR(DK_IPVZ1,p)};
     double xh[3];
     xh[0] = x0[0] + 0.5*dt*v0[0];
     xh[1] = x0[1] + 0.5*dt*v0[1];
     xh[2] = x0[2] + 0.5*dt*v0[2];
-    const int lev = PI(DK_PLEV,p);
-    double ug[3] = {0.0, 0.0, 0.0};
-    const bool ok = SmrCloudForEach<true>(g, B, t, cg, xh, lev,
-        [&](int b, int k, int j, int i, double w, double m1x, double m1y, double m1z) {
-          GatherLinear(g, B[b], cg, gp, b, k, j, i, w, m1x, m1y, m1z, xh, ug);
-        });
-    if (!ok) {dk::RecordError(err, DK_EHALO, p); continue;}
-    const double h = 0.5*dt;
-    const double lambda = h/PR(DK_IPTS,p);
+    const dk::CoopCloud cl = dk::CoopSpans(g, B, t, cg, xh, PI(DK_PLEV,p), lane, lf);
+    if (cl.total < 0) {
+      if (lane == 0) dk::RecordError(err, DK_EHALO, p);
+      continue;
+    }
+    double ug[3];
+    CoopGather(g, cl, lf, gp, xh, lane, ug);
+    const double h = 0.5*dt, ts = PR(DK_IPTS,p);
+    const double lambda = h/ts;
     const double aa = 1.0 + lambda;
-    const double rr[3] = {v0[0] + lambda*ug[0], v0[1] + lambda*ug[1], v0[2] + lambda*ug[2]};
-    const double vh[3] = {rr[0]/aa, rr[1]/aa, rr[2]/aa};
-    PR(DK_IPVX,p) = 2.0*vh[0] - v0[0];
-    PR(DK_IPVY,p) = 2.0*vh[1] - v0[1];
-    PR(DK_IPVZ,p) = 2.0*vh[2] - v0[2];
-    PR(DK_IPX,p) = x0[0] + dt*vh[0];
-    PR(DK_IPY,p) = x0[1] + dt*vh[1];
-    PR(DK_IPZ,p) = x0[2] + dt*vh[2];
-    PR(DK_IPX1,p) = xh[0]; PR(DK_IPY1,p) = xh[1]; PR(DK_IPZ1,p) = xh[2];
-    const double ts = PR(DK_IPTS,p);
-    const double dvx = dt*(ug[0]-vh[0])/ts;
-    const double dvy = dt*(ug[1]-vh[1])/ts;
-    const double dvz = dt*(ug[2]-vh[2])/ts;
-    PR(DK_IPRX,p) = dvx; PR(DK_IPRY,p) = dvy; PR(DK_IPRZ,p) = dvz;
-    if (!br) continue;
+    double vh[3], dv[3];
+    for (int d=0; d<3; ++d) {
+      vh[d] = (v0[d] + lambda*ug[d])/aa;
+      dv[d] = dt*(ug[d] - vh[d])/ts;
+    }
     const double mass = -PR(DK_IPM,p);
-    SmrCloudForEach<false>(g, B, t, cg, xh, lev, [&](int b, int k, int j, int i, double w) {
-      const DevBlock &bb = B[b];
-      const double dw = mass*w/(bb.dx1*bb.dx2*bb.dx3);
-      unsafeAtomicAdd(&dmom[Idx(g,b,3,0,k,j,i)], dw*dvx);
-      unsafeAtomicAdd(&dmom[Idx(g,b,3,1,k,j,i)], dw*dvy);
-      unsafeAtomicAdd(&dmom[Idx(g,b,3,2,k,j,i)], dw*dvz);
-    });
+    // (the group's lanes read the particle together, before lane 0 writes it: one wavefront)
+    __builtin_amdgcn_wave_barrier();
+    if (lane == 0)
+      for (int d=0; d<3; ++d) {
+        PR(DK_IPVX+2*d,p) = 2.0*vh[d] - v0[d];
+        PR(DK_IPX+2*d,p) = x0[d] + dt*vh[d];
+        PR(DK_IPX1+2*d,p) = xh[d];
+        PR(DK_IPRX+d,p) = dv[d];
+      }
+    if (!br) continue;
+    dk::CoopCells<false>(cl, lf, xh, lane,
+        [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
+          const double dw = mass*w/(L.d[0]*L.d[1]*L.d[2]);
+          const long long i0 = Idx(g, L.b, 3, 0, k + g.ks, j + g.js, i + g.is);
+          for (int d=0; d<3; ++d) unsafeAtomicAdd(&dmom[i0 + d*g.ncb], dw*dv[d]);
+        });
   }
 }
 
@@ -403,7 +427,7 @@ int CloudPredictor(dk_ctx *c, double dt, int rate_dep) {
   if (c->np == 0) return Check(hipGetLastError());
   if (c->smr) {
     const int t = ProfBegin(c, "cloud_predictor");
-    k_smr_cloud_predictor<<<Grid(c->np), kBlock, 0, c->stream>>>(
+    k_smr_cloud_predictor<<<Grid(c->np*kCoop), kBlock, 0, c->stream>>>(
         g, c->d_blocks, c->tree, MakeCloudGeo(c), c->rdata, c->idata, (long long)c->cap,
         (long long)c->np, c->gpack, c->qdep, dt, rate_dep, c->d_err);
     ProfEnd(c, t);
@@ -426,7 +450,7 @@ int CloudAdvance(dk_ctx *c, double dt) {
   if (c->np == 0) return Check(hipGetLastError());
   if (c->smr) {
     const int t = ProfBegin(c, "cloud_advance");
-    k_smr_cloud_advance<<<Grid(c->np), kBlock, 0, c->stream>>>(
+    k_smr_cloud_advance<<<Grid(c->np*kCoop), kBlock, 0, c->stream>>>(
         g, c->d_blocks, c->tree, MakeCloudGeo(c), c->rdata, c->idata, (long long)c->cap,
         (long long)c->np, c->gpack, c->dmom, dt, c->P.back_reaction, c->d_err);
     ProfEnd(c, t);

@@ -2570,53 +2570,57 @@ k_pa(KArgs A, const float *us, float *scr, double *defect, const DevBlock *__res
 // (one wavefront per SIMD); a bound of 3 wavefronts per SIMD spills some of them and runs
 // C4's cross-level clouds 12 % faster (2 and 4: 11 % and 8 %).
 
-// LeafApi<LeafTraversal3D>::GatherLinear (src/dust/dust_leaf_api.hpp:202-220) from the FP32
-// 12-component pack of leaf b
-__device__ inline void GatherLinearF(const Geo &g, const DevBlock &b, const dk::CloudGeo &cg,
-                                     const float *gp, int m, int k, int j, int i, double w,
-                                     double m1x, double m1y, double m1z, const double x[3],
-                                     double u[3]) {
-  const double xc = b.x1min + (i - g.is + 0.5)*b.dx1;
-  const double yc = b.x2min + (j - g.js + 0.5)*b.dx2;
-  const double zc = b.x3min + (k - g.ks + 0.5)*b.dx3;
-  const double cx = 0.5*(m1x + dk::MinImage(x[0] - xc, cg.len[0])*w)/b.dx1;
-  const double cy = 0.5*(m1y + dk::MinImage(x[1] - yc, cg.len[1])*w)/b.dx2;
-  const double cz = 0.5*(m1z + dk::MinImage(x[2] - zc, cg.len[2])*w)/b.dx3;
+// a group of lanes per cross-level cloud of the list (dk_cloudwalk.hpp)
+constexpr int kCoop = dk::kCoop;
+
+// the group's linear gather (GatherLinear) from the FP32 12-component pack
+__device__ inline void CoopGatherF(const Geo &g, const dk::CoopCloud &cl, const dk::CoopLeaf *lf,
+                                   const float *gp, const double x[3], int lane, double u[3]) {
+  double s[3] = {0.0, 0.0, 0.0};
+  dk::CoopCells<true>(cl, lf, x, lane,
+      [&](const dk::CoopLeaf &L, int k, int j, int i, double w, double m1x, double m1y, double m1z) {
+        double cf[3];
+        dk::CoopLinear(L, k, j, i, w, m1x, m1y, m1z, x, cf);
+        const long long i0 = Idx(g, L.b, 12, 0, k + g.ks, j + g.js, i + g.is);
 #pragma unroll
-  for (int c=0; c<3; ++c)
-    u[c] += w*gp[Idx(g, m, 12, c, k, j, i)] + cx*gp[Idx(g, m, 12, 3 + c, k, j, i)] +
-            cy*gp[Idx(g, m, 12, 6 + c, k, j, i)] + cz*gp[Idx(g, m, 12, 9 + c, k, j, i)];
+        for (int c=0; c<3; ++c)
+          s[c] += w*gp[i0 + c*g.ncb] + cf[0]*gp[i0 + (3 + c)*g.ncb] +
+                  cf[1]*gp[i0 + (6 + c)*g.ncb] + cf[2]*gp[i0 + (9 + c)*g.ncb];
+      });
+  for (int c=0; c<3; ++c) u[c] = dk::CoopSum(s[c]);
 }
 
 // CloudPredictorT (src/dust/dust_cloud3d.cpp:1369-1437): the gather of the pack at x, the rate
 // and the impulse -dt rate (u - v) into qdep 0 and 1-3 (k_pp's values, per leaf cell volume)
-__global__ void __launch_bounds__(kBlock, 3) k_fxl_predictor(KArgs A, dk::CloudGeo cg,
+__global__ void __launch_bounds__(kBlock) k_fxl_predictor(KArgs A, dk::CloudGeo cg,
                                                           const float *gp, float *qdep) {
+  __shared__ dk::CoopLeaf leaves[kBlock/kCoop][8];
   const Geo &g = A.g;
   const int n = *A.xl_n;
-  for (int t = blockIdx.x*blockDim.x + threadIdx.x; t < n; t += gridDim.x*blockDim.x) {
+  const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
+  dk::CoopLeaf *lf = leaves[grp];
+  for (int t = blockIdx.x*(kBlock/kCoop) + grp; t < n; t += gridDim.x*(kBlock/kCoop)) {
     const int q = A.xl_list[t];
     const double x[3] = {A.dst.X(0, q), A.dst.X(1, q), A.dst.X(2, q)};
-    const float v[3] = {A.dst.V(0, q), A.dst.V(1, q), A.dst.V(2, q)};
-    const float ts = A.dst.TS(q), mass = A.dst.M(q);
     const int lev = A.plev[A.dst.ORIG(q)];
-    double ug[3] = {0.0, 0.0, 0.0};
-    const bool ok = dk::SmrCloudForEach<true>(g, A.B, A.tree, cg, x, lev,
-        [&](int b, int k, int j, int i, double w, double m1x, double m1y, double m1z) {
-          GatherLinearF(g, A.B[b], cg, gp, b, k, j, i, w, m1x, m1y, m1z, x, ug);
-        });
-    if (!ok) {dk::RecordError(A.err, DK_EHALO, q); continue;}
-    const double mrate = static_cast<double>(mass)/static_cast<double>(ts);
+    const dk::CoopCloud cl = dk::CoopSpans(g, A.B, A.tree, cg, x, lev, lane, lf);
+    if (cl.total < 0) {
+      if (lane == 0) dk::RecordError(A.err, DK_EHALO, q);
+      continue;
+    }
+    double ug[3];
+    CoopGatherF(g, cl, lf, gp, x, lane, ug);
+    const double mrate = static_cast<double>(A.dst.M(q))/static_cast<double>(A.dst.TS(q));
     double gi[3];
     for (int d=0; d<3; ++d) gi[d] = -A.dt*mrate*(static_cast<double>(static_cast<float>(ug[d])) -
-                                                 static_cast<double>(v[d]));
-    dk::SmrCloudForEach<false>(g, A.B, A.tree, cg, x, lev,
-        [&](int b, int k, int j, int i, double w) {
-          const double wv = w*A.B[b].ivol;
-          if (A.rate_dep)
-            unsafeAtomicAdd(&qdep[Idx(g, b, 4, 0, k, j, i)], static_cast<float>(wv*mrate));
+                                                 static_cast<double>(A.dst.V(d, q)));
+    dk::CoopCells<false>(cl, lf, x, lane,
+        [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
+          const double wv = w*A.B[L.b].ivol;
+          const long long i0 = Idx(g, L.b, 4, 0, k + g.ks, j + g.js, i + g.is);
+          if (A.rate_dep) unsafeAtomicAdd(&qdep[i0], static_cast<float>(wv*mrate));
           for (int d=0; d<3; ++d)
-            unsafeAtomicAdd(&qdep[Idx(g, b, 4, 1 + d, k, j, i)], static_cast<float>(wv*gi[d]));
+            unsafeAtomicAdd(&qdep[i0 + (1 + d)*g.ncb], static_cast<float>(wv*gi[d]));
         });
   }
 }
@@ -2624,26 +2628,29 @@ __global__ void __launch_bounds__(kBlock, 3) k_fxl_predictor(KArgs A, dk::CloudG
 // CloudAdvanceT (src/dust/dust_cloud3d.cpp:1449-1536) with CloudPC2Push (:118-158): the gather
 // of u* at the half-step position, k_pa's kick and drift, R and the impulse -m (v - v0) into
 // dmom (FP64, per leaf cell volume)
-__global__ void __launch_bounds__(kBlock, 3) k_fxl_advance(KArgs A, dk::CloudGeo cg,
+__global__ void __launch_bounds__(kBlock) k_fxl_advance(KArgs A, dk::CloudGeo cg,
                                                         const float *gp, double *dmom) {
+  __shared__ dk::CoopLeaf leaves[kBlock/kCoop][8];
   const Geo &g = A.g;
   const int n = *A.xl_n;
+  const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
+  dk::CoopLeaf *lf = leaves[grp];
   const float hf = static_cast<float>(0.5*A.dt);
-  for (int t = blockIdx.x*blockDim.x + threadIdx.x; t < n; t += gridDim.x*blockDim.x) {
+  for (int t = blockIdx.x*(kBlock/kCoop) + grp; t < n; t += gridDim.x*(kBlock/kCoop)) {
     const int q = A.xl_list[t];
     double x[3] = {A.dst.X(0, q), A.dst.X(1, q), A.dst.X(2, q)};
     float v[3] = {A.dst.V(0, q), A.dst.V(1, q), A.dst.V(2, q)};
-    const float ts = A.dst.TS(q), mass = A.dst.M(q);
     const int lev = A.plev[A.dst.ORIG(q)];
     double xh[3];
     Pc2Mid(A, x, v, xh);
-    double ug[3] = {0.0, 0.0, 0.0};
-    const bool ok = dk::SmrCloudForEach<true>(g, A.B, A.tree, cg, xh, lev,
-        [&](int b, int k, int j, int i, double w, double m1x, double m1y, double m1z) {
-          GatherLinearF(g, A.B[b], cg, gp, b, k, j, i, w, m1x, m1y, m1z, xh, ug);
-        });
-    if (!ok) {dk::RecordError(A.err, DK_EHALO, q); continue;}
-    const float lam = hf/ts;
+    const dk::CoopCloud cl = dk::CoopSpans(g, A.B, A.tree, cg, xh, lev, lane, lf);
+    if (cl.total < 0) {
+      if (lane == 0) dk::RecordError(A.err, DK_EHALO, q);
+      continue;
+    }
+    double ug[3];
+    CoopGatherF(g, cl, lf, gp, xh, lane, ug);
+    const float lam = hf/A.dst.TS(q);
     const float aa = 1.0f + lam;
     double dv[3];
     for (int d=0; d<3; ++d) {
@@ -2654,12 +2661,16 @@ __global__ void __launch_bounds__(kBlock, 3) k_fxl_advance(KArgs A, dk::CloudGeo
       v[d] = vn;
       dv[d] = static_cast<double>(vn) - static_cast<double>(vo);
     }
-    for (int d=0; d<3; ++d) {A.dst.X(d, q) = x[d]; A.dst.V(d, q) = v[d]; A.dst.R(d, q) = dv[d];}
-    const double fac = -static_cast<double>(mass);
-    dk::SmrCloudForEach<false>(g, A.B, A.tree, cg, xh, lev,
-        [&](int b, int k, int j, int i, double w) {
-          const double wv = fac*w*A.B[b].ivol;
-          for (int d=0; d<3; ++d) unsafeAtomicAdd(&dmom[Idx(g, b, 3, d, k, j, i)], wv*dv[d]);
+    const double fac = -static_cast<double>(A.dst.M(q));
+    // (the group's lanes read the particle together, before lane 0 writes it: one wavefront)
+    __builtin_amdgcn_wave_barrier();
+    if (lane == 0)
+      for (int d=0; d<3; ++d) {A.dst.X(d, q) = x[d]; A.dst.V(d, q) = v[d]; A.dst.R(d, q) = dv[d];}
+    dk::CoopCells<false>(cl, lf, xh, lane,
+        [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
+          const double wv = fac*w*A.B[L.b].ivol;
+          const long long i0 = Idx(g, L.b, 3, 0, k + g.ks, j + g.js, i + g.is);
+          for (int d=0; d<3; ++d) unsafeAtomicAdd(&dmom[i0 + d*g.ncb], wv*dv[d]);
         });
   }
 }
@@ -3890,7 +3901,7 @@ static int FastStagePc2(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
         g, T, f->scr_f, f->qdep, nullptr, f->item_start, f->ov_scr, f->ov_def)));
     if ((e = FoldT<float>(c, f->qdep, 4, st->time))) return e;
     if (c->smr)
-      TIMED("cloud_xlevel", (k_fxl_predictor<<<Grid(f->np), kBlock, 0, c->stream>>>(
+      TIMED("cloud_xlevel", (k_fxl_predictor<<<Grid(f->np*kCoop), kBlock, 0, c->stream>>>(
           A, dk::MakeCloudGeo(c), gf, f->qdep)));
     if (dk::StiffnessActive(c->P) && (e = StiffnessRecord<float>(c, f->qdep, 4, 0, st->dt))) return e;
     TIMED("pc2_apply", (k_pc2_apply<<<CellGrid(c), kBlock, 0, c->stream>>>(
@@ -3901,7 +3912,7 @@ static int FastStagePc2(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
         g, T, f->scr_f, f->dmom, f->defect, f->item_start, f->ov_scr, f->ov_def)));
     if ((e = FoldT<double>(c, f->dmom, 3, st->time))) return e;
     if (c->smr)
-      TIMED("cloud_xlevel", (k_fxl_advance<<<Grid(f->np), kBlock, 0, c->stream>>>(
+      TIMED("cloud_xlevel", (k_fxl_advance<<<Grid(f->np*kCoop), kBlock, 0, c->stream>>>(
           A, dk::MakeCloudGeo(c), gf, f->dmom)));
     TIMED("pc2_commit", (k_pc2_commit<<<CellGrid(c), kBlock, 0, c->stream>>>(
         g, c->u0, f->dmom, f->qdep, st->gam1[st->nexp_stages - 1])));
