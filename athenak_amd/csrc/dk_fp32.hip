@@ -257,6 +257,17 @@ __device__ inline int BlockOff(double x, double lo, double hi, double l) {
   return static_cast<int>((x - lo + l)/l) - 1;
 }
 
+// A position and its register across a periodic face, without branches: as an if / else the
+// compiler kept a loop-invariant number (the blocks per direction) over the branches in registers
+// that it saved in one of them only, under that branch's lane mask, so that the lanes of the other
+// branch went on with another number: a particle crossing a shear-periodic x1 face and the lower
+// x3 face in one stage was given the wrong block.  (The assembly of the key pass shows the copy;
+// whether the lanes held the right number from before depended on the registers' allocation.)
+__device__ inline void Wrap(bool lo, bool hi, double len, double &x, double &x1) {
+  x = lo ? x + len : (hi ? x - len : x);
+  x1 = lo ? x1 + len : (hi ? x1 - len : x1);
+}
+
 // VEL: also the new velocity (the key pass needs the position only).  b0: the particle's block
 // (s.gid) before the push, passed in so that a caller whose particles share one block reads it
 // once for all of them.  SMR: a refined mesh (the routing across levels, a separate
@@ -352,7 +363,7 @@ __device__ inline bool PushMigrate(const KArgs &A, const DevBlock &b0, PState &s
     if (ynew >= g.x2max) ynew -= lym;
     const double dy = ynew - s.x[1];
     s.x[1] = ynew; s.x1[1] += dy;
-    if (lo3) {s.x[2] += lzm; s.x1[2] += lzm;} else if (hi3) {s.x[2] -= lzm; s.x1[2] -= lzm;}
+    Wrap(lo3, hi3, lzm, s.x[2], s.x1[2]);
     int b2 = static_cast<int>(((s.x[1] - g.x2min)/lym)*static_cast<double>(g.nmbx2));
     b2 = (b2 < 0) ? 0 : ((b2 > g.nmbx2-1) ? (g.nmbx2-1) : b2);
     int b3 = static_cast<int>(((s.x[2] - g.x3min)/lzm)*static_cast<double>(g.nmbx3));
@@ -367,9 +378,9 @@ __device__ inline bool PushMigrate(const KArgs &A, const DevBlock &b0, PState &s
   else nb = b.nghbr[Dir(ix, iy, iz)];
   if (nb < 0) return false;
   s.gid = nb;
-  if (lo1) {s.x[0] += lxm; s.x1[0] += lxm;} else if (hi1) {s.x[0] -= lxm; s.x1[0] -= lxm;}
-  if (lo2) {s.x[1] += lym; s.x1[1] += lym;} else if (hi2) {s.x[1] -= lym; s.x1[1] -= lym;}
-  if (lo3) {s.x[2] += lzm; s.x1[2] += lzm;} else if (hi3) {s.x[2] -= lzm; s.x1[2] -= lzm;}
+  Wrap(lo1, hi1, lxm, s.x[0], s.x1[0]);
+  Wrap(lo2, hi2, lym, s.x[1], s.x1[1]);
+  Wrap(lo3, hi3, lzm, s.x[2], s.x1[2]);
   return true;
 }
 
@@ -427,9 +438,9 @@ __device__ inline bool Pc2Route(const KArgs &A, const DevBlock &b, PState &s, do
       ok = false;
     } else {
       s.gid = nb;
-      if ((ix < 0) && (b.face & 1)) s.x[0] += A.lxm; else if ((ix > 0) && (b.face & 2)) s.x[0] -= A.lxm;
-      if ((iy < 0) && (b.face & 4)) s.x[1] += A.lym; else if ((iy > 0) && (b.face & 8)) s.x[1] -= A.lym;
-      if ((iz < 0) && (b.face & 16)) s.x[2] += A.lzm; else if ((iz > 0) && (b.face & 32)) s.x[2] -= A.lzm;
+      Wrap((ix < 0) && (b.face & 1), (ix > 0) && (b.face & 2), A.lxm, s.x[0], s.x1[0]);
+      Wrap((iy < 0) && (b.face & 4), (iy > 0) && (b.face & 8), A.lym, s.x[1], s.x1[1]);
+      Wrap((iz < 0) && (b.face & 16), (iz > 0) && (b.face & 32), A.lzm, s.x[2], s.x1[2]);
       Pc2Mid(A, s.x, s.v, xh);
     }
   }
