@@ -518,11 +518,14 @@ __global__ void k_stiff_partial(Geo g, const T *q, int nv, int comp, const doubl
   if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
 }
 
-// chi = dt max, the running maximum and the rate maximum (rec[0..2]; dust_pm.cpp:315-331)
-__global__ void k_stiff_record(const double *partial, int nblk, double dt, double *rec) {
-  if (threadIdx.x != 0) return;
+// chi = dt max, the running maximum and the rate maximum (rec[0..2]; dust_pm.cpp:315-331): one
+// wavefront over the partials (one thread took 45 us for its 512 dependent loads)
+__global__ void __launch_bounds__(64) k_stiff_record(const double *partial, int nblk, double dt,
+                                                     double *rec) {
   double r = 0.0;
-  for (int b=0; b<nblk; ++b) r = fmax(r, partial[b]);
+  for (int b=threadIdx.x; b<nblk; b+=64) r = fmax(r, partial[b]);
+  for (int o=32; o>0; o>>=1) r = fmax(r, __shfl_xor(r, o, 64));
+  if (threadIdx.x != 0) return;
   const double chi = dt*r;
   rec[0] = chi;
   rec[1] = (rec[1] < chi) ? chi : rec[1];
