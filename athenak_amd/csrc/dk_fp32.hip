@@ -27,7 +27,6 @@
 // 500-564) -> consistent split (dust_pm.cpp:660-685).
 
 #include <hip/hip_runtime.h>
-#include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cmath>
@@ -48,8 +47,8 @@ using dk::kBlock;
 
 namespace {
 
-constexpr int kSegSmall = 32;       // lists longer than this are ordered by k_medsort
-constexpr int kMedMax = 512;        // lists longer than this are ordered by k_bigsort
+constexpr int kSegSmall = 32;       // lists longer than this are medium ones (k_longsort)
+constexpr int kMedMax = 512;        // lists longer than this are long ones (k_longsort)
 constexpr int kBigMax = 16384;      // longest list of one cell in the FP32 form
 constexpr int kPartRank = 8192;     // a stayer's rank: part*kPartRank + its rank in the part
 constexpr int kKeyThreads = 256;    // the key pass: one particle per thread per chunk (default)
@@ -106,22 +105,17 @@ struct Fast {
   int *stay = nullptr;              // per cell: the particles that stayed in its tile
   // [0], [1]: counts of medium and long lists; their cells from [2] up and from [1 + nkeys] down
   int *big = nullptr;
-  // work items (KArgs): parts per tile, their scan, the tile of every item; overflow slots
-  int *nparts = nullptr, *item_start = nullptr, *item_tile = nullptr;
+  // work items (KArgs): the tiles' first items, the tile of every item; overflow slots
+  int *item_start = nullptr, *item_tile = nullptr;
   long long item_cap = 0, ov_cap = 0;
-  void *iscan_tmp = nullptr;
-  size_t iscan_bytes = 0;
   float *ov_scr = nullptr, *ov_q = nullptr, *ov_pr = nullptr;
   double *ov_def = nullptr, *ov_dc = nullptr;
   int *ov_cnt = nullptr;
-  // shearing box: the items of the tiles inside a block's x2 range ([0]) and of the tiles on its
-  // x2 faces ([1]), in item order, their counts (ilist_n), and the scan that splits them
+  // the two item classes' lists in item order (shearing box: the tiles inside a block's x2 range
+  // and those on its x2 faces; else the tiles of one part and those of several), their counts
   int *ilist[2] = {nullptr, nullptr};
-  int *ilist_n = nullptr, *iflag = nullptr, *iflag_scan = nullptr;
-  void *lscan_tmp = nullptr;
-  size_t lscan_bytes = 0;
-  void *scan_tmp = nullptr;
-  size_t scan_bytes = 0;
+  int *ilist_n = nullptr;
+  int *scan_part = nullptr;         // the workgroups' sums of the key and item scans
   int32_t *itag = nullptr;          // caller's PTAG, PSP, PLEV, PTAGH by original index
   // fields, gas layout with ghosts
   float *qdep = nullptr;            // Q, P1, P2, P3
@@ -1561,57 +1555,100 @@ __global__ void __launch_bounds__(kX3Groups) k_x3sum(const double *part, double 
   if (threadIdx.x == 0) {ledger[0] += sm[0]; ledger[1] += sc[0];}
 }
 
-// the parts of every tile: at most W particles each, at least one (the entry after the last tile
-// is 0, for the scan)
-__global__ void k_nparts(Tiles Tl, const int *start, int W, int *nparts) {
-  GRID_STRIDE(t, (long long)Tl.nt + 1) {
-    if (t == Tl.nt) {nparts[t] = 0; continue;}
-    const long long k0 = t*(long long)Tl.TC;
-    const int n = start[k0 + Tl.TC] - start[k0];
-    nparts[t] = max(1, (n + W - 1)/W);
+// inclusive prefix sum over a workgroup of nw wavefronts (sh: nw ints, free before and after a
+// barrier); tot: the workgroup's sum
+__device__ inline int BlockScan(int v, int *sh, int nw, int &tot) {
+  const int w = threadIdx.x >> 6;
+  int a = WaveInclScan(v);
+  if ((threadIdx.x & 63) == 63) sh[w] = a;
+  __syncthreads();
+  tot = 0;
+  for (int q = 0; q < nw; ++q) {
+    if (q < w) a += sh[q];
+    tot += sh[q];
   }
+  __syncthreads();
+  return a;
 }
 
-// the tile of every work item
-__global__ void k_item_tile(Tiles Tl, const int *item_start, int *item_tile) {
-  GRID_STRIDE(t, (long long)Tl.nt) {
-    const int i0 = item_start[t], i1 = item_start[t + 1];
-    for (int i = i0; i < i1; ++i) item_tile[i] = static_cast<int>(t);
-  }
+// The work items of the present order: the parts of every tile (at most W particles each, at
+// least one), the tile of every item, and the two classes' lists in item order (class 1: in the
+// shearing box the tiles on a block's x2 faces, else the tiles of more than one part).  Two
+// launches over kItemTiles tiles a workgroup: the workgroups' sums, then each workgroup's prefix
+// of them and its own tiles; one launch when one workgroup holds every tile.  (Three scans of a
+// library and six kernels before: 12.6 -> 5 us at 256 tiles, where every launch is its latency.)
+constexpr int kItemThreads = 256, kItemPer = 4, kItemTiles = kItemThreads*kItemPer;
+__device__ inline int TileParts(const Tiles &Tl, const int *start, int W, int t, int &f) {
+  const long long k0 = t*(long long)Tl.TC;
+  const int n = max(1, (start[k0 + Tl.TC] - start[k0] + W - 1)/W);
+  f = Tl.SY ? (EdgeTile(Tl, t) ? 1 : 0) : ((n > 1) ? 1 : 0);
+  return n;
 }
-
-// the class of every item slot (1: a tile on a block's x2 face; 0 beyond the last item)
-// (multi: the items of tiles of more than one part, where crowded cells are, instead)
-__global__ void k_item_flags(Tiles Tl, const int *item_start, const int *item_tile, long long n,
-                             int *flag, int multi) {
-  const int nitem = item_start[Tl.nt];
-  GRID_STRIDE(i, n) {
-    int f = 0;
-    if (i < nitem) {
-      const int t = item_tile[i];
-      f = multi ? ((item_start[t + 1] - item_start[t] > 1) ? 1 : 0) : (EdgeTile(Tl, t) ? 1 : 0);
+__global__ void __launch_bounds__(kItemThreads)
+k_item_sums(Tiles Tl, const int *start, int W, int rounds, int *part) {
+  __shared__ int sh[kItemThreads/64];
+  const int base = blockIdx.x*rounds*kItemTiles;
+  int n = 0, n1 = 0;
+  for (int q = 0; q < rounds*kItemPer; ++q) {
+    const int t = base + q*kItemThreads + threadIdx.x;
+    if (t >= Tl.nt) break;
+    int f;
+    const int np = TileParts(Tl, start, W, t, f);
+    n += np;
+    n1 += f ? np : 0;
+  }
+  int tot, tot1;
+  BlockScan(n, sh, kItemThreads/64, tot);
+  BlockScan(n1, sh, kItemThreads/64, tot1);
+  if (threadIdx.x == 0) {part[2*blockIdx.x] = tot; part[2*blockIdx.x + 1] = tot1;}
+}
+__global__ void __launch_bounds__(kItemThreads)
+k_item_lists(Tiles Tl, const int *start, int W, int rounds, const int *part, int *item_start,
+             int *item_tile, int *list0, int *list1, int *count) {
+  __shared__ int sh[kItemThreads/64];
+  int b = 0, b1 = 0;   // items and class-1 items before this workgroup's tiles
+  {
+    int v = 0, v1 = 0;
+    for (int w = threadIdx.x; w < static_cast<int>(blockIdx.x); w += kItemThreads) {
+      v += part[2*w];
+      v1 += part[2*w + 1];
     }
-    flag[i] = f;
+    BlockScan(v, sh, kItemThreads/64, b);
+    BlockScan(v1, sh, kItemThreads/64, b1);
   }
-}
-
-// the two item lists in item order (e: the exclusive scan of the flags over n + 1 slots)
-__global__ void k_item_lists(Tiles Tl, const int *item_start, const int *flag, const int *e,
-                             long long n, int *list0, int *list1, int *count) {
-  const int nitem = item_start[Tl.nt];
-  GRID_STRIDE(i, (long long)nitem) {
-    if (flag[i]) list1[e[i]] = static_cast<int>(i);
-    else list0[i - e[i]] = static_cast<int>(i);
+  for (int q = 0; q < rounds; ++q) {
+    const int t0 = (blockIdx.x*rounds + q)*kItemTiles + threadIdx.x*kItemPer;
+    int n[kItemPer], f[kItemPer], sn = 0, s1 = 0;
+#pragma unroll
+    for (int k=0; k<kItemPer; ++k) {
+      n[k] = 0; f[k] = 0;
+      if (t0 + k < Tl.nt) n[k] = TileParts(Tl, start, W, t0 + k, f[k]);
+      sn += n[k];
+      s1 += f[k] ? n[k] : 0;
+    }
+    int tot, tot1;
+    int i = b + BlockScan(sn, sh, kItemThreads/64, tot) - sn;
+    int i1 = b1 + BlockScan(s1, sh, kItemThreads/64, tot1) - s1;
+#pragma unroll
+    for (int k=0; k<kItemPer; ++k) {
+      if (t0 + k >= Tl.nt) break;
+      item_start[t0 + k] = i;
+      for (int e=0; e<n[k]; ++e) {
+        item_tile[i + e] = t0 + k;
+        if (f[k]) list1[i1 + e] = i + e;
+        else list0[i - i1 + e] = i + e;
+      }
+      i += n[k];
+      i1 += f[k] ? n[k] : 0;
+    }
+    b += tot;
+    b1 += tot1;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    count[1] = e[n];
-    count[0] = nitem - e[n];
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+    item_start[Tl.nt] = b;
+    count[0] = b - b1;
+    count[1] = b1;
   }
-}
-
-// the count of every cell: the particles that stay in its tile plus the arrivals
-__global__ void k_total(int *count, const int *stay, long long nkeys) {
-  GRID_STRIDE(c, nkeys) count[c] += stay[c];
 }
 
 // placement: stayers first (part*kPartRank + their rank in the part: a later part's stayers after
@@ -1689,44 +1726,16 @@ __global__ void __launch_bounds__(kBlock) k_segsort(const int *start, const int 
   }
 }
 
-// one wavefront per medium list: an element's place is the count of smaller source slots in the
-// list (the slots are distinct), the list staged in LDS
-__global__ void __launch_bounds__(64) k_medsort(const int *start, const int *stay, int *perm,
-                                                 const int *big) {
-  constexpr int kPer = kMedMax/64;
-  __shared__ int sh[kMedMax];
-  const int nmed = big[0];
-  const int lane = threadIdx.x;
-  for (int e = blockIdx.x; e < nmed; e += gridDim.x) {
-    const int c = big[2 + e];
-    const int s0 = start[c] + stay[c], n = start[c + 1] - s0;
-    int v[kPer], r[kPer];
-#pragma unroll
-    for (int t=0; t<kPer; ++t) {
-      const int i = t*64 + lane;
-      v[t] = (i < n) ? perm[s0 + i] : INT_MAX;
-      r[t] = 0;
-      sh[i] = v[t];
-    }
-    __syncthreads();
-    for (int j=0; j<n; ++j) {
-      const int x = sh[j];
-#pragma unroll
-      for (int t=0; t<kPer; ++t) r[t] += (x < v[t]) ? 1 : 0;
-    }
-#pragma unroll
-    for (int t=0; t<kPer; ++t)
-      if (t*64 + lane < n) perm[s0 + r[t]] = v[t];
-    __syncthreads();
-  }
-}
-
-// one workgroup per long list: bitonic sort in LDS (padded to a power of two)
-__global__ void __launch_bounds__(1024) k_bigsort(const int *start, const int *stay, int *perm,
-                                                  const int *big, long long nkeys,
-                                                  dk::ErrWord *err) {
+// The medium and long lists of one launch.  A medium list: a wavefront each, an element's place is
+// the count of smaller source slots in the list (the slots are distinct), the list staged in LDS.
+// A long list: the workgroup sorts it in LDS by a bitonic network (padded to a power of two).
+// Every workgroup leaves at once when there are none.
+constexpr int kLongThreads = 1024;
+__global__ void __launch_bounds__(kLongThreads) k_longsort(const int *start, const int *stay,
+                                                           int *perm, const int *big,
+                                                           long long nkeys, dk::ErrWord *err) {
   __shared__ int sh[kBigMax];
-  const int nbig = big[1];
+  const int nmed = big[0], nbig = big[1];
   for (int e = blockIdx.x; e < nbig; e += gridDim.x) {
     const int c = big[1 + nkeys - e];
     const int s0 = start[c] + stay[c], n = start[c + 1] - s0;
@@ -1752,6 +1761,38 @@ __global__ void __launch_bounds__(1024) k_bigsort(const int *start, const int *s
       }
     }
     for (int i = threadIdx.x; i < n; i += blockDim.x) perm[s0 + i] = sh[i];
+    __syncthreads();
+  }
+  constexpr int kPer = kMedMax/64, kWaves = kLongThreads/64;
+  static_assert(kWaves*kMedMax <= kBigMax, "the wavefronts' lists fit the long list's LDS");
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int *mine = sh + wv*kMedMax;
+  // (the bound is the workgroup's: its wavefronts meet at the barriers)
+  for (int e0 = blockIdx.x*kWaves; e0 < nmed; e0 += gridDim.x*kWaves) {
+    const int e = e0 + wv;
+    int s0 = 0, n = 0;
+    if (e < nmed) {
+      const int c = big[2 + e];
+      s0 = start[c] + stay[c];
+      n = start[c + 1] - s0;
+    }
+    int v[kPer], r[kPer];
+#pragma unroll
+    for (int t=0; t<kPer; ++t) {
+      const int i = t*64 + lane;
+      v[t] = (i < n) ? perm[s0 + i] : INT_MAX;
+      r[t] = 0;
+      mine[i] = v[t];
+    }
+    __syncthreads();
+    for (int j=0; j<n; ++j) {
+      const int x = mine[j];
+#pragma unroll
+      for (int t=0; t<kPer; ++t) r[t] += (x < v[t]) ? 1 : 0;
+    }
+#pragma unroll
+    for (int t=0; t<kPer; ++t)
+      if (t*64 + lane < n) perm[s0 + r[t]] = v[t];
     __syncthreads();
   }
 }
@@ -2709,136 +2750,593 @@ __global__ void k_fix_qt(KArgs A, float *qt0, float *qt1, float *qt2) {
   }
 }
 
-// the push residues and dust corrections of a tile's later parts added in part order (as
-// k_fix_qt)
+// the push residues and dust corrections of a tile's later parts added in part order, and the
+// parts' counts of stayers made offsets: a thread per cell and momentum component, and one per
+// cell for the counts (every target has one writer: its own cell, the cell above, below).  Bound
+// by the chain of loads along a crowded tile's parts, which the four threads of a cell share.
 __global__ void k_fix_key(KArgs A, int do_key, double *pres) {
   const Geo &g = A.g;
   const Tiles &Tl = A.T;
   if (A.item_start[Tl.nt] == Tl.nt) return;   // every tile is one part
-  GRID_STRIDE(u, (long long)Tl.nt*Tl.TC) {
-    const int tile = static_cast<int>(u/Tl.TC), l = static_cast<int>(u - (long long)tile*Tl.TC);
+  const long long n = (long long)Tl.nt*Tl.TC;
+  GRID_STRIDE(u, 4*n) {
+    const int d = static_cast<int>(u/n);
+    const long long key = u - d*n;
+    const int tile = static_cast<int>(key/Tl.TC);
+    const int l = static_cast<int>(key - (long long)tile*Tl.TC);
     const int i0 = A.item_start[tile], np = A.item_start[tile + 1] - i0;
     if (np <= 1) continue;
+    if (d == 3) {
+      if (!do_key) continue;
+      // the stayers of each later part follow those of the parts before it: its count becomes
+      // its offset, and the cell's stay count the total
+      int base = A.stay[key];
+#pragma unroll 4
+      for (int p = 1; p < np; ++p) {
+        int &o = A.ov_cnt[((long long)i0 - tile + p - 1)*Tl.TC + l];
+        const int w = o;
+        o = base;
+        base += w;
+      }
+      A.stay[key] = base;
+      continue;
+    }
+    if (!A.cell_sums) continue;   // (pc2 sums neither: both are zero)
     const TileInfo t = TileOf(Tl, tile);
     int ci, cj, ck;
     CellIdx(Tl, t, l, ci, cj, ck);
-    const long long c = Idx(g, t.m, 3, 0, g.ks + ck, g.js + cj, g.is + ci);
+    const long long c = Idx(g, t.m, 3, d, g.ks + ck, g.js + cj, g.is + ci);
     // the later parts' shares in the key pass's form (own cell plus the tile neighbours' shares
     // for it in dc0, the tile's edge rows passing theirs on in dc1 / dc2), part by part
     const int row = (l >> Tl.LX) & (Tl.TY - 1);
-    for (int d=0; d<3; ++d) {
-      double pr = do_key ? pres[c + d*g.ncb] : 0.0;
-      double own = 0.0, up = 0.0, dn = 0.0;
+    double pr = do_key ? pres[c] : 0.0;
+    double own = 0.0, up = 0.0, dn = 0.0;
+    if (A.pending) {
+      own = A.dc0[c];
+      if (row == Tl.TY - 1) up = A.dc1[c + g.n1];
+      if (row == 0) dn = A.dc2[c - g.n1];
+    }
+#pragma unroll 4
+    for (int p = 1; p < np; ++p) {
+      const long long o = (long long)i0 - tile + p - 1;
+      if (do_key) pr += static_cast<double>(A.ov_pr[(o*3 + d)*Tl.TC + l]);
       if (A.pending) {
-        own = A.dc0[c + d*g.ncb];
-        if (row == Tl.TY - 1) up = A.dc1[c + g.n1 + d*g.ncb];
-        if (row == 0) dn = A.dc2[c - g.n1 + d*g.ncb];
-      }
-      for (int p = 1; p < np; ++p) {
-        const long long o = (long long)i0 - tile + p - 1;
-        if (do_key) pr += static_cast<double>(A.ov_pr[(o*3 + d)*Tl.TC + l]);
-        if (A.pending) {
-          const double *od = A.ov_dc + o*9*Tl.TC;
-          own += od[(3 + d)*Tl.TC + l];
-          if (row > 0) own += od[(6 + d)*Tl.TC + l - Tl.TX];
-          if (row < Tl.TY - 1) own += od[d*Tl.TC + l + Tl.TX];
-          if (row == Tl.TY - 1) up += od[(6 + d)*Tl.TC + l];
-          if (row == 0) dn += od[d*Tl.TC + l];
-        }
-      }
-      if (do_key) pres[c + d*g.ncb] = pr;
-      if (A.pending) {
-        A.dc0[c + d*g.ncb] = own;
-        if (row == Tl.TY - 1) A.dc1[c + g.n1 + d*g.ncb] = up;
-        if (row == 0) A.dc2[c - g.n1 + d*g.ncb] = dn;
+        const double *od = A.ov_dc + o*9*Tl.TC;
+        own += od[(3 + d)*Tl.TC + l];
+        if (row > 0) own += od[(6 + d)*Tl.TC + l - Tl.TX];
+        if (row < Tl.TY - 1) own += od[d*Tl.TC + l + Tl.TX];
+        if (row == Tl.TY - 1) up += od[(6 + d)*Tl.TC + l];
+        if (row == 0) dn += od[d*Tl.TC + l];
       }
     }
-    if (do_key) {
-      // the stayers of each later part follow those of the parts before it: its count becomes
-      // its offset, and the cell's stay count the total
-      const long long k = (long long)tile*Tl.TC + l;
-      int base = A.stay[k];
-      for (int p = 1; p < np; ++p) {
-        int &o = A.ov_cnt[((long long)i0 - tile + p - 1)*Tl.TC + l];
-        const int n = o;
-        o = base;
-        base += n;
-      }
-      A.stay[k] = base;
+    if (do_key) pres[c] = pr;
+    if (A.pending) {
+      A.dc0[c] = own;
+      if (row == Tl.TY - 1) A.dc1[c + g.n1] = up;
+      if (row == 0) A.dc2[c - g.n1] = dn;
     }
   }
 }
 
-// every padded cell sums the tile regions covering it, in ascending tile order and, within a tile,
-// in part order (the later parts' regions in their overflow slots) (grid: x over the cells of a
-// block, y over the blocks), in the output type TO; with defect, the first cell of every tile
-// then adds the tile's defects (NV values per tile and part) in part order
-template <typename T, int NV, typename TO = T>
-__global__ void k_combine(Geo g, Tiles Tl, const T *scr, TO *out, const double *defect,
-                          const int *item_start, const float *ov_scr, const double *ov_def) {
-  const int m = blockIdx.y;
-  const unsigned ncb = static_cast<unsigned>(g.ncb);
-  // (any tile of more than one part: only then are the overflow slots read)
-  const bool multi = item_start[Tl.nt] > Tl.nt;
-  for (unsigned rr = blockIdx.x*blockDim.x + threadIdx.x; rr < ncb;
-       rr += gridDim.x*blockDim.x) {
-    const unsigned t2 = rr/static_cast<unsigned>(g.n1);
-    const unsigned k_ = t2/static_cast<unsigned>(g.n2);
-    const int i = static_cast<int>(rr - t2*g.n1);
-    const int j = static_cast<int>(t2 - k_*g.n2);
-    const int k = static_cast<int>(k_);
-    // region coordinates relative to tile 0: r = (i - is + 1) - tx*TX etc.
-    const int ai = i - g.is + 1, aj = j - g.js + 1 + Tl.SY, ak = k - g.ks + 1;
-    TO sum[NV];
+// The cells' first slots in the new order: the exclusive scan of every cell's stayers plus
+// arrivals, in two launches over kScanKeys keys a workgroup and round: the workgroups' sums, then
+// each workgroup's prefix of them and its own keys.  The arrivals' counts and the long lists'
+// counters are left cleared for the next key pass.  (A fill, the sum of the two counts and a
+// library's scan before; both read each count once more than a look-back scan, 0.03 ms at 16.8
+// million keys.)
+constexpr int kScanThreads = 256, kScanPer = 16, kScanKeys = kScanThreads*kScanPer;
+constexpr int kScanGroups = 4096;   // at most this many workgroups: more keys take more rounds
+__global__ void __launch_bounds__(kScanThreads)
+k_key_sums(const int *count, const int *stay, long long nkeys, int rounds, int *part) {
+  __shared__ int sh[kScanThreads/64];
+  int n = 0;
+  for (int q = 0; q < rounds*(kScanPer/4); ++q) {
+    const long long c = (long long)blockIdx.x*rounds*kScanKeys +
+                        4*((long long)q*kScanThreads + threadIdx.x);
+    if (c + 4 <= nkeys) {   // (the arrays 256-aligned)
+      const int4 u = *reinterpret_cast<const int4*>(count + c);
+      const int4 v = *reinterpret_cast<const int4*>(stay + c);
+      n += u.x + v.x + u.y + v.y + u.z + v.z + u.w + v.w;
+    } else {
+      for (int k=0; k<4; ++k)
+        if (c + k < nkeys) n += count[c + k] + stay[c + k];
+    }
+  }
+  int tot;
+  BlockScan(n, sh, kScanThreads/64, tot);
+  if (threadIdx.x == 0) part[blockIdx.x] = tot;
+}
+__global__ void __launch_bounds__(kScanThreads)
+k_key_scan(int *count, const int *stay, long long nkeys, int rounds, const int *part, int *start,
+           int *big) {
+  __shared__ int sh[kScanThreads/64];
+  if (blockIdx.x == 0 && threadIdx.x < 2) big[threadIdx.x] = 0;
+  int b = 0;
+  {
+    int v = 0;
+    for (int w = threadIdx.x; w < static_cast<int>(blockIdx.x); w += kScanThreads) v += part[w];
+    BlockScan(v, sh, kScanThreads/64, b);
+  }
+  for (int q = 0; q < rounds; ++q) {
+    const long long c0 = ((long long)blockIdx.x*rounds + q)*kScanKeys +
+                         (long long)threadIdx.x*kScanPer;
+    int n[kScanPer], sn = 0;
+    if (c0 + kScanPer <= nkeys) {   // (16-byte loads: 16 keys a thread, the arrays 256-aligned)
 #pragma unroll
-    for (int v=0; v<NV; ++v) sum[v] = TO(0);
-    if (ai >= 0 && aj >= 0 && ak >= 0) {
-      // (arithmetic shifts: a negative lower bound clamps to 0 either way)
-      const int tz0 = max(0, (ak - Tl.RZ + Tl.TZ) >> Tl.LZ), tz1 = min(Tl.ntz - 1, ak >> Tl.LZ);
-      const int ty0 = max(0, (aj - Tl.RY + Tl.TY) >> Tl.LY), ty1 = min(Tl.nty - 1, aj >> Tl.LY);
-      const int tx0 = max(0, (ai - Tl.RX + Tl.TX) >> Tl.LX), tx1 = min(Tl.ntx - 1, ai >> Tl.LX);
-      for (int tz=tz0; tz<=tz1; ++tz) {
-        const int rz = ak - tz*Tl.TZ;
-        if (rz < 0 || rz >= Tl.RZ) continue;
-        for (int ty=ty0; ty<=ty1; ++ty) {
-          const int ry = aj - ty*Tl.TY;
-          if (ry < 0 || ry >= Tl.RY) continue;
-          for (int tx=tx0; tx<=tx1; ++tx) {
-            const int rx = ai - tx*Tl.TX;
-            if (rx < 0 || rx >= Tl.RX) continue;
-            const long long base = ScrRow(Tl, m, tz, ty, NV, 0, rz, ry) + tx*Tl.RX + rx;
-            const long long vstride = (long long)Tl.RZ*Tl.RY*Tl.ntx*Tl.RX;
-#pragma unroll
-            for (int v=0; v<NV; ++v) sum[v] += static_cast<TO>(scr[base + v*vstride]);
-            if (!multi) continue;
-            const int tile = (m*Tl.ntz + tz)*Tl.nty*Tl.ntx + ty*Tl.ntx + tx;
-            const int i0 = item_start[tile], np = item_start[tile + 1] - i0;
-            for (int p = 1; p < np; ++p) {
-              const float *o = ov_scr + ((long long)(i0 - tile + p - 1)*4*Tl.RN +
-                                         (rz*Tl.RY + ry)*Tl.RX + rx);
-#pragma unroll
-              for (int v=0; v<NV; ++v) sum[v] += static_cast<TO>(o[v*Tl.RN]);
-            }
-          }
-        }
+      for (int k=0; k<kScanPer; k+=4) {
+        const int4 u = *reinterpret_cast<const int4*>(count + c0 + k);
+        const int4 v = *reinterpret_cast<const int4*>(stay + c0 + k);
+        n[k] = u.x + v.x; n[k + 1] = u.y + v.y; n[k + 2] = u.z + v.z; n[k + 3] = u.w + v.w;
+        *reinterpret_cast<int4*>(count + c0 + k) = make_int4(0, 0, 0, 0);
       }
-      // the tile whose first cell this is (active cells only)
-      const int li = ai - 1, lj = aj - 1 - Tl.SY, lk = ak - 1;
-      if (defect != nullptr && li < Tl.ntx*Tl.TX && lj >= 0 && lj < Tl.nty*Tl.TY &&
-          lk < Tl.ntz*Tl.TZ && (li & (Tl.TX - 1)) == 0 && (lj & (Tl.TY - 1)) == 0 &&
-          (lk & (Tl.TZ - 1)) == 0 && li >= 0 && lk >= 0) {
-        const long long ct = (long long)m*Tl.ntb +
-                             ((lk >> Tl.LZ)*Tl.nty + (lj >> Tl.LY))*Tl.ntx + (li >> Tl.LX);
+    } else {
 #pragma unroll
-        for (int v=0; v<NV; ++v) sum[v] += defect[NV*ct + v];
-        const int i0 = item_start[ct], np = multi ? item_start[ct + 1] - i0 : 1;
-        for (int p = 1; p < np; ++p)
-#pragma unroll
-          for (int v=0; v<NV; ++v) sum[v] += ov_def[NV*((long long)i0 - ct + p - 1) + v];
+      for (int k=0; k<kScanPer; ++k) {
+        n[k] = 0;
+        if (c0 + k < nkeys) {n[k] = count[c0 + k] + stay[c0 + k]; count[c0 + k] = 0;}
       }
     }
 #pragma unroll
-    for (int v=0; v<NV; ++v) out[Idx(g,m,NV,v,k,j,i)] = sum[v];
+    for (int k=0; k<kScanPer; ++k) sn += n[k];
+    int tot;
+    int i = b + BlockScan(sn, sh, kScanThreads/64, tot) - sn;
+    if (c0 + kScanPer <= nkeys) {
+#pragma unroll
+      for (int k=0; k<kScanPer; k+=4) {
+        int4 v;
+        v.x = i; i += n[k];
+        v.y = i; i += n[k + 1];
+        v.z = i; i += n[k + 2];
+        v.w = i; i += n[k + 3];
+        *reinterpret_cast<int4*>(start + c0 + k) = v;
+      }
+    } else {
+#pragma unroll
+      for (int k=0; k<kScanPer; ++k)
+        if (c0 + k < nkeys) {start[c0 + k] = i; i += n[k];}
+    }
+    b += tot;
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) start[nkeys] = b;
+}
+
+// The tile regions' sum at one padded cell, in the output type TO: the regions covering it in
+// ascending tile order and, within a tile, in part order (the later parts' regions in their
+// overflow slots); with defect, the first cell of every tile then adds the tile's defects (NV
+// values per tile and part) in part order.
+struct Regions {
+  Geo g;
+  Tiles T;
+  const DevBlock *B;
+  const int *slot_dir;
+  const float *scr;
+  const int *item_start;
+  const float *ov_scr;
+  const double *defect, *ov_def;
+  int fold_x3;          // physical x3 faces: the ghost deposits fold back (not dropped)
+  int pairs;            // at most two tiles' regions cover a cell per axis (FoldedSum)
+  // the scratch (ScrRow) in words: a block, a component, the next tile in x2 and x3
+  long long sm;
+  int vs, sy, sz;
+};
+
+template <int NV, typename TO>
+__device__ inline void RegionSum(const Regions &R, bool multi, int m, int k, int j, int i,
+                                 TO sum[NV]) {
+  const Geo &g = R.g;
+  const Tiles &Tl = R.T;
+#pragma unroll
+  for (int v=0; v<NV; ++v) sum[v] = TO(0);
+  // region coordinates relative to tile 0: r = (i - is + 1) - tx*TX etc.
+  const int ai = i - g.is + 1, aj = j - g.js + 1 + Tl.SY, ak = k - g.ks + 1;
+  if (ai < 0 || aj < 0 || ak < 0) return;
+  // (arithmetic shifts: a negative lower bound clamps to 0 either way)
+  const int tz0 = max(0, (ak - Tl.RZ + Tl.TZ) >> Tl.LZ), tz1 = min(Tl.ntz - 1, ak >> Tl.LZ);
+  const int ty0 = max(0, (aj - Tl.RY + Tl.TY) >> Tl.LY), ty1 = min(Tl.nty - 1, aj >> Tl.LY);
+  const int tx0 = max(0, (ai - Tl.RX + Tl.TX) >> Tl.LX), tx1 = min(Tl.ntx - 1, ai >> Tl.LX);
+  for (int tz=tz0; tz<=tz1; ++tz) {
+    const int rz = ak - tz*Tl.TZ;
+    if (rz < 0 || rz >= Tl.RZ) continue;
+    for (int ty=ty0; ty<=ty1; ++ty) {
+      const int ry = aj - ty*Tl.TY;
+      if (ry < 0 || ry >= Tl.RY) continue;
+      for (int tx=tx0; tx<=tx1; ++tx) {
+        const int rx = ai - tx*Tl.TX;
+        if (rx < 0 || rx >= Tl.RX) continue;
+        const long long base = ScrRow(Tl, m, tz, ty, NV, 0, rz, ry) + tx*Tl.RX + rx;
+        const long long vstride = (long long)Tl.RZ*Tl.RY*Tl.ntx*Tl.RX;
+#pragma unroll
+        for (int v=0; v<NV; ++v) sum[v] += static_cast<TO>(R.scr[base + v*vstride]);
+        if (!multi) continue;
+        const int tile = (m*Tl.ntz + tz)*Tl.nty*Tl.ntx + ty*Tl.ntx + tx;
+        const int i0 = R.item_start[tile], np = R.item_start[tile + 1] - i0;
+        for (int p = 1; p < np; ++p) {
+          const float *o = R.ov_scr + ((long long)(i0 - tile + p - 1)*4*Tl.RN +
+                                       (rz*Tl.RY + ry)*Tl.RX + rx);
+#pragma unroll
+          for (int v=0; v<NV; ++v) sum[v] += static_cast<TO>(o[v*Tl.RN]);
+        }
+      }
+    }
+  }
+  // the tile whose first cell this is (active cells only)
+  const int li = ai - 1, lj = aj - 1 - Tl.SY, lk = ak - 1;
+  if (R.defect != nullptr && li < Tl.ntx*Tl.TX && lj >= 0 && lj < Tl.nty*Tl.TY &&
+      lk < Tl.ntz*Tl.TZ && (li & (Tl.TX - 1)) == 0 && (lj & (Tl.TY - 1)) == 0 &&
+      (lk & (Tl.TZ - 1)) == 0 && li >= 0 && lk >= 0) {
+    const long long ct = (long long)m*Tl.ntb +
+                         ((lk >> Tl.LZ)*Tl.nty + (lj >> Tl.LY))*Tl.ntx + (li >> Tl.LX);
+#pragma unroll
+    for (int v=0; v<NV; ++v) sum[v] += R.defect[NV*ct + v];
+    const int i0 = R.item_start[ct], np = multi ? R.item_start[ct + 1] - i0 : 1;
+    for (int p = 1; p < np; ++p)
+#pragma unroll
+      for (int v=0; v<NV; ++v) sum[v] += R.ov_def[NV*((long long)i0 - ct + p - 1) + v];
+  }
+}
+
+// the same with the ghost deposits beyond a physical x3 face mirrored into the block's first and
+// last layer (a region reaches one layer beyond; src/bvals/bvals_dep_general.cpp)
+template <int NV, typename TO>
+__device__ inline void RegionSumX3(const Regions &R, bool multi, int m, int k, int j, int i,
+                                   TO sum[NV]) {
+  const Geo &g = R.g;
+  RegionSum<NV, TO>(R, multi, m, k, j, i, sum);
+  if (!R.fold_x3 || (k != g.ks && k != g.ke)) return;
+  TO more[NV];
+  if (k == g.ks && R.B[m].nghbr[Dir(0, 0, -1)] < 0) {
+    RegionSum<NV, TO>(R, multi, m, k - 1, j, i, more);
+#pragma unroll
+    for (int v=0; v<NV; ++v) sum[v] += more[v];
+  }
+  if (k == g.ke && R.B[m].nghbr[Dir(0, 0, 1)] < 0) {
+    RegionSum<NV, TO>(R, multi, m, k + 1, j, i, more);
+#pragma unroll
+    for (int v=0; v<NV; ++v) sum[v] += more[v];
+  }
+}
+
+// The cell passes that follow a deposit, by what they do with the cell's folded sums.
+// the sums alone (refined meshes: the leaf walk adds to them; also the pc2 field that a later
+// pass reads)
+template <int NV, typename TO>
+struct CellStore {
+  TO *out;
+  __device__ void operator()(const Geo &g, int m, int k, int j, int i, const TO sum[NV]) const {
+#pragma unroll
+    for (int v=0; v<NV; ++v) out[Idx(g, m, NV, v, k, j, i)] = sum[v];
+  }
+};
+
+// One axis of an active cell (index l along it) in the tile grid: its own tile and the other tile
+// whose region reaches it (o: across the block's lower or upper face), each with the cell's place
+// in that region.  Slot 0 is the lower tile of the block, slot 1 the upper; of two tiles across a
+// face slot 0 is the cell's own.
+struct FoldAxis {
+  int off[2];     // the slot's offset in the scratch
+  int t[2];       // its tile index
+  bool two;
+  int o;
+};
+__device__ inline FoldAxis MakeFoldAxis(int l, int lt, int T, int nt, int h, int tstride,
+                                        int rstride) {
+  FoldAxis a;
+  const int tA = l >> lt, x = l & (T - 1);
+  const bool low = x < h, high = x >= T - h;
+  a.two = low || high;
+  const int tB = low ? tA - 1 : tA + 1;
+  a.o = !a.two ? 0 : ((tB < 0) ? -1 : ((tB >= nt) ? 1 : 0));
+  const int tb = (tB < 0) ? nt - 1 : ((tB >= nt) ? 0 : tB);
+  const int rA = x + h, rB = low ? rA + T : rA - T;
+  const int oA = tA*tstride + rA*rstride, oB = tb*tstride + rB*rstride;
+  const bool swap = low && a.o == 0;    // (the lower tile first)
+  a.off[0] = swap ? oB : oA;
+  a.off[1] = swap ? oA : oB;
+  a.t[0] = swap ? tb : tA;
+  a.t[1] = swap ? tA : tb;
+  return a;
+}
+
+// The folded sums at an active cell (indices li, lj, lk from 0), Tiles with R.pairs: the words of
+// the at most eight regions that hold the cell's deposits, in this block and across its faces,
+// loaded together, then added as the fold adds them: the block's own tiles in ascending order
+// (each with its later parts, then the defect), then every neighbour's sum in NeighborIndex order
+// (the crossed axes as bits x1, x2, x3: 1 to 7).  Beyond a physical x3 face the block's own ghost
+// layer takes the neighbour's place and is added to the sum it mirrors.  snb: the block's
+// neighbours by direction (< 0: none, -1: a physical face); EDGE: the cell may lie on a block face.
+template <int NV, typename TO, bool EDGE>
+__device__ inline void FoldedSum(const Regions &R, bool multi, const int *snb, int m, int li,
+                                 int lj, int lk, TO sum[NV]) {
+  const Tiles &Tl = R.T;
+  const int row = Tl.ntx*Tl.RX;
+  const FoldAxis ax = MakeFoldAxis(li, Tl.LX, Tl.TX, Tl.ntx, 1, Tl.RX, 1);
+  const FoldAxis ay = MakeFoldAxis(lj, Tl.LY, Tl.TY, Tl.nty, 1 + Tl.SY, R.sy, row);
+  FoldAxis az = MakeFoldAxis(lk, Tl.LZ, Tl.TZ, Tl.ntz, 1, R.sz, Tl.RY*row);
+  bool mirror = false;
+  if constexpr (EDGE) {
+    if (az.o != 0 && R.fold_x3 && snb[Dir(0, 0, az.o)] == -1) {
+      mirror = true;
+      az.t[1] = az.t[0];
+      az.off[1] = az.t[0]*R.sz + ((az.o < 0) ? 0 : Tl.RZ - 1)*Tl.RY*row;
+    }
+  }
+  const int cross = EDGE ? ((ax.o ? 1 : 0) | (ay.o ? 2 : 0) | (az.o ? 4 : 0)) : 0;
+  float val[8][NV];
+  int np[8];            // (multi) parts of the slot's tile, and its first item less the tile
+  long long ov[8];
+#pragma unroll
+  for (int q=0; q<8; ++q) {
+    bool ok = (!(q & 1) || ax.two) && (!(q & 2) || ay.two) && (!(q & 4) || az.two);
+    int nb = m;
+    if constexpr (EDGE) {
+      const int c = q & cross;
+      if (c != 0) {
+        const int d = Dir((c & 1) ? ax.o : 0, (c & 2) ? ay.o : 0, ((c & 4) && !mirror) ? az.o : 0);
+        if (d != 13) nb = snb[d];
+        ok = ok && nb >= 0;
+      }
+    }
+#pragma unroll
+    for (int v=0; v<NV; ++v) val[q][v] = 0.0f;
+    np[q] = 0;
+    ov[q] = 0;
+    if (ok) {
+      const float *p = R.scr + nb*R.sm + (ax.off[q & 1] + ay.off[(q >> 1) & 1] + az.off[q >> 2]);
+#pragma unroll
+      for (int v=0; v<NV; ++v) val[q][v] = p[v*R.vs];
+      if (multi) {
+        const int tile = ((nb*Tl.ntz + az.t[q >> 2])*Tl.nty + ay.t[(q >> 1) & 1])*Tl.ntx +
+                         ax.t[q & 1];
+        const int i0 = R.item_start[tile];
+        np[q] = R.item_start[tile + 1] - i0;
+        // (the cell's place in the region)
+        const int rx = ax.off[q & 1] - ax.t[q & 1]*Tl.RX;
+        const int ry = (ay.off[(q >> 1) & 1] - ay.t[(q >> 1) & 1]*R.sy)/row;
+        const int rz = (az.off[q >> 2] - az.t[q >> 2]*R.sz)/(Tl.RY*row);
+        ov[q] = (long long)(i0 - tile)*4*Tl.RN + (rz*Tl.RY + ry)*Tl.RX + rx;
+      }
+    }
+  }
+  // one slot's words, then its later parts'
+  const auto slot = [&](int q, TO sub[NV]) {
+#pragma unroll
+    for (int v=0; v<NV; ++v) sub[v] += static_cast<TO>(val[q][v]);
+    if (multi)
+      for (int p = 1; p < np[q]; ++p) {
+        const float *o = R.ov_scr + ov[q] + (long long)(p - 1)*4*Tl.RN;
+#pragma unroll
+        for (int v=0; v<NV; ++v) sub[v] += static_cast<TO>(o[v*Tl.RN]);
+      }
+  };
+#pragma unroll
+  for (int v=0; v<NV; ++v) sum[v] = TO(0);
+#pragma unroll
+  for (int q=0; q<8; ++q)
+    if (!EDGE || (q & cross) == 0) slot(q, sum);
+  if (R.defect != nullptr && (li & (Tl.TX - 1)) == 0 && (lj & (Tl.TY - 1)) == 0 &&
+      (lk & (Tl.TZ - 1)) == 0) {
+    const long long ct = (long long)m*Tl.ntb +
+                         ((lk >> Tl.LZ)*Tl.nty + (lj >> Tl.LY))*Tl.ntx + (li >> Tl.LX);
+#pragma unroll
+    for (int v=0; v<NV; ++v) sum[v] += R.defect[NV*ct + v];
+    const int i0 = R.item_start[ct], n = multi ? R.item_start[ct + 1] - i0 : 1;
+    for (int p = 1; p < n; ++p)
+#pragma unroll
+      for (int v=0; v<NV; ++v) sum[v] += R.ov_def[NV*((long long)i0 - ct + p - 1) + v];
+  }
+  if constexpr (EDGE) {
+    const auto group = [&](int c, TO sub[NV]) {
+#pragma unroll
+      for (int v=0; v<NV; ++v) sub[v] = TO(0);
+#pragma unroll
+      for (int q=0; q<8; ++q)
+        if ((q & cross) == c) slot(q, sub);
+    };
+    TO sub[NV], more[NV];
+    const int nxy = mirror ? 4 : 8;
+    for (int c = mirror ? 0 : 1; c < nxy; ++c) {
+      if ((c & ~cross) != 0) continue;
+      if (mirror) {
+        group(c | 4, more);
+        if (c == 0) {
+#pragma unroll
+          for (int v=0; v<NV; ++v) sum[v] += more[v];
+          continue;
+        }
+      }
+      group(c, sub);
+#pragma unroll
+      for (int v=0; v<NV; ++v) {
+        if (mirror) sub[v] += more[v];
+        sum[v] += sub[v];
+      }
+    }
+  }
+}
+
+// Combine, ghost fold and the cell pass in one launch: a thread per active cell adds the tile
+// regions at its cell, then op takes the sums.  The cells within a region's reach of a block face
+// (the shell) also add their neighbours' ghost cells that hold their deposits, each ghost cell's
+// own sum first and the neighbours in NeighborIndex order (src/mesh/nghbr_index.hpp:19-54); they
+// have workgroups of their own after those of the inner cells (in row order every wavefront would
+// hold a shell cell and wait for its look-ups: 1.5x the time at 256^3 cells).  The cells of a
+// shear-periodic x1 face leave their sums in out for k_fold_shear_cells, which adds what crosses
+// that face.  Bound by the regions' reads at large sizes and by latency at small ones, hence all
+// words of a cell loaded before the first is added (FoldedSum: 32^3 cells 20 -> 11 us).  (As three
+// kernels the padded field was written, folded in place and read again, and a shell cell made 26
+// dependent look-ups of which at most 7 count: 32^3 cells 23 us and the cell pass.)
+struct Shell {
+  int wx, wy, wz;            // layers of the shell at either end of each axis
+  unsigned inner, total;     // inner cells and all cells of a block
+  int inner_blocks;          // workgroups of the inner cells
+};
+inline Shell MakeShell(const Geo &g, int SY) {
+  Shell S;
+  S.wx = 1; S.wy = 1 + SY; S.wz = 1;
+  const long long ix = std::max(0, g.nx1 - 2*S.wx), iy = std::max(0, g.nx2 - 2*S.wy);
+  const long long iz = std::max(0, g.nx3 - 2*S.wz);
+  S.inner = static_cast<unsigned>(ix*iy*iz);
+  S.total = static_cast<unsigned>((long long)g.nx1*g.nx2*g.nx3);
+  S.inner_blocks = static_cast<int>((S.inner + kBlock - 1)/kBlock);
+  return S;
+}
+
+// the s-th shell cell (active indices): whole x3 layers, then x2 rows of the others, then the ends
+// of the remaining rows
+__device__ inline void ShellAt(const Geo &g, const Shell &S, unsigned s, int &i, int &j, int &k) {
+  const unsigned e1 = min(2*S.wx, g.nx1), e2 = min(2*S.wy, g.nx2), e3 = min(2*S.wz, g.nx3);
+  const unsigned plane = static_cast<unsigned>(g.nx2)*g.nx1, a = e3*plane;
+  const unsigned b = (g.nx3 - e3)*e2*g.nx1;
+  unsigned li, lj, lk;
+  if (s < a) {
+    const unsigned t = s/plane, r = s - t*plane;
+    lk = (t < static_cast<unsigned>(S.wz)) ? t : g.nx3 - e3 + t;
+    lj = r/g.nx1;
+    li = r - lj*g.nx1;
+  } else if (s < a + b) {
+    const unsigned r0 = s - a, rows = e2*g.nx1, t = r0/rows, r = r0 - t*rows, q = r/g.nx1;
+    lk = S.wz + t;
+    lj = (q < static_cast<unsigned>(S.wy)) ? q : g.nx2 - e2 + q;
+    li = r - q*g.nx1;
+  } else {
+    const unsigned r0 = s - a - b, row = (g.nx2 - e2)*e1, t = r0/row, r = r0 - t*row, q = r/e1;
+    const unsigned u = r - q*e1;
+    lk = S.wz + t;
+    lj = S.wy + q;
+    li = (u < static_cast<unsigned>(S.wx)) ? u : g.nx1 - e1 + u;
+  }
+  i = g.is + static_cast<int>(li); j = g.js + static_cast<int>(lj); k = g.ks + static_cast<int>(lk);
+}
+
+template <int NV, typename TO, class Op>
+__global__ void __launch_bounds__(kBlock) k_fold_cells(Regions R, Shell S, TO *out, int shear,
+                                                       Op op) {
+  __shared__ int snb[27];
+  const Geo &g = R.g;
+  const int m = blockIdx.y;
+  const bool multi = R.item_start[R.T.nt] > R.T.nt;
+  TO sum[NV];
+  if (static_cast<int>(blockIdx.x) < S.inner_blocks) {
+    const unsigned t = blockIdx.x*kBlock + threadIdx.x;
+    if (t >= S.inner) return;
+    const unsigned nx = g.nx1 - 2*S.wx, ny = g.nx2 - 2*S.wy, q = t/nx, kk = q/ny;
+    const int i = g.is + S.wx + static_cast<int>(t - q*nx);
+    const int j = g.js + S.wy + static_cast<int>(q - kk*ny);
+    const int k = g.ks + S.wz + static_cast<int>(kk);
+    if (R.pairs) FoldedSum<NV, TO, false>(R, multi, snb, m, i - g.is, j - g.js, k - g.ks, sum);
+    else RegionSum<NV, TO>(R, multi, m, k, j, i, sum);
+    op(g, m, k, j, i, sum);
+    return;
+  }
+  if (threadIdx.x < 27) {
+    // this block's neighbour in every direction (-1: a physical face; -2: another level, or a
+    // shear face)
+    const int d = threadIdx.x, o1 = d % 3;
+    const DevBlock &bm = R.B[m];
+    int nb = (d == 13) ? m : bm.nghbr[d];
+    if (nb >= 0 && R.B[nb].level != bm.level) nb = -2;
+    if (shear && ((o1 == 0 && bm.lx1 == 0) || (o1 == 2 && bm.lx1 == g.nmbx1 - 1))) nb = -2;
+    snb[d] = nb;
+  }
+  __syncthreads();
+  const unsigned t = (blockIdx.x - S.inner_blocks)*kBlock + threadIdx.x;
+  if (t >= S.total - S.inner) return;
+  int i, j, k;
+  ShellAt(g, S, t, i, j, k);
+  if (R.pairs) {
+    FoldedSum<NV, TO, true>(R, multi, snb, m, i - g.is, j - g.js, k - g.ks, sum);
+  } else {
+    // tiles of one or two cells along an axis: every neighbour's ghost cell on its own
+    RegionSumX3<NV, TO>(R, multi, m, k, j, i, sum);
+    // the offsets per axis whose ghost cells a region can reach: bit (o + 1)
+    const int a1 = 2 | ((i < g.is + S.wx) ? 1 : 0) | ((i > g.ie - S.wx) ? 4 : 0);
+    const int a2 = 2 | ((j < g.js + S.wy) ? 1 : 0) | ((j > g.je - S.wy) ? 4 : 0);
+    const int a3 = 2 | ((k < g.ks + S.wz) ? 1 : 0) | ((k > g.ke - S.wz) ? 4 : 0);
+    for (int s=0; s<26; ++s) {
+      const int d = R.slot_dir[s], o1 = d % 3, o2 = (d/3) % 3, o3 = d/9;
+      const int nb = snb[d];
+      if (!((a1 >> o1) & (a2 >> o2) & (a3 >> o3) & 1) || nb < 0) continue;
+      TO more[NV];
+      RegionSumX3<NV, TO>(R, multi, nb, k - (o3 - 1)*g.nx3, j - (o2 - 1)*g.nx2,
+                          i - (o1 - 1)*g.nx1, more);
+#pragma unroll
+      for (int v=0; v<NV; ++v) sum[v] += more[v];
+    }
+  }
+  if (shear && ((i == g.is && R.B[m].lx1 == 0) || (i == g.ie && R.B[m].lx1 == g.nmbx1 - 1))) {
+#pragma unroll
+    for (int v=0; v<NV; ++v) out[Idx(g, m, NV, v, k, j, i)] = sum[v];
+  } else {
+    op(g, m, k, j, i, sum);
+  }
+}
+
+// The cells of the shear-periodic x1 faces: the ghost deposits beyond the opposite face, moved in
+// x2 by shc cells and split between the two cells they overlap (src/bvals/bvals_dep_general.cpp:
+// 100-160, as a gather over the source cells that can reach the target: the order and the shares
+// of the fold of a padded field, dk_mesh.hip), then the cell pass.
+template <int NV, typename TO, class Op>
+__global__ void __launch_bounds__(kBlock) k_fold_shear_cells(Regions R, const TO *out, double shc,
+                                                             Op op) {
+  const Geo &g = R.g;
+  const bool multi = R.item_start[R.T.nt] > R.T.nt;
+  const int nface = g.nmbx2*g.nmbx3, ny = g.nx2*g.nmbx2;
+  const unsigned n = 2u*nface*g.nx3*g.nx2;
+  const bool perz = (g.bc_x3 == DK_X3_PERIODIC);
+  for (unsigned t = blockIdx.x*blockDim.x + threadIdx.x; t < n; t += gridDim.x*blockDim.x) {
+    unsigned r0 = t, q = r0/g.nx2;
+    const int jt = g.js + static_cast<int>(r0 - q*g.nx2);
+    r0 = q;
+    q = r0/g.nx3;
+    const int kt = g.ks + static_cast<int>(r0 - q*g.nx3);
+    r0 = q;
+    q = r0/nface;
+    const int f = static_cast<int>(r0 - q*nface), tside = static_cast<int>(q);
+    const int byt = f % g.nmbx2, bzt = f/g.nmbx2;
+    const int mt = ((tside == 0) ? 0 : g.nmbx1 - 1) + g.nmbx1*(byt + g.nmbx2*bzt);
+    const int it = (tside == 0) ? g.is : g.ie;
+    const int sside = 1 - tside, bxs = (sside == 0) ? 0 : g.nmbx1 - 1;
+    const int isrc = (sside == 0) ? (g.is - 1) : (g.ie + 1);
+    const double sh = (sside == 0) ? -shc : shc;
+    const int GJt = byt*g.nx2 + (jt - g.js), GKt = bzt*g.nx3 + (kt - g.ks);
+    int kb[3], kl[3];
+    const int kmask = dk::RowCopies(GKt, g.nx3, g.nmbx3, g.ng, g.ks, perz, kb, kl);
+    const int d0 = (ny < 5) ? 0 : 1, d1 = (ny < 5) ? ny : 3;
+    const int base = GJt - static_cast<int>(floor(sh)) - 2;
+    TO sum[NV];
+#pragma unroll
+    for (int v=0; v<NV; ++v) sum[v] = out[Idx(g, mt, NV, v, kt, jt, it)];
+    for (int kq=0; kq<3; ++kq) {
+      if (!((kmask >> kq) & 1)) continue;
+      const int kbq = (kq == 0) ? kb[0] : ((kq == 1) ? kb[1] : kb[2]);
+      const int klq = (kq == 0) ? kl[0] : ((kq == 1) ? kl[1] : kl[2]);
+      for (int d=d0; d<d1; ++d) {
+        const int r = (((base + d) % ny) + ny) % ny;
+        int jb[3], jl[3];
+        const int jmask = dk::RowCopies(r, g.nx2, g.nmbx2, g.ng, g.js, true, jb, jl);
+        for (int p=0; p<3; ++p) {
+          if (!((jmask >> p) & 1)) continue;
+          const int jbp = (p == 0) ? jb[0] : ((p == 1) ? jb[1] : jb[2]);
+          const int jlp = (p == 0) ? jl[0] : ((p == 1) ? jl[1] : jl[2]);
+          const int ms = bxs + g.nmbx1*(jbp + g.nmbx2*kbq);
+          const int gj = jbp*g.nx2 + (jlp - g.js);    // the source's unwrapped row
+          const double lo = gj + sh;
+          const int c0 = static_cast<int>(floor(lo));
+          const double fr = lo - c0;
+          const bool first = (((c0 % ny) + ny) % ny) == GJt && (1.0 - fr) > 0.0;
+          const bool second = ((((c0 + 1) % ny) + ny) % ny) == GJt && fr > 0.0;
+          if (!first && !second) continue;
+          TO val[NV];
+          RegionSumX3<NV, TO>(R, multi, ms, klq, jlp, isrc, val);
+#pragma unroll
+          for (int v=0; v<NV; ++v) {
+            if (first) sum[v] += static_cast<TO>(1.0 - fr)*val[v];
+            if (second) sum[v] += static_cast<TO>(fr)*val[v];
+          }
+        }
+      }
+    }
+    op(g, mt, kt, jt, it, sum);
   }
 }
 
@@ -2962,70 +3460,95 @@ __global__ void k_fpack(Geo g, const float *vel, float *gp) {
 
 // pc2 apply-predictor (dust_pm.cpp:387-402): with damping, the cells where chi = dt rate/rho
 // exceeds 1 scale their g by 1/chi (kept: the commit removes the same values); u0 += g
-__global__ void k_pc2_apply(Geo g, double *u0, float *qd, int damp, double dt) {
-  BLOCK_CELLS(m, k, j, i)
-    float q[3];
-    for (int c=0; c<3; ++c) q[c] = qd[Idx(g,m,4,1+c,k,j,i)];
+struct CellPc2Apply {
+  double *u0;
+  float *qd;
+  int damp;
+  double dt;
+  __device__ void operator()(const Geo &g, int m, int k, int j, int i, const float sum[4]) const {
+    float q[3] = {sum[1], sum[2], sum[3]};
     if (damp) {
-      const double chi = dt*static_cast<double>(qd[Idx(g,m,4,0,k,j,i)])/
-                         u0[Idx(g,m,DK_NGAS,DK_IDN,k,j,i)];
+      const double chi = dt*static_cast<double>(sum[0])/u0[Idx(g,m,DK_NGAS,DK_IDN,k,j,i)];
       if (chi > 1.0) {
         const double sc = 1.0/chi;
-        for (int c=0; c<3; ++c) {
-          q[c] = static_cast<float>(static_cast<double>(q[c])*sc);
-          qd[Idx(g,m,4,1+c,k,j,i)] = q[c];
-        }
+        for (int c=0; c<3; ++c) q[c] = static_cast<float>(static_cast<double>(q[c])*sc);
       }
     }
-    for (int c=0; c<3; ++c) u0[Idx(g,m,DK_NGAS,DK_IM1+c,k,j,i)] += static_cast<double>(q[c]);
+    qd[Idx(g,m,4,0,k,j,i)] = sum[0];
+    for (int c=0; c<3; ++c) {
+      qd[Idx(g,m,4,1+c,k,j,i)] = q[c];
+      u0[Idx(g,m,DK_NGAS,DK_IM1+c,k,j,i)] += static_cast<double>(q[c]);
+    }
   }
-}
+};
 
 // pc2 commit (dust_pm.cpp:596-601): u0 += dmom - gam1 g (the predictor's share of the stage
 // combination taken back, the actual impulse given)
-__global__ void k_pc2_commit(Geo g, double *u0, const double *dmom, const float *qd,
-                             double gam1) {
-  BLOCK_CELLS(m, k, j, i)
+struct CellPc2Commit {
+  double *u0;
+  const float *qd;
+  double gam1;
+  __device__ void operator()(const Geo &g, int m, int k, int j, int i, const double sum[3]) const {
     for (int c=0; c<3; ++c)
       u0[Idx(g,m,DK_NGAS,DK_IM1+c,k,j,i)] +=
-          dmom[Idx(g,m,3,c,k,j,i)] - gam1*static_cast<double>(qd[Idx(g,m,4,1+c,k,j,i)]);
+          sum[c] - gam1*static_cast<double>(qd[Idx(g,m,4,1+c,k,j,i)]);
+  }
+};
+
+// a cell pass over fields that hold the folded sums (refined meshes, after the leaf walk)
+template <int NV, typename TO, class Op>
+__global__ void __launch_bounds__(kBlock) k_cells(Geo g, const TO *in, Op op) {
+  BLOCK_CELLS(m, k, j, i)
+    TO sum[NV];
+    for (int v=0; v<NV; ++v) sum[v] = in[Idx(g, m, NV, v, k, j, i)];
+    op(g, m, k, j, i, sum);
   }
 }
 
-// the local guess u* = (M + P)/(rho + Q) (dust_solver.cpp:643-649)
-__global__ void k_guess(Geo g, const double *u0, const float *qd, float *us) {
-  BLOCK_CELLS(m, k, j, i)
-    const double pinv = 1.0/(u0[Idx(g,m,DK_NGAS,DK_IDN,k,j,i)] +
-                             static_cast<double>(qd[Idx(g,m,4,0,k,j,i)]));
-    for (int c=0; c<3; ++c)
+// the local guess u* = (M + P)/(rho + Q) (dust_solver.cpp:643-649); Q and P are kept
+struct CellGuess {
+  const double *u0;
+  float *qd, *us;
+  __device__ void operator()(const Geo &g, int m, int k, int j, int i, const float sum[4]) const {
+    const double pinv = 1.0/(u0[Idx(g,m,DK_NGAS,DK_IDN,k,j,i)] + static_cast<double>(sum[0]));
+    qd[Idx(g,m,4,0,k,j,i)] = sum[0];
+    for (int c=0; c<3; ++c) {
+      qd[Idx(g,m,4,1+c,k,j,i)] = sum[1+c];
       us[Idx(g,m,3,c,k,j,i)] = static_cast<float>(
-          (u0[Idx(g,m,DK_NGAS,DK_IM1+c,k,j,i)] + static_cast<double>(qd[Idx(g,m,4,1+c,k,j,i)]))*pinv);
+          (u0[Idx(g,m,DK_NGAS,DK_IM1+c,k,j,i)] + static_cast<double>(sum[1+c]))*pinv);
+    }
   }
-}
+};
 
-// one defect-correction sweep x += (rho + Q)^-1 (M + P - (Ax)) (dust_solver.cpp:243-252)
-__global__ void k_dc(Geo g, const double *u0, const float *qd, const float *ap, float *us) {
-  BLOCK_CELLS(m, k, j, i)
+// one defect-correction sweep x += (rho + Q)^-1 (M + P - (Ax)) (dust_solver.cpp:243-252); sum: the
+// operator's particle part
+struct CellCorrect {
+  const double *u0;
+  const float *qd;
+  float *us;
+  __device__ void operator()(const Geo &g, int m, int k, int j, int i, const float sum[3]) const {
     const double rho = u0[Idx(g,m,DK_NGAS,DK_IDN,k,j,i)];
     const double pinv = 1.0/(rho + static_cast<double>(qd[Idx(g,m,4,0,k,j,i)]));
     for (int d=0; d<3; ++d) {
       const long long id = Idx(g,m,3,d,k,j,i);
       const double x = static_cast<double>(us[id]);
-      const double av = static_cast<double>(ap[id]) + rho*x;
+      const double av = static_cast<double>(sum[d]) + rho*x;
       const double rv = u0[Idx(g,m,DK_NGAS,DK_IM1+d,k,j,i)] +
                         static_cast<double>(qd[Idx(g,m,4,1+d,k,j,i)]) - av;
       us[id] = static_cast<float>(x + pinv*rv);
     }
   }
-}
+};
 
 // the consistent split (dust_pm.cpp:670-685): the residual r = (D - G)/(rho + Q) of the
 // dust per unit coupled mass res = r Q/qt for the particles centred here; the gas gets
-// D - (the dust's actual change) at the next stage start
-__global__ void k_split(Geo g, const double *u0, const float *us, const float *qd,
-                        const float *qt0, const float *qt1, const float *qt2, const double *dmom,
-                        float *res) {
-  BLOCK_CELLS(m, k, j, i)
+// D - (the dust's actual change) at the next stage start (D is kept)
+struct CellSplit {
+  const double *u0;
+  const float *us, *qd, *qt0, *qt1, *qt2;
+  double *dmom;
+  float *res;
+  __device__ void operator()(const Geo &g, int m, int k, int j, int i, const double sum[3]) const {
     const double rho = u0[Idx(g,m,DK_NGAS,DK_IDN,k,j,i)];
     const long long i1 = Idx(g,m,1,0,k,j,i);
     const double qt = static_cast<double>(qt0[i1]) + static_cast<double>(qt1[i1]) +
@@ -3036,13 +3559,14 @@ __global__ void k_split(Geo g, const double *u0, const float *us, const float *q
       double rs = 0.0;
       if (qt > 0.0) {
         const double gg = rho*static_cast<double>(us[id]) - u0[Idx(g,m,DK_NGAS,DK_IM1+c,k,j,i)];
-        const double r = (dmom[id] - gg)/(rho + q);
+        const double r = (sum[c] - gg)/(rho + q);
         rs = r*q/qt;
       }
+      dmom[id] = sum[c];
       res[id] = static_cast<float>(rs);
     }
   }
-}
+};
 
 // bind: the caller's FP64 SoA into the store (original order)
 __global__ void k_bind(const double *r, const int32_t *iv, long long cap, long long np, Store S,
@@ -3364,11 +3888,6 @@ dim3 CellGrid(const dk_ctx *c) {
   return dim3(static_cast<unsigned>(std::min<long long>(b, 65535)), c->g.nmb);
 }
 
-dim3 CombineGrid(const dk_ctx *c) {
-  const long long b = (c->g.ncb + kBlock - 1)/kBlock;
-  return dim3(static_cast<unsigned>(std::min<long long>(b, 4096)), c->g.nmb);
-}
-
 #define TIMED(label, launch) \
   do { const int tk_ = dk::ProfBegin(c, label); launch; dk::ProfEnd(c, tk_); } while (0)
 
@@ -3436,52 +3955,56 @@ KArgs MakeArgs(dk_ctx *c) {
   return A;
 }
 
-// counting sort of the store by the keys of the key pass: scan, placement, and the arrivals of
-// every cell in ascending source slot after its stayers (whose ranks are in slot order): a fixed
-// order
-int SortKeys(dk_ctx *c) {
-  Fast *f = c->fast;
-  int e;
-  TIMED("total", (k_total<<<Grid(f->nkeys), kBlock, 0, c->stream>>>(f->count, f->stay,
-                                                                     f->nkeys)));
-  TIMED("scan", e = dk::Check(hipcub::DeviceScan::ExclusiveSum(
-      f->scan_tmp, f->scan_bytes, f->count, f->start, (int)(f->nkeys + 1), c->stream)));
-  if (e) return e;
-  TIMED("place", (k_place<<<Grid((f->np + kPlaceU - 1)/kPlaceU), kBlock, 0, c->stream>>>(
-      f->key, f->rank, f->start, f->stay, f->np, f->T.TC, f->item_start, f->ov_cnt, f->perm)));
-  if ((e = FillV<int>(c, f->big, 2, 0))) return e;
-  TIMED("segsort", (k_segsort<<<Grid(f->nkeys), kBlock, 0, c->stream>>>(
-                        f->start, f->stay, f->nkeys, f->perm, f->big)));
-  TIMED("medsort", (k_medsort<<<4096, 64, 0, c->stream>>>(f->start, f->stay, f->perm, f->big)));
-  TIMED("bigsort", (k_bigsort<<<256, 1024, 0, c->stream>>>(f->start, f->stay, f->perm, f->big,
-                                                            f->nkeys, c->d_err)));
+// workgroups and rounds of the key scan's launches
+void ScanShape(long long nkeys, int &groups, int &rounds) {
+  const long long per = (nkeys + kScanKeys - 1)/kScanKeys;
+  rounds = static_cast<int>((per + kScanGroups - 1)/kScanGroups);
+  groups = static_cast<int>((per + rounds - 1)/rounds);
+}
+
+// the later parts' shares of a key pass added (pres: also the push residues and the stayers'
+// counts; null: the corrections alone)
+int FixKey(dk_ctx *c, const KArgs &A, double *pres) {
+  const Fast *f = c->fast;
+  TIMED("fix", (k_fix_key<<<Grid(4*(long long)f->T.nt*f->T.TC), kBlock, 0, c->stream>>>(
+                    A, pres != nullptr, pres)));
   return dk::Check(hipGetLastError());
 }
 
-// the work items of the present order: parts per tile, their scan, the tile of every item
+// counting sort of the store by the keys of the key pass (after FixKey): scan, placement, and the
+// arrivals of every cell in ascending source slot after its stayers (whose ranks are in slot
+// order): a fixed order
+int SortKeys(dk_ctx *c) {
+  Fast *f = c->fast;
+  int groups, rounds;
+  ScanShape(f->nkeys, groups, rounds);
+  TIMED("scan", (k_key_sums<<<groups, kScanThreads, 0, c->stream>>>(
+      f->count, f->stay, f->nkeys, rounds, f->scan_part)));
+  TIMED("scan", (k_key_scan<<<groups, kScanThreads, 0, c->stream>>>(
+      f->count, f->stay, f->nkeys, rounds, f->scan_part, f->start, f->big)));
+  TIMED("place", (k_place<<<Grid((f->np + kPlaceU - 1)/kPlaceU), kBlock, 0, c->stream>>>(
+      f->key, f->rank, f->start, f->stay, f->np, f->T.TC, f->item_start, f->ov_cnt, f->perm)));
+  TIMED("segsort", (k_segsort<<<Grid(f->nkeys), kBlock, 0, c->stream>>>(
+                        f->start, f->stay, f->nkeys, f->perm, f->big)));
+  TIMED("longsort", (k_longsort<<<256, kLongThreads, 0, c->stream>>>(
+                         f->start, f->stay, f->perm, f->big, f->nkeys, c->d_err)));
+  return dk::Check(hipGetLastError());
+}
+
+// the work items of the present order
 int BuildItems(dk_ctx *c) {
   Fast *f = c->fast;
   const Tiles &T = f->T;
   const int W = PartChunks(T.SY)*kPPT*3*T.TC;
-  TIMED("items", (k_nparts<<<Grid(T.nt + 1), kBlock, 0, c->stream>>>(T, f->start, W,
-                                                                      f->nparts)));
-  int e;
-  TIMED("items", e = dk::Check(hipcub::DeviceScan::ExclusiveSum(
-      f->iscan_tmp, f->iscan_bytes, f->nparts, f->item_start, T.nt + 1, c->stream)));
-  if (e) return e;
-  TIMED("items", (k_item_tile<<<Grid(T.nt), kBlock, 0, c->stream>>>(T, f->item_start,
-                                                                     f->item_tile)));
-  {
-    TIMED("items", (k_item_flags<<<Grid(f->item_cap + 1), kBlock, 0, c->stream>>>(
-        T, f->item_start, f->item_tile, f->item_cap + 1, f->iflag, T.SY ? 0 : 1)));
-    TIMED("items", e = dk::Check(hipcub::DeviceScan::ExclusiveSum(
-        f->lscan_tmp, f->lscan_bytes, f->iflag, f->iflag_scan, (int)(f->item_cap + 1),
-        c->stream)));
-    if (e) return e;
-    TIMED("items", (k_item_lists<<<Grid(f->item_cap), kBlock, 0, c->stream>>>(
-        T, f->item_start, f->iflag, f->iflag_scan, f->item_cap, f->ilist[0], f->ilist[1],
-        f->ilist_n)));
-  }
+  const int per = (T.nt + kItemTiles - 1)/kItemTiles;
+  const int rounds = (per + kScanGroups/4 - 1)/(kScanGroups/4);
+  const int groups = (per + rounds - 1)/rounds;
+  if (groups > 1)
+    TIMED("items", (k_item_sums<<<groups, kItemThreads, 0, c->stream>>>(T, f->start, W, rounds,
+                                                                         f->scan_part)));
+  TIMED("items", (k_item_lists<<<groups, kItemThreads, 0, c->stream>>>(
+      T, f->start, W, rounds, f->scan_part, f->item_start, f->item_tile, f->ilist[0],
+      f->ilist[1], f->ilist_n)));
   return dk::Check(hipGetLastError());
 }
 
@@ -3494,22 +4017,14 @@ int AllocItems(dk_ctx *c, long long n) {
   if (ov <= f->ov_cap && f->item_start) return DK_OK;
   for (void *p : {(void*)f->item_tile, (void*)f->ov_scr, (void*)f->ov_q, (void*)f->ov_pr,
                   (void*)f->ov_def, (void*)f->ov_dc, (void*)f->ov_cnt, (void*)f->ilist[0],
-                  (void*)f->ilist[1], (void*)f->iflag, (void*)f->iflag_scan, f->lscan_tmp,
-                  (void*)f->x3p})
+                  (void*)f->ilist[1], (void*)f->x3p})
     if (p) (void)hipFree(p);
   f->x3p = nullptr;
   f->item_tile = nullptr; f->ov_scr = nullptr; f->ov_q = nullptr; f->ov_pr = nullptr;
   f->ov_def = nullptr; f->ov_dc = nullptr; f->ov_cnt = nullptr;
-  f->ilist[0] = nullptr; f->ilist[1] = nullptr; f->iflag = nullptr; f->iflag_scan = nullptr;
-  f->lscan_tmp = nullptr;
-  if (f->nparts == nullptr) {
-    if (Alloc((void**)&f->nparts, sizeof(int)*(T.nt + 1))) return DK_ENOMEM;
-    if (Alloc((void**)&f->item_start, sizeof(int)*(T.nt + 1))) return DK_ENOMEM;
-    if (hipcub::DeviceScan::ExclusiveSum(nullptr, f->iscan_bytes, f->nparts, f->item_start,
-                                         T.nt + 1) != hipSuccess)
-      return DK_EHIP;
-    if (Alloc(&f->iscan_tmp, std::max<size_t>(f->iscan_bytes, 16))) return DK_ENOMEM;
-  }
+  f->ilist[0] = nullptr; f->ilist[1] = nullptr;
+  if (f->item_start == nullptr && Alloc((void**)&f->item_start, sizeof(int)*(T.nt + 1)))
+    return DK_ENOMEM;
   f->item_cap = T.nt + ov;
   f->ov_cap = ov;
   if (Alloc((void**)&f->item_tile, sizeof(int)*f->item_cap) ||
@@ -3524,20 +4039,44 @@ int AllocItems(dk_ctx *c, long long n) {
   if (c->g.bc_x3 == DK_X3_OUTFLOW &&
       Alloc((void**)&f->x3p, sizeof(double)*2*((size_t)f->item_cap + kX3Groups)))
     return DK_ENOMEM;
-  {
-    if (f->ilist_n == nullptr && Alloc((void**)&f->ilist_n, sizeof(int)*2)) return DK_ENOMEM;
-    if (Alloc((void**)&f->ilist[0], sizeof(int)*f->item_cap) ||
-        Alloc((void**)&f->ilist[1], sizeof(int)*f->item_cap) ||
-        Alloc((void**)&f->iflag, sizeof(int)*(f->item_cap + 1)) ||
-        Alloc((void**)&f->iflag_scan, sizeof(int)*(f->item_cap + 1)))
-      return DK_ENOMEM;
-    f->lscan_bytes = 0;
-    if (hipcub::DeviceScan::ExclusiveSum(nullptr, f->lscan_bytes, f->iflag, f->iflag_scan,
-                                         (int)(f->item_cap + 1)) != hipSuccess)
-      return DK_EHIP;
-    if (Alloc(&f->lscan_tmp, std::max<size_t>(f->lscan_bytes, 16))) return DK_ENOMEM;
-  }
+  if (f->ilist_n == nullptr && Alloc((void**)&f->ilist_n, sizeof(int)*2)) return DK_ENOMEM;
+  if (Alloc((void**)&f->ilist[0], sizeof(int)*f->item_cap) ||
+      Alloc((void**)&f->ilist[1], sizeof(int)*f->item_cap))
+    return DK_ENOMEM;
   return DK_OK;
+}
+
+// The combine, the fold and the cell pass op of a deposit's NV components (out: the field that
+// holds them, in the type of the sums): one launch, and one more for the cells of the
+// shear-periodic x1 faces.
+template <int NV, typename TO, class Op>
+int FoldCells(dk_ctx *c, const char *label, TO *out, bool defect, double t, const Op &op) {
+  const Fast *f = c->fast;
+  const Geo &g = c->g;
+  Regions R;
+  R.g = g; R.T = f->T; R.B = c->d_blocks; R.slot_dir = c->d_slot_dir;
+  R.scr = f->scr_f; R.item_start = f->item_start; R.ov_scr = f->ov_scr;
+  R.defect = defect ? f->defect : nullptr; R.ov_def = f->ov_def;
+  R.fold_x3 = c->M.bc_x3 != DK_X3_PERIODIC && !c->M.x3_dep_drop;
+  const Tiles &T = f->T;
+  R.pairs = T.TX >= 2 && T.TY >= 2*(1 + T.SY) && T.TZ >= 2 &&
+            (long long)T.ntb*T.RN*NV < (1LL << 30);
+  R.vs = T.RZ*T.RY*T.ntx*T.RX;
+  R.sy = NV*R.vs;
+  R.sz = T.nty*R.sy;
+  R.sm = (long long)T.ntz*R.sz;
+  const int shear = c->M.bc_x1 == DK_X1_SHEAR;
+  const Shell S = MakeShell(g, f->T.SY);
+  const dim3 grid(S.inner_blocks + (S.total - S.inner + kBlock - 1)/kBlock, g.nmb);
+  TIMED(label, (k_fold_cells<NV, TO, Op><<<grid, kBlock, 0, c->stream>>>(R, S, out, shear, op)));
+  if (shear) {
+    const double lx = c->M.x1max - c->M.x1min, ly = c->M.x2max - c->M.x2min;
+    const double ysh = std::fmod(c->P.qshear*c->P.omega0*lx*t, ly);
+    const long long n = 2LL*g.nmbx2*g.nmbx3*g.nx3*g.nx2;
+    TIMED("fold_shear", (k_fold_shear_cells<NV, TO, Op><<<Grid(n), kBlock, 0, c->stream>>>(
+        R, out, ysh/(ly/(g.nx2*g.nmbx2)), op)));
+  }
+  return dk::Check(hipGetLastError());
 }
 
 // the pending consistent-dust correction alone (before an export or a diagnostic)
@@ -3546,8 +4085,7 @@ int Flush(dk_ctx *c) {
   if (!f->pending) return DK_OK;
   KArgs A = MakeArgs(c);
   TIMED("key", LaunchKey(c, A, 0, nullptr));
-  TIMED("fix", (k_fix_key<<<Grid((long long)f->T.nt*f->T.TC), kBlock, 0, c->stream>>>(
-      A, 0, nullptr)));
+  if (const int e = FixKey(c, A, nullptr)) return e;
   dk_gas_src z;
   std::memset(&z, 0, sizeof(z));
   const long long nact = (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3;
@@ -3649,10 +4187,7 @@ int FastCreate(dk_ctx *c) {
   for (int q=0; q<2; ++q) (void)hipMemset(f->pres[q], 0, sizeof(double)*3*nc);
   (void)hipMemset(f->ustar, 0, sizeof(float)*3*nc);
   (void)hipMemset(f->res, 0, sizeof(float)*3*nc);
-  if (hipcub::DeviceScan::ExclusiveSum(nullptr, f->scan_bytes, f->count, f->start,
-                                       (int)(f->nkeys + 1)) != hipSuccess)
-    return DK_EHIP;
-  return Alloc(&f->scan_tmp, std::max<size_t>(f->scan_bytes, 16));
+  return Alloc((void**)&f->scan_part, sizeof(int)*kScanGroups);
 }
 
 void FastDestroy(dk_ctx *c) {
@@ -3660,11 +4195,10 @@ void FastDestroy(dk_ctx *c) {
   if (f == nullptr) return;
   for (auto &ev : f->tev)
     if (ev) {(void)hipEventDestroy(ev); ev = nullptr;}
-  for (void *p : {(void*)f->nparts, (void*)f->item_start, (void*)f->item_tile, f->iscan_tmp,
+  for (void *p : {(void*)f->item_start, (void*)f->item_tile,
                   (void*)f->ov_scr, (void*)f->ov_q, (void*)f->ov_pr, (void*)f->ov_def,
                   (void*)f->ov_dc, (void*)f->ov_cnt, (void*)f->ilist[0], (void*)f->ilist[1],
-                  (void*)f->ilist_n, (void*)f->iflag, (void*)f->iflag_scan, f->lscan_tmp,
-                  (void*)f->x3p})
+                  (void*)f->ilist_n, (void*)f->x3p})
     if (p) (void)hipFree(p);
   for (int b=0; b<2; ++b) {
     Store &S = f->s[b];
@@ -3672,7 +4206,7 @@ void FastDestroy(dk_ctx *c) {
       if (p) (void)hipFree(p);
   }
   for (void *p : {(void*)f->key, (void*)f->rank, (void*)f->count, (void*)f->start,
-                  (void*)f->perm, (void*)f->big, (void*)f->stay, f->scan_tmp, (void*)f->itag, (void*)f->qdep,
+                  (void*)f->perm, (void*)f->big, (void*)f->stay, (void*)f->scan_part, (void*)f->itag, (void*)f->qdep,
                   (void*)f->ustar, (void*)f->ap, (void*)f->res, (void*)f->dmom, (void*)f->pres[0], (void*)f->pres[1],
                   (void*)f->scr_f, (void*)f->defect, (void*)f->cpack, (void*)f->xl_list,
                   (void*)f->xl_n})
@@ -3899,34 +4433,39 @@ static int FastStagePc2(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
     const long long nin = (long long)gg.nmb*(gg.n1 - 2)*(gg.n2 - 2)*(gg.n3 - 2);
     TIMED("cloud_pack", (k_fpack<<<Grid(nin), kBlock, 0, c->stream>>>(gg, f->ustar, f->cpack)));
   }
-  if ((e = FillV<int>(c, f->count, f->nkeys + 1, 0))) return e;
   TIMED("key", LaunchKey(c, A, 1, f->pres[1 - f->pres_rd], !s1));
-  TIMED("fix", (k_fix_key<<<Grid((long long)T.nt*T.TC), kBlock, 0, c->stream>>>(
-      A, 1, f->pres[1 - f->pres_rd])));
+  if ((e = FixKey(c, A, f->pres[1 - f->pres_rd]))) return e;
   if ((e = SortKeys(c))) return e;
   if ((e = BuildItems(c))) return e;
   if (c->smr && (e = FillV<int>(c, f->xl_n, 1, 0))) return e;
   if (s1) {
     TIMED("pc2_predictor", LaunchPP(c, A, gf, f->scr_f, cl));
-    TIMED("combine", (k_combine<float, 4><<<CombineGrid(c), kBlock, 0, c->stream>>>(
-        g, T, f->scr_f, f->qdep, nullptr, f->item_start, f->ov_scr, f->ov_def)));
-    if ((e = FoldT<float>(c, f->qdep, 4, st->time))) return e;
-    if (c->smr)
+    const CellPc2Apply apply{c->u0, f->qdep, c->P.pc2_damping, st->dt};
+    if (c->smr) {
+      if ((e = FoldCells<4, float>(c, "fold", f->qdep, false, st->time,
+                                   CellStore<4, float>{f->qdep}))) return e;
       TIMED("cloud_xlevel", (k_fxl_predictor<<<Grid(f->np*kCoop), kBlock, 0, c->stream>>>(
           A, dk::MakeCloudGeo(c), gf, f->qdep)));
+      TIMED("pc2_apply", (k_cells<4, float><<<CellGrid(c), kBlock, 0, c->stream>>>(
+          g, f->qdep, apply)));
+    } else if ((e = FoldCells<4, float>(c, "fold_apply", f->qdep, false, st->time, apply))) {
+      return e;
+    }
+    // (the record reads the rate and rho, which the predictor's application leaves as they are)
     if (dk::StiffnessActive(c->P) && (e = StiffnessRecord<float>(c, f->qdep, 4, 0, st->dt))) return e;
-    TIMED("pc2_apply", (k_pc2_apply<<<CellGrid(c), kBlock, 0, c->stream>>>(
-        g, c->u0, f->qdep, c->P.pc2_damping, st->dt)));
   } else {
     TIMED("pc2_advance", LaunchPA(c, A, gf, f->scr_f, f->defect, cl));
-    TIMED("combine", (k_combine<float, 3, double><<<CombineGrid(c), kBlock, 0, c->stream>>>(
-        g, T, f->scr_f, f->dmom, f->defect, f->item_start, f->ov_scr, f->ov_def)));
-    if ((e = FoldT<double>(c, f->dmom, 3, st->time))) return e;
-    if (c->smr)
+    const CellPc2Commit commit{c->u0, f->qdep, st->gam1[st->nexp_stages - 1]};
+    if (c->smr) {
+      if ((e = FoldCells<3, double>(c, "fold", f->dmom, true, st->time,
+                                    CellStore<3, double>{f->dmom}))) return e;
       TIMED("cloud_xlevel", (k_fxl_advance<<<Grid(f->np*kCoop), kBlock, 0, c->stream>>>(
           A, dk::MakeCloudGeo(c), gf, f->dmom)));
-    TIMED("pc2_commit", (k_pc2_commit<<<CellGrid(c), kBlock, 0, c->stream>>>(
-        g, c->u0, f->dmom, f->qdep, st->gam1[st->nexp_stages - 1])));
+      TIMED("pc2_commit", (k_cells<3, double><<<CellGrid(c), kBlock, 0, c->stream>>>(
+          g, f->dmom, commit)));
+    } else if ((e = FoldCells<3, double>(c, "fold_commit", f->dmom, true, st->time, commit))) {
+      return e;
+    }
   }
   f->cur = 1 - f->cur;
   f->regs_dead = 0;
@@ -3968,7 +4507,6 @@ int FastStage(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
     A.dsh = c->P.qshear*c->P.omega0*lx*(ShearRouteTime(st) - st->time);
   }
   // 1. key pass (with the pending correction), histogram
-  if ((e = FillV<int>(c, f->count, f->nkeys + 1, 0))) return e;
   // the push of this stage writes its residue into the buffer the next stage's start reads
   TIMED("key", LaunchKey(c, A, 1, f->pres[1 - f->pres_rd]));
   if (f->x3p != nullptr)   // the outflow ledger (bvals_part.cpp:184-186) of the items just run
@@ -3976,8 +4514,7 @@ int FastStage(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
                             f->item_start, T.nt, f->x3p, f->x3p + 2*(size_t)f->item_cap),
                         k_x3sum<<<1, kX3Groups, 0, c->stream>>>(
                             f->x3p + 2*(size_t)f->item_cap, c->d_scalar + 12)));
-  TIMED("fix", (k_fix_key<<<Grid((long long)T.nt*T.TC), kBlock, 0, c->stream>>>(
-      A, 1, f->pres[1 - f->pres_rd])));
+  if ((e = FixKey(c, A, f->pres[1 - f->pres_rd]))) return e;
   // 2. stage start cell pass: previous split's gas share, u1 <- u0, gas update, drag history
   {
     // with isothermal fluxes the gas update and the drag history run after the cell pass, in
@@ -4006,29 +4543,23 @@ int FastStage(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
   f->cur = 1 - f->cur;
   A.src = f->s[f->cur];
   A.dst = f->s[1 - f->cur];
-  TIMED("combine", (k_combine<float, 4><<<CombineGrid(c), kBlock, 0, c->stream>>>(
-      g, T, f->scr_f, f->qdep, nullptr, f->item_start, f->ov_scr, f->ov_def)));
-  if ((e = FoldT<float>(c, f->qdep, 4, st->time))) return e;
-  // 5. local guess + dc1/dc2 sweeps
-  TIMED("guess", (k_guess<<<CellGrid(c), kBlock, 0, c->stream>>>(g, c->u0, f->qdep, f->ustar)));
+  // 5. the deposit's fold with the local guess, then dc1/dc2 sweeps
+  if ((e = FoldCells<4, float>(c, "fold_guess", f->qdep, false, st->time,
+                               CellGuess{c->u0, f->qdep, f->ustar}))) return e;
   const int nsweeps = (c->P.solver == DK_DC2) ? 2 : ((c->P.solver == DK_DC1) ? 1 : 0);
   for (int sw=0; sw<nsweeps; ++sw) {
     if ((e = FillGhostsT<float>(c, f->ustar, 3, true, st->time))) return e;
     TIMED("p2_operator", LaunchP2(c, A, f->ustar, f->scr_f));
-    TIMED("combine", (k_combine<float, 3><<<CombineGrid(c), kBlock, 0, c->stream>>>(
-        g, T, f->scr_f, f->ap, nullptr, f->item_start, f->ov_scr, f->ov_def)));
-    if ((e = FoldT<float>(c, f->ap, 3, st->time))) return e;
-    TIMED("dc", (k_dc<<<CellGrid(c), kBlock, 0, c->stream>>>(g, c->u0, f->qdep, f->ap, f->ustar)));
+    if ((e = FoldCells<3, float>(c, "fold_dc", f->ap, false, st->time,
+                                 CellCorrect{c->u0, f->qdep, f->ustar}))) return e;
   }
   if ((e = FillGhostsT<float>(c, f->ustar, 3, true, st->time))) return e;
-  // 6. gather-kick + impulse deposit
+  // 6. gather-kick + impulse deposit, its fold with the consistent split: the dust's residual per
+  // unit coupled mass
   TIMED("p3_gather_kick", LaunchP3(c, A, f->ustar, f->scr_f, f->defect));
-  TIMED("combine", (k_combine<float, 3, double><<<CombineGrid(c), kBlock, 0, c->stream>>>(
-      g, T, f->scr_f, f->dmom, f->defect, f->item_start, f->ov_scr, f->ov_def)));
-  if ((e = FoldT<double>(c, f->dmom, 3, st->time))) return e;
-  // 7. consistent split: the dust's residual per unit coupled mass
-  TIMED("split", (k_split<<<CellGrid(c), kBlock, 0, c->stream>>>(
-      g, c->u0, f->ustar, f->qdep, f->qt[0], f->qt[1], f->qt[2], f->dmom, f->res)));
+  if ((e = FoldCells<3, double>(c, "fold_split", f->dmom, true, st->time,
+                                CellSplit{c->u0, f->ustar, f->qdep, f->qt[0], f->qt[1], f->qt[2],
+                                          f->dmom, f->res}))) return e;
   f->pending = 1;
   f->regs_dead = !A.regs_live;
   f->pres_rd = 1 - f->pres_rd;

@@ -50,9 +50,11 @@ struct SmrTree {
   double lo[3], len[3];
 };
 
+// (a block's padded cells fit 32 bits, dk_create checks: the cell's index in 32-bit arithmetic, and
+// one 64-bit product that is the same for all lanes of a launch over blocks)
 __host__ __device__ inline long long Idx(const Geo &g, int m, int nvar, int v, int k, int j,
                                          int i) {
-  return ((((long long)m*nvar + v)*g.n3 + k)*g.n2 + j)*(long long)g.n1 + i;
+  return ((long long)m*nvar + v)*g.ncb + ((k*g.n2 + j)*g.n1 + i);
 }
 
 __host__ __device__ inline int Dir(int ox1, int ox2, int ox3) {
@@ -84,6 +86,30 @@ __device__ inline void PMWeights(const double x, const double xmin, const double
 // qdep[4] and UpdateStiffness records chi whenever the stiffness record is asked for or the
 // feedback damping of stiff cells needs it (phst_track, the particle history, is not built)
 inline bool StiffnessActive(const dk_physics &P) { return P.stiffness != 0 || P.pc2_damping != 0; }
+
+// The cells of a padded block field that hold global row r (0 <= r < nx*nb) along one axis, in
+// fixed slots: [0] the active row of block r/nx, [1] the upper ghost copy in block r/nx - 1,
+// [2] the lower ghost copy in block r/nx + 1 (periodic wrap, or none beyond a physical face).
+// blk/loc receive block row and padded index; the bit s of the result is set when slot s holds a
+// copy (fixed slots, so that callers' loops keep the arrays in registers).
+__device__ inline int RowCopies(int r, int nx, int nb, int ng, int start, bool periodic,
+                                int blk[3], int loc[3]) {
+  int mask = 1;
+  const int b = r/nx, l = r - b*nx;
+  blk[0] = b; loc[0] = start + l;
+  blk[1] = 0; loc[1] = 0; blk[2] = 0; loc[2] = 0;
+  if (l < ng) {                 // the upper ghost rows of block b - 1
+    int b2 = b - 1;
+    if (b2 < 0) b2 = periodic ? b2 + nb : -1;
+    if (b2 >= 0) {blk[1] = b2; loc[1] = start + nx + l; mask |= 2;}
+  }
+  if (l >= nx - ng) {           // the lower ghost rows of block b + 1
+    int b2 = b + 1;
+    if (b2 >= nb) b2 = periodic ? b2 - nb : -1;
+    if (b2 >= 0) {blk[2] = b2; loc[2] = start - (nx - l); mask |= 4;}
+  }
+  return mask;
+}
 
 // First error wins: code and particle index.
 struct ErrWord {
