@@ -63,6 +63,8 @@ constexpr int kMaxTileCells = 128;
 // reads one contiguous 256 B or 512 B piece, and every column of a particle is addressed from
 // one base with a constant offset, so that a kernel holds few addresses in registers.
 constexpr int kGrp = 64;
+constexpr long long kTags = DK_NIDATA - 1;   // the caller's integers that the store keeps
+static_assert(kTags == 4, "one 16-byte word a particle");
 struct Store {
   double *d;
   float *f;
@@ -116,7 +118,9 @@ struct Fast {
   int *ilist[2] = {nullptr, nullptr};
   int *ilist_n = nullptr;
   int *scan_part = nullptr;         // the workgroups' sums of the key and item scans
-  int32_t *itag = nullptr;          // caller's PTAG, PSP, PLEV, PTAGH by original index
+  // the caller's PTAG, PSP, PLEV, PTAGH of an original index, side by side: the export takes
+  // them in the store's order, one 16-byte word a particle instead of four scattered ones
+  int32_t *itag = nullptr;
   // fields, gas layout with ghosts
   float *qdep = nullptr;            // Q, P1, P2, P3
   float *qt[3] = {nullptr, nullptr, nullptr};   // centre mass m c/V: own, from below, above
@@ -221,7 +225,7 @@ struct KArgs {
   // level by original index, and the list of the store slots whose clouds the tile kernels
   // leave to the leaf traversal (xl_n: its length)
   dk::SmrTree tree;
-  const int32_t *plev;
+  const int32_t *plev;              // (stride kTags)
   int *xl_list, *xl_n;
 };
 
@@ -1172,7 +1176,7 @@ __device__ inline bool CrossLevel(const Geo &g, const DevBlock &b, int lev, cons
 }
 
 // What the key pass reads of one particle (store slot q): position, velocity, rate (when the
-// push or the pending correction uses it), the stage registers x1, v1 (at stage 2 of imex: where
+// push or the correction alone uses it), the stage registers x1, v1 (at stage 2 of imex: where
 // the stage-1 key pass wrote them, the other store at the slot of the last sort's permutation),
 // mass and, with a pending correction, stopping time, the slot's tile-local cell and the
 // residual rows of that cell and the cells beside it in x2 (the centre is one of them).
@@ -1192,7 +1196,7 @@ __device__ inline void KeyFetch(const KArgs &A, const TileInfo &t, const int *st
                                 int do_key, int pq, KeyIn &k) {
   const Geo &g = A.g;
   const Tiles &Tl = A.T;
-  const bool rates = A.atw_dt != 0.0 || !do_key;
+  const bool rates = do_key ? A.atw_dt != 0.0 : A.regs_live != 0;
   k.cell = 0;
   k.ts = 0.0f;
 #pragma unroll
@@ -1229,14 +1233,17 @@ __device__ inline void KeyFetch(const KArgs &A, const TileInfo &t, const int *st
 // (dust_push.cpp:249-297, bvals_part.cpp:164-429) written back in place, the push rounding
 // residue summed per cell for the gas, and every particle's new tile-major key and rank: a
 // particle that stays in its tile takes its rank from a count in LDS (the tile owns those
-// cells: stay[]), one that leaves it from a global count of arrivals (count[]).  With do_key = 0
-// only the pending correction is applied (written to v and R).  MID: the pc2 stage-2 form, keyed
-// by the half-step position (Pc2Route) instead of pushed.
+// cells: stay[]), one that leaves it from a global count of arrivals (count[]).  Without KEY
+// only the pending correction is applied (written to v and R): code of its own, without the
+// push's registers and without reading the rates unless they are kept (117 million particles:
+// 3.1 -> 2.6 ms, each time step's reduction and export).  MID: the pc2 stage-2 form, keyed by the
+// half-step position (Pc2Route) instead of pushed.
 // (Bk: the block table again, as a restrict pointer: the tile's block, read by every particle,
 // is then read with scalar loads once per item instead of vector loads in every chunk)
-template <bool OV, bool MID = false, bool SMR = false>
+template <bool OV, bool MID = false, bool SMR = false, bool KEY = true>
 __global__ void __launch_bounds__(kKeyThreadsMax, (OV || SMR) ? 2 : 4)
-k_key(KArgs A, int do_key, double *pres, const DevBlock *__restrict__ Bk) {
+k_key(KArgs A, double *pres, const DevBlock *__restrict__ Bk) {
+  constexpr int do_key = KEY;
   extern __shared__ double lds_d[];
   const Geo &g = A.g;
   const Tiles &Tl = A.T;
@@ -2334,7 +2341,7 @@ k_pp(KArgs A, const float *uv, float *scr, const DevBlock *__restrict__ Bk) {
         float val[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         bool xl = false;   // (refined meshes: a cross-level cloud, deposited by k_fxl_predictor)
         if constexpr (CLOUD)
-          xl = A.xl_list != nullptr && CrossLevel(g, b, A.plev[orig], x, L.ci, L.cj, L.ck);
+          xl = A.xl_list != nullptr && CrossLevel(g, b, A.plev[kTags*orig], x, L.ci, L.cj, L.ck);
         if (TileKey(Tl, t.m, L.ci, L.cj, L.ck) != kp) {
           dk::RecordError(A.err, DK_EHALO, p);
         } else if (xl) {
@@ -2490,7 +2497,7 @@ k_pa(KArgs A, const float *us, float *scr, double *defect, const DevBlock *__res
         double dv[3] = {0.0, 0.0, 0.0};
         bool xl = false;   // (refined meshes: a cross-level cloud, advanced by k_fxl_advance)
         if constexpr (CLOUD)
-          xl = A.xl_list != nullptr && CrossLevel(g, b, A.plev[orig], xh, L.ci, L.cj, L.ck);
+          xl = A.xl_list != nullptr && CrossLevel(g, b, A.plev[kTags*orig], xh, L.ci, L.cj, L.ck);
         if (TileKey(Tl, t.m, L.ci, L.cj, L.ck) != kp) {
           dk::RecordError(A.err, DK_EHALO, p);
         } else if (xl) {
@@ -2654,7 +2661,7 @@ __global__ void __launch_bounds__(kBlock) k_fxl_predictor(KArgs A, dk::CloudGeo 
   for (int t = blockIdx.x*(kBlock/kCoop) + grp; t < n; t += gridDim.x*(kBlock/kCoop)) {
     const int q = A.xl_list[t];
     const double x[3] = {A.dst.X(0, q), A.dst.X(1, q), A.dst.X(2, q)};
-    const int lev = A.plev[A.dst.ORIG(q)];
+    const int lev = A.plev[kTags*A.dst.ORIG(q)];
     const dk::CoopCloud cl = dk::CoopSpans(g, A.B, A.tree, cg, x, lev, lane, lf);
     if (cl.total < 0) {
       if (lane == 0) dk::RecordError(A.err, DK_EHALO, q);
@@ -2692,7 +2699,7 @@ __global__ void __launch_bounds__(kBlock) k_fxl_advance(KArgs A, dk::CloudGeo cg
     const int q = A.xl_list[t];
     double x[3] = {A.dst.X(0, q), A.dst.X(1, q), A.dst.X(2, q)};
     float v[3] = {A.dst.V(0, q), A.dst.V(1, q), A.dst.V(2, q)};
-    const int lev = A.plev[A.dst.ORIG(q)];
+    const int lev = A.plev[kTags*A.dst.ORIG(q)];
     double xh[3];
     Pc2Mid(A, x, v, xh);
     const dk::CoopCloud cl = dk::CoopSpans(g, A.B, A.tree, cg, xh, lev, lane, lf);
@@ -3583,7 +3590,7 @@ __global__ void k_bind(const double *r, const int32_t *iv, long long cap, long l
     S.M(p) = static_cast<float>(r[(long long)DK_IPM*cap + p]);
     S.GID(p) = iv[(long long)DK_PGID*cap + p];
     S.ORIG(p) = static_cast<int>(p);
-    for (int c=1; c<DK_NIDATA; ++c) itag[(long long)(c - 1)*np + p] = iv[(long long)c*cap + p];
+    for (int c=1; c<DK_NIDATA; ++c) itag[kTags*p + c - 1] = iv[(long long)c*cap + p];
   }
 }
 
@@ -3620,7 +3627,7 @@ __global__ void k_permute_all(Store src, Store dst, const int *perm, long long n
 // to x, x1 and the block, as the reference's state holds them; A: its mesh numbers, with
 // gam0 = 1 and gam1 = beta_dt = 0 so that PushMigrate only routes)
 __global__ void k_export(KArgs A, Store S, Store O, const int *perm, const int *key, Tiles Tl,
-                         long long np, const int32_t *itag, long long np0, double *r,
+                         long long np, const int32_t *itag, double *r,
                          int32_t *iv, long long cap, int regs_dead, int r_other, int migrate) {
   GRID_STRIDE(q, np) {
     const int pq = perm[q];
@@ -3651,7 +3658,11 @@ __global__ void k_export(KArgs A, Store S, Store O, const int *perm, const int *
     r[(long long)DK_IPM*cap + q] = static_cast<double>(S.M(q));
     iv[(long long)DK_PGID*cap + q] = s.gid;
     const int o = S.ORIG(q);
-    for (int c=1; c<DK_NIDATA; ++c) iv[(long long)c*cap + q] = itag[(long long)(c - 1)*np0 + o];
+    const int4 tg = *reinterpret_cast<const int4*>(itag + kTags*o);
+    iv[(long long)1*cap + q] = tg.x;
+    iv[(long long)2*cap + q] = tg.y;
+    iv[(long long)3*cap + q] = tg.z;
+    iv[(long long)4*cap + q] = tg.w;
   }
 }
 
@@ -3742,27 +3753,42 @@ KArgs ClassArgs(const dk_ctx *c, const KArgs &A0, int cls, bool &sy);
 // (mid: the pc2 stage-2 form).  Without the shearing box over the two item classes of the tile
 // kernels, one workgroup per item each (the lists of the last sort describe the present order);
 // in the shearing box over all items, the extra parts in a looping launch.
-void LaunchKey(dk_ctx *c, const KArgs &A, int do_key, double *pres, bool mid = false) {
+// pres null: the pending correction alone.
+void LaunchKey(dk_ctx *c, const KArgs &A, double *pres, bool mid = false) {
   const Fast *f = c->fast;
   const size_t lds = LdsKey(f->T, f->key_threads);
+  const int nt = f->key_threads;
+  if (pres == nullptr) {
+    if (!f->T.SY) {
+      bool sy;
+      for (int cls = 0; cls < 2; ++cls) {
+        const KArgs Ac = ClassArgs(c, A, cls, sy);
+        k_key<false, false, false, false><<<Ac.nfirst, nt, lds, c->stream>>>(Ac, pres, c->d_blocks);
+      }
+      return;
+    }
+    k_key<false, false, false, false><<<f->T.nt, nt, lds, c->stream>>>(A, pres, c->d_blocks);
+    k_key<true, false, false, false><<<OverGrid(c), nt, lds, c->stream>>>(A, pres, c->d_blocks);
+    return;
+  }
   if (!f->T.SY) {
     bool sy;
     for (int cls = 0; cls < 2; ++cls) {
       const KArgs Ac = ClassArgs(c, A, cls, sy);
-      if (mid) k_key<false, true><<<Ac.nfirst, f->key_threads, lds, c->stream>>>(Ac, do_key, pres, c->d_blocks);
+      if (mid) k_key<false, true><<<Ac.nfirst, f->key_threads, lds, c->stream>>>(Ac, pres, c->d_blocks);
       else if (c->smr)
-        k_key<false, false, true><<<Ac.nfirst, f->key_threads, lds, c->stream>>>(Ac, do_key, pres, c->d_blocks);
-      else k_key<false><<<Ac.nfirst, f->key_threads, lds, c->stream>>>(Ac, do_key, pres, c->d_blocks);
+        k_key<false, false, true><<<Ac.nfirst, f->key_threads, lds, c->stream>>>(Ac, pres, c->d_blocks);
+      else k_key<false><<<Ac.nfirst, f->key_threads, lds, c->stream>>>(Ac, pres, c->d_blocks);
     }
     return;
   }
   if (mid) {
-    k_key<false, true><<<f->T.nt, f->key_threads, lds, c->stream>>>(A, do_key, pres, c->d_blocks);
-    k_key<true, true><<<OverGrid(c), f->key_threads, lds, c->stream>>>(A, do_key, pres, c->d_blocks);
+    k_key<false, true><<<f->T.nt, f->key_threads, lds, c->stream>>>(A, pres, c->d_blocks);
+    k_key<true, true><<<OverGrid(c), f->key_threads, lds, c->stream>>>(A, pres, c->d_blocks);
     return;
   }
-  k_key<false><<<f->T.nt, f->key_threads, lds, c->stream>>>(A, do_key, pres, c->d_blocks);
-  k_key<true><<<OverGrid(c), f->key_threads, lds, c->stream>>>(A, do_key, pres, c->d_blocks);
+  k_key<false><<<f->T.nt, f->key_threads, lds, c->stream>>>(A, pres, c->d_blocks);
+  k_key<true><<<OverGrid(c), f->key_threads, lds, c->stream>>>(A, pres, c->d_blocks);
 }
 
 // a deposit kernel of the scheme of the context with the x2-shift code SYV
@@ -3940,7 +3966,7 @@ KArgs MakeArgs(dk_ctx *c) {
   A.regs_live = !f->regs_dead;
   A.tree = c->tree;
   if (c->smr) {
-    A.plev = f->itag + (long long)(DK_PLEV - 1)*f->np;
+    A.plev = f->itag + (DK_PLEV - 1);
     A.xl_list = f->xl_list; A.xl_n = f->xl_n;
   }
   A.res = f->res; A.dc0 = f->dc[0]; A.dc1 = f->dc[1]; A.dc2 = f->dc[2];
@@ -4084,7 +4110,7 @@ int Flush(dk_ctx *c) {
   Fast *f = c->fast;
   if (!f->pending) return DK_OK;
   KArgs A = MakeArgs(c);
-  TIMED("key", LaunchKey(c, A, 0, nullptr));
+  TIMED("flush", LaunchKey(c, A, nullptr));
   if (const int e = FixKey(c, A, nullptr)) return e;
   dk_gas_src z;
   std::memset(&z, 0, sizeof(z));
@@ -4281,10 +4307,10 @@ int FastExport(dk_ctx *c) {
   if ((e = Flush(c))) return e;
   KArgs A = MakeArgs(c);
   A.gam0 = 1.0; A.gam1 = 0.0; A.beta_dt = 0.0;
-  k_export<<<Grid(f->np), kBlock, 0, c->stream>>>(A, f->s[f->cur], f->s[1 - f->cur], f->perm,
-                                                   f->key, f->T, f->np, f->itag, f->np,
+  TIMED("export", (k_export<<<Grid(f->np), kBlock, 0, c->stream>>>(A, f->s[f->cur], f->s[1 - f->cur], f->perm,
+                                                   f->key, f->T, f->np, f->itag,
                                                    c->rdata, c->idata, (long long)c->cap,
-                                                   f->regs_dead, f->r_other, f->unmigrated);
+                                                   f->regs_dead, f->r_other, f->unmigrated)));
   return dk::Check(hipGetLastError());
 }
 
@@ -4297,7 +4323,7 @@ __global__ void k_fstop(Store S, long long np, const int32_t *itag, double *part
   double mx = 0.0, mn = 3.4028234663852886e38;
   GRID_STRIDE(q, np) {
     const double ts = static_cast<double>(S.TS(q));
-    const int sp = itag[(long long)(DK_PSP - 1)*np + S.ORIG(q)];
+    const int sp = itag[kTags*S.ORIG(q) + DK_PSP - 1];
     if (!isfinite(ts) || !(ts > 0.0) || sp < 0) {dk::RecordError(err, DK_ESTOP, q); continue;}
     mx = fmax(mx, ts);
     mn = fmin(mn, ts);
@@ -4316,20 +4342,44 @@ __global__ void k_fstop(Store S, long long np, const int32_t *itag, double *part
 
 // NewTimeStep over the store (dust_newdt.cpp:135-145, as the plain form's k_newdt): min over
 // particles of dx/max(|v|, 1e-30), the azimuthal velocity without the background shear in the
-// 3-D shearing box, every stopping time validated (dust_newdt.cpp:34-99); the block of slot q
-// from the last sort's key
-__global__ void k_fnewdt(const DevBlock *B, Store S, const int *perm, const int *key, Tiles Tl,
-                         long long np, double qo, double *partial, dk::ErrWord *err) {
+// 3-D shearing box, every stopping time validated (dust_newdt.cpp:34-99).  The store is
+// block-major: a workgroup takes an even run of slots and goes through the blocks in it, so a
+// thread keeps the largest speeds of a block and divides once (a rounded quotient falls as its
+// divisor grows: the minimum's bits are the same).  Bound by the reads (16 to 24 bytes a
+// particle: 0.67 ms for 117 million, 4.2 TB/s; with the block from the last sort's key through its
+// permutation and three FP64 divides a particle, 0.88).
+__global__ void __launch_bounds__(kBlock)
+k_fnewdt(const DevBlock *B, Store S, const int *start, long long keys_blk, int nmb, long long np,
+         double qo, double *partial, dk::ErrWord *err) {
   __shared__ double sh[kBlock];
   double dtmin = 3.4028234663852886e38;   // the largest float, the reference's start value
-  GRID_STRIDE(q, np) {
-    const int m = key[perm[q]]/Tl.TC/Tl.ntb;
-    const double ts = static_cast<double>(S.TS(q));
-    if (!isfinite(ts) || !(ts > 0.0)) dk::RecordError(err, DK_ESTOP, q);
-    const double vy = static_cast<double>(S.V(1, q)) - qo*S.X(0, q);
-    dtmin = fmin(B[m].dx1/fmax(fabs(static_cast<double>(S.V(0, q))), 1.0e-30), dtmin);
-    dtmin = fmin(B[m].dx2/fmax(fabs(vy), 1.0e-30), dtmin);
-    dtmin = fmin(B[m].dx3/fmax(fabs(static_cast<double>(S.V(2, q))), 1.0e-30), dtmin);
+  const long long q0 = np*blockIdx.x/gridDim.x, q1 = np*(blockIdx.x + 1LL)/gridDim.x;
+  // the block of the first slot: the last one that starts at or before it
+  int m = 0;
+  for (int hi = nmb; hi - m > 1; ) {
+    const int mid = (m + hi) >> 1;
+    if (start[mid*keys_blk] <= q0) m = mid;
+    else hi = mid;
+  }
+  for (long long a = q0; a < q1 && m < nmb; ++m) {
+    const long long e = min(q1, static_cast<long long>(start[(m + 1)*keys_blk]));
+    double sx = 1.0e-30, sy = 1.0e-30, sz = 1.0e-30;
+    bool any = false;
+    long long bad = -1;
+#pragma unroll 4
+    for (long long q = a + threadIdx.x; q < e; q += kBlock) {
+      const float ts = S.TS(q);
+      if (!isfinite(ts) || !(ts > 0.0f)) bad = q;
+      double vy = static_cast<double>(S.V(1, q));
+      if (qo != 0.0) vy -= qo*S.X(0, q);
+      sx = fmax(sx, fabs(static_cast<double>(S.V(0, q))));
+      sy = fmax(sy, fabs(vy));
+      sz = fmax(sz, fabs(static_cast<double>(S.V(2, q))));
+      any = true;
+    }
+    if (bad >= 0) dk::RecordError(err, DK_ESTOP, bad);
+    if (any) dtmin = fmin(fmin(dtmin, B[m].dx1/sx), fmin(B[m].dx2/sy, B[m].dx3/sz));
+    a = max(a, e);
   }
   sh[threadIdx.x] = dtmin;
   __syncthreads();
@@ -4354,8 +4404,9 @@ int FastNewDt(dk_ctx *c, double qo, double *partial, int nb) {
   if (f == nullptr || c->u0 == nullptr) return DK_ESTATE;
   int e;
   if ((e = Flush(c))) return e;
-  k_fnewdt<<<nb, kBlock, 0, c->stream>>>(c->d_blocks, f->s[f->cur], f->perm, f->key, f->T,
-                                          f->np, qo, partial, c->d_err);
+  TIMED("newdt", (k_fnewdt<<<nb, kBlock, 0, c->stream>>>(
+      c->d_blocks, f->s[f->cur], f->start, (long long)f->T.ntb*f->T.TC, c->g.nmb, f->np, qo,
+      partial, c->d_err)));
   return dk::Check(hipGetLastError());
 }
 
@@ -4433,7 +4484,7 @@ static int FastStagePc2(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
     const long long nin = (long long)gg.nmb*(gg.n1 - 2)*(gg.n2 - 2)*(gg.n3 - 2);
     TIMED("cloud_pack", (k_fpack<<<Grid(nin), kBlock, 0, c->stream>>>(gg, f->ustar, f->cpack)));
   }
-  TIMED("key", LaunchKey(c, A, 1, f->pres[1 - f->pres_rd], !s1));
+  TIMED("key", LaunchKey(c, A, f->pres[1 - f->pres_rd], !s1));
   if ((e = FixKey(c, A, f->pres[1 - f->pres_rd]))) return e;
   if ((e = SortKeys(c))) return e;
   if ((e = BuildItems(c))) return e;
@@ -4508,7 +4559,7 @@ int FastStage(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
   }
   // 1. key pass (with the pending correction), histogram
   // the push of this stage writes its residue into the buffer the next stage's start reads
-  TIMED("key", LaunchKey(c, A, 1, f->pres[1 - f->pres_rd]));
+  TIMED("key", LaunchKey(c, A, f->pres[1 - f->pres_rd]));
   if (f->x3p != nullptr)   // the outflow ledger (bvals_part.cpp:184-186) of the items just run
     TIMED("x3_ledger", (k_x3part<<<kX3Groups, 256, 0, c->stream>>>(
                             f->item_start, T.nt, f->x3p, f->x3p + 2*(size_t)f->item_cap),
