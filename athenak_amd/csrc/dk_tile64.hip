@@ -19,10 +19,10 @@
 // The order of a cell's additions is not fixed (as with the per-particle atomics).
 //
 // Measured, per launch, per-particle kernels -> tile kernels with their combine: 8.4 million
-// particles on 128^3 cells (shearing box), deposit of Q, P 33.5 -> 0.90 ms, operator 25.6 -> 0.70,
-// kick 25.8 -> 0.92, the bins of a stage 0.14 ms; 2.1 million, half of them in clumps, 11.7 ->
-// 0.24, 8.8 -> 0.18, 8.9 -> 0.22 ms; pc2 predictor and advance of 1 million in uneven blocks
-// 5.5 -> 0.20 and 4.3 -> 0.20 ms.
+// particles on 128^3 cells (shearing box), deposit of Q, P 33.5 -> 0.50 ms, operator 25.6 -> 0.55,
+// kick 25.8 -> 0.73, the bins of a stage 0.14 ms; 2.1 million, half of them in clumps, 11.7 ->
+// 0.14, 8.8 -> 0.15, 8.9 -> 0.18 ms; pc2 predictor and advance of 1 million in uneven blocks
+// 5.5 -> 0.18 and 4.3 -> 0.14 ms.
 
 #include <hip/hip_runtime.h>
 
@@ -40,14 +40,22 @@ using dk::Stencil;
 namespace {
 
 constexpr int kTX = 8, kTY = 4, kTZ = 4, kTC = kTX*kTY*kTZ;   // cells of a tile
-constexpr int kNT = 3*kTC;        // threads of a tile kernel: one per (cell, slab)
+// threads of a tile kernel: one wavefront per SIMD, so that a CU holds as many workgroups as a SIMD
+// holds wavefronts (three at the 130 to 167 registers of the nine sums of three or four values).
+// Six wavefronts, one thread per (cell, slab), load two SIMDs twice: one workgroup a CU for the
+// deposit and two for the others (8.4 million particles: deposit 0.83 -> 0.42, operator 0.63 ->
+// 0.47, kick 0.84 -> 0.65 ms)
+constexpr int kNT = 256;
 // particles of a chunk: 512, the mean of a tile at 4 particles per cell, and three standard
 // deviations of a random filling, so that such a tile is one chunk; the records of 576 keep
 // three workgroups on a CU (52 KB of LDS each)
 constexpr int kChunk = 576;
 constexpr int kPer = (kChunk + kNT - 1)/kNT;
 constexpr int kItemMax = 2*kChunk;
-constexpr int kRun = 8;           // records a thread sums before it adds to the region
+// records a thread sums before it adds to the region: longer runs add less often, shorter ones
+// spread a crowded cell over more threads (2.1 million particles, half of them in clumps: the three
+// passes 1.41 ms at 4, 1.08 at 6, 0.97 at 8, 0.86 at 12 and 16; even fillings alike from 6 on)
+constexpr int kRun = 16;
 // the centre cells of a tile's particles: its own, and in the shearing box those one row off in x2
 // (every particle belongs to the tile of its cell clamped into the block)
 constexpr int kCellMax = kTX*(kTY + 2)*kTZ;
@@ -377,7 +385,7 @@ __host__ __device__ constexpr size_t Lds64(int RN) {
 }
 
 template <int OP>
-__global__ void __launch_bounds__(kNT) k_t64(Args64 A) {
+__global__ void __launch_bounds__(kNT, 3) k_t64(Args64 A) {
   constexpr int NC = NComp<OP>();
   extern __shared__ double lds[];
   const Geo &g = A.g;
