@@ -1804,12 +1804,20 @@ __global__ void __launch_bounds__(kLongThreads) k_longsort(const int *start, con
   }
 }
 
+// Registers of the tile kernels (the second argument of their launch bounds): their workgroups are
+// six wavefronts, which load two of a CU's SIMDs twice, so a CU holds half as many workgroups as
+// a SIMD holds wavefronts, and an odd number of wavefronts is worth no more than the even one below
+// it.  Measured per launch, 5 or 4 -> 6 wavefronts a SIMD: P1's crowded-cell code 1.30 -> 1.12 ms
+// (128^3 clumps), P2 and P3 on the x2 faces of a sheared block 0.305 -> 0.297 and 0.354 -> 0.347
+// (128^3); the pc2 predictor to 8 and the advance to 6 0.61 -> 0.57 and 0.65 -> 0.63 (128^3).  Left at
+// 4: the cloud kernels (2.4 -> 2.8 ms, spills) and the crowded-cell code of P2 and P3 (0.79 -> 0.81).
+
 //----------------------------------------------------------------------------------------
 // P1: the pushed particles (the key pass pushed them in place) gathered into the new order, and
 // the deposit of Q = sum m c W/V and P = sum m c W v/V (dust_pm.cpp:225-274) and of the centre
 // mass m c/V (dust_pm.cpp:660-667)
 template <int S, bool SY, bool OV, bool SPLIT = false>
-__global__ void __launch_bounds__(kCellThreads, (SY || OV || SPLIT) ? 4 : 6)
+__global__ void __launch_bounds__(kCellThreads, 6)
 k_p1(KArgs A, float *qt0, float *qt1, float *qt2, float *scr, const DevBlock *__restrict__ Bk) {
   extern __shared__ double lds_d[];
   const Geo &g = A.g;
@@ -1973,7 +1981,7 @@ k_p1(KArgs A, float *qt0, float *qt1, float *qt2, float *scr, const DevBlock *__
 
 // P2: the particle part of the dc1 operator, result += G^T (m c/V) G u* (dust_solver.cpp:151-201)
 template <int S, bool SY, bool OV, bool SPLIT = false>
-__global__ void __launch_bounds__(kCellThreads, (SY || OV || SPLIT) ? 4 : 8)
+__global__ void __launch_bounds__(kCellThreads, SY ? 6 : ((OV || SPLIT) ? 4 : 8))
 k_p2(KArgs A, const float *us, float *scr, const DevBlock *__restrict__ Bk) {
   extern __shared__ double lds_d[];
   const Geo &g = A.g;
@@ -2266,13 +2274,13 @@ __device__ inline void P3Body(const KArgs &A, const float *us, float *scr, doubl
 }
 
 template <int S, bool SY, bool OV, bool SPLIT = false>
-__global__ void __launch_bounds__(kCellThreads, (SY || OV || SPLIT) ? 4 : 8)
+__global__ void __launch_bounds__(kCellThreads, SY ? 6 : ((OV || SPLIT) ? 4 : 8))
 k_p3(KArgs A, const float *us, float *scr, double *defect, const DevBlock *__restrict__ Bk) {
   P3Body<S, SY, true, OV, SPLIT>(A, us, scr, defect, Bk);
 }
 
 template <int S, bool SY, bool OV, bool SPLIT = false>
-__global__ void __launch_bounds__(kCellThreads, (SY || OV || SPLIT) ? 4 : 8)
+__global__ void __launch_bounds__(kCellThreads, SY ? 6 : ((OV || SPLIT) ? 4 : 8))
 k_p3n(KArgs A, const float *us, float *scr, double *defect, const DevBlock *__restrict__ Bk) {
   P3Body<S, SY, false, OV, SPLIT>(A, us, scr, defect, Bk);
 }
@@ -2284,7 +2292,7 @@ k_p3n(KArgs A, const float *us, float *scr, double *defect, const DevBlock *__re
 // the source order (the next key pass and an export read them through this sort's permutation).
 // (CLOUD: refinable clouds at the mesh level, the linear gather from the 12-component pack uv)
 template <int S, bool OV, bool SPLIT = false, bool CLOUD = false>
-__global__ void __launch_bounds__(kCellThreads, (OV || SPLIT || CLOUD) ? 4 : 6)
+__global__ void __launch_bounds__(kCellThreads, CLOUD ? 4 : ((OV || SPLIT) ? 6 : 8))
 k_pp(KArgs A, const float *uv, float *scr, const DevBlock *__restrict__ Bk) {
   extern __shared__ double lds_d[];
   const Geo &g = A.g;
@@ -2439,7 +2447,7 @@ k_pp(KArgs A, const float *uv, float *scr, const DevBlock *__restrict__ Bk) {
 // the impulse is deposited in FP32 and every tile's FP64 defect goes to the combine.
 // (CLOUD: as k_pp, the linear gather from the 12-component pack us of u*)
 template <int S, bool OV, bool SPLIT = false, bool CLOUD = false>
-__global__ void __launch_bounds__(kCellThreads, 4)
+__global__ void __launch_bounds__(kCellThreads, CLOUD ? 4 : 6)
 k_pa(KArgs A, const float *us, float *scr, double *defect, const DevBlock *__restrict__ Bk) {
   extern __shared__ double lds_d[];
   const Geo &g = A.g;
