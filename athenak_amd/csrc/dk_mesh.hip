@@ -294,43 +294,79 @@ __device__ inline void ShellCell(const Geo &g, unsigned s, int &i, int &j, int &
 // shear-periodic x1 face are left to k_fold_shear.
 constexpr int kFoldVars = 5;
 
+// Bound by latency (2 to 20 thousand cells, 26 dependent look-ups a cell at 32^3 cells).  So
+// the block's neighbours are looked up once per workgroup, and where a block is at least 2 ng cells
+// wide (a cell is near at most one face per axis: 7 strips) all strips' values are loaded before
+// the first is added (15 -> 7 us; 22 x 18 x 26 cell blocks with walls, 26 -> 8 us).
 template <typename T>
-__global__ void k_fold(Geo g, const DevBlock *B, const int *slot_dir, T *a, int nvar) {
-  __shared__ int sdir[26];
+__global__ void __launch_bounds__(kBlock) k_fold(Geo g, const DevBlock *B, const int *slot_dir,
+                                                 T *a, int nvar) {
+  __shared__ int sdir[26], snb[27];
+  const int m = blockIdx.y;
   if (threadIdx.x < 26) sdir[threadIdx.x] = slot_dir[threadIdx.x];
+  if (threadIdx.x < 27) {
+    // (on a refined mesh only same-level neighbours fold: no deposit of the FP32 tile kernels
+    // reaches a region of another level, whose clouds go to the leaf traversal)
+    const int d = threadIdx.x, o1 = d % 3;
+    const DevBlock &bm = B[m];
+    int nb = bm.nghbr[d];
+    if (nb >= 0 && B[nb].level != bm.level) nb = -1;
+    if (g.bc_x1 == DK_X1_SHEAR &&
+        ((o1 == 0 && bm.lx1 == 0) || (o1 == 2 && bm.lx1 == g.nmbx1 - 1)))
+      nb = -1;
+    snb[d] = nb;
+  }
   __syncthreads();
   const unsigned nsh = static_cast<unsigned>(ShellCount(g));
-  const bool shear = (g.bc_x1 == DK_X1_SHEAR);
-  const int m = blockIdx.y;
+  const bool wide = g.nx1 >= 2*g.ng && g.nx2 >= 2*g.ng && g.nx3 >= 2*g.ng;
   BLOCK_STRIDE(t, nsh) {
     int i, j, k;
     ShellCell(g, t, i, j, k);
-    const DevBlock &bm = B[m];
-    // the allowed offsets per axis: bit (o + 1) set when offset o covers this cell
-    const int a1 = 2 | ((i < g.is + g.ng) ? 1 : 0) | ((i > g.ie - g.ng) ? 4 : 0);
-    const int a2 = 2 | ((j < g.js + g.ng) ? 1 : 0) | ((j > g.je - g.ng) ? 4 : 0);
-    const int a3 = 2 | ((k < g.ks + g.ng) ? 1 : 0) | ((k > g.ke - g.ng) ? 4 : 0);
+    const bool l1 = i < g.is + g.ng, h1 = i > g.ie - g.ng, l2 = j < g.js + g.ng;
+    const bool h2 = j > g.je - g.ng, l3 = k < g.ks + g.ng, h3 = k > g.ke - g.ng;
     // every variable's sum in slot order (at most kFoldVars variables: the deposits fold 3-5)
     T sum[kFoldVars];
 #pragma unroll
     for (int v=0; v<kFoldVars; ++v) sum[v] = (v < nvar) ? a[Idx(g, m, nvar, v, k, j, i)] : T(0);
-    for (int s=0; s<26; ++s) {
-      const int d = sdir[s];
-      const int o1 = d % 3, o2 = (d/3) % 3, o3 = d/9;
-      if (!((a1 >> o1) & 1) || !((a2 >> o2) & 1) || !((a3 >> o3) & 1)) continue;
-      const int nb = bm.nghbr[d];
-      // (on a refined mesh only same-level neighbours fold: no deposit of the FP32 tile
-      // kernels reaches a region of another level, whose clouds go to the leaf traversal)
-      if (nb < 0 || B[nb].level != bm.level) continue;
-      if (shear && o1 != 1) {
-        const bool crosses = (o1 == 0) ? (bm.lx1 == 0) : (bm.lx1 == g.nmbx1 - 1);
-        if (crosses) continue;
-      }
-      const long long src = Idx(g, nb, nvar, 0, k - (o3 - 1)*g.nx3, j - (o2 - 1)*g.nx2,
-                                i - (o1 - 1)*g.nx1);
+    if (wide) {
+      // the strips by the axes they cross (x1, x2, x3 as bits): 1 to 7 is the slots' order
+      const int o1 = l1 ? -1 : (h1 ? 1 : 0), o2 = l2 ? -1 : (h2 ? 1 : 0);
+      const int o3 = l3 ? -1 : (h3 ? 1 : 0);
+      const int cross = (o1 ? 1 : 0) | (o2 ? 2 : 0) | (o3 ? 4 : 0);
+      T val[7][kFoldVars];
+      unsigned have = 0;
 #pragma unroll
-      for (int v=0; v<kFoldVars; ++v)
-        if (v < nvar) sum[v] += a[src + v*g.ncb];
+      for (int c=1; c<8; ++c) {
+        const int p1 = (c & 1) ? o1 : 0, p2 = (c & 2) ? o2 : 0, p3 = (c & 4) ? o3 : 0;
+        const int nb = (c & ~cross) ? -1 : snb[Dir(p1, p2, p3)];
+#pragma unroll
+        for (int v=0; v<kFoldVars; ++v) val[c - 1][v] = T(0);
+        if (nb >= 0) {
+          have |= 1u << c;
+          const long long src = Idx(g, nb, nvar, 0, k - p3*g.nx3, j - p2*g.nx2, i - p1*g.nx1);
+#pragma unroll
+          for (int v=0; v<kFoldVars; ++v)
+            if (v < nvar) val[c - 1][v] = a[src + v*g.ncb];
+        }
+      }
+#pragma unroll
+      for (int c=1; c<8; ++c)
+        if ((have >> c) & 1)
+#pragma unroll
+          for (int v=0; v<kFoldVars; ++v) sum[v] += val[c - 1][v];
+    } else {
+      // the allowed offsets per axis: bit (o + 1) set when offset o covers this cell
+      const int a1 = 2 | (l1 ? 1 : 0) | (h1 ? 4 : 0), a2 = 2 | (l2 ? 1 : 0) | (h2 ? 4 : 0);
+      const int a3 = 2 | (l3 ? 1 : 0) | (h3 ? 4 : 0);
+      for (int s=0; s<26; ++s) {
+        const int d = sdir[s], o1 = d % 3, o2 = (d/3) % 3, o3 = d/9, nb = snb[d];
+        if (!((a1 >> o1) & (a2 >> o2) & (a3 >> o3) & 1) || nb < 0) continue;
+        const long long src = Idx(g, nb, nvar, 0, k - (o3 - 1)*g.nx3, j - (o2 - 1)*g.nx2,
+                                  i - (o1 - 1)*g.nx1);
+#pragma unroll
+        for (int v=0; v<kFoldVars; ++v)
+          if (v < nvar) sum[v] += a[src + v*g.ncb];
+      }
     }
 #pragma unroll
     for (int v=0; v<kFoldVars; ++v)
