@@ -330,8 +330,12 @@ __global__ void __launch_bounds__(kBlock) k_smr_cloud_predictor(
   __shared__ dk::CoopLeaf leaves[kBlock/kCoop][8];
   const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
   dk::CoopLeaf *lf = leaves[grp];
-  for (long long p = (long long)blockIdx.x*(kBlock/kCoop) + grp; p < np;
-       p += (long long)gridDim.x*(kBlock/kCoop)) {
+  const int nv = rate_dep ? 4 : 3;
+  dk::CoopHeld<4, double> sum;
+  const int run = dk::CoopRun(np);
+  const long long ngrp = (long long)gridDim.x*(kBlock/kCoop);
+  for (long long u = 0, p = ((long long)blockIdx.x*(kBlock/kCoop) + grp)*run; p < np;
+       ++u, p += (u % run) ? 1 : (ngrp - 1)*run + 1) {
     const double x[3] = {PR(DK_IPX,p), PR(DK_IPY,p), PR(DK_IPZ,p)};
     const dk::CoopCloud cl = dk::CoopSpans(g, B, t, cg, x, PI(DK_PLEV,p), lane, lf);
     if (cl.total < 0) {
@@ -347,13 +351,14 @@ __global__ void __launch_bounds__(kBlock) k_smr_cloud_predictor(
     dk::CoopCells<false>(cl, lf, x, lane,
         [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
           const double inv_volume = 1.0/(L.d[0]*L.d[1]*L.d[2]);
-          const long long i0 = Idx(g, L.b, 5, 1, k + g.ks, j + g.js, i + g.is);
-          unsafeAtomicAdd(&qdep[i0], inv_volume*w*gx);
-          unsafeAtomicAdd(&qdep[i0 + g.ncb], inv_volume*w*gy);
-          unsafeAtomicAdd(&qdep[i0 + 2*g.ncb], inv_volume*w*gz);
-          if (rate_dep) unsafeAtomicAdd(&qdep[i0 + 3*g.ncb], inv_volume*w*mass_rate);
+          sum.Take(qdep, g.ncb, 0, nv, Idx(g, L.b, 5, 1, k + g.ks, j + g.js, i + g.is));
+          sum.v[0] += inv_volume*w*gx;
+          sum.v[1] += inv_volume*w*gy;
+          sum.v[2] += inv_volume*w*gz;
+          sum.v[3] += inv_volume*w*mass_rate;
         });
   }
+  sum.Flush(qdep, g.ncb, 0, nv);
 }
 
 // CloudAdvanceT on a statically refined mesh (periodic, no shearing box)
@@ -364,8 +369,11 @@ __global__ void __launch_bounds__(kBlock) k_smr_cloud_advance(
   __shared__ dk::CoopLeaf leaves[kBlock/kCoop][8];
   const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
   dk::CoopLeaf *lf = leaves[grp];
-  for (long long p = (long long)blockIdx.x*(kBlock/kCoop) + grp; p < np;
-       p += (long long)gridDim.x*(kBlock/kCoop)) {
+  dk::CoopHeld<3, double> sum;
+  const int run = dk::CoopRun(np);
+  const long long ngrp = (long long)gridDim.x*(kBlock/kCoop);
+  for (long long u = 0, p = ((long long)blockIdx.x*(kBlock/kCoop) + grp)*run; p < np;
+       ++u, p += (u % run) ? 1 : (ngrp - 1)*run + 1) {
     const double x0[3] = {PR(DK_IPX1,p), PR(DK_IPY1,p), PR(DK_IPZ1,p)};
     const double v0[3] = {PR(DK_IPVX1,p), PR(DK_IPVY1,p), PR(DK_IPVZ1,p)};
     double xh[3];
@@ -401,10 +409,11 @@ __global__ void __launch_bounds__(kBlock) k_smr_cloud_advance(
     dk::CoopCells<false>(cl, lf, xh, lane,
         [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
           const double dw = mass*w/(L.d[0]*L.d[1]*L.d[2]);
-          const long long i0 = Idx(g, L.b, 3, 0, k + g.ks, j + g.js, i + g.is);
-          for (int d=0; d<3; ++d) unsafeAtomicAdd(&dmom[i0 + d*g.ncb], dw*dv[d]);
+          sum.Take(dmom, g.ncb, 0, 3, Idx(g, L.b, 3, 0, k + g.ks, j + g.js, i + g.is));
+          for (int d=0; d<3; ++d) sum.v[d] += dw*dv[d];
         });
   }
+  sum.Flush(dmom, g.ncb, 0, 3);
 }
 
 }  // namespace

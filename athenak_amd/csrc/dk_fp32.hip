@@ -2666,7 +2666,11 @@ __global__ void __launch_bounds__(kBlock) k_fxl_predictor(KArgs A, dk::CloudGeo 
   const int n = *A.xl_n;
   const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
   dk::CoopLeaf *lf = leaves[grp];
-  for (int t = blockIdx.x*(kBlock/kCoop) + grp; t < n; t += gridDim.x*(kBlock/kCoop)) {
+  const int from = A.rate_dep ? 0 : 1;
+  dk::CoopHeld<4, float> sum;
+  const int run = dk::CoopRun(n), ngrp = gridDim.x*(kBlock/kCoop);
+  for (long long u = 0, t = (long long)(blockIdx.x*(kBlock/kCoop) + grp)*run; t < n;
+       ++u, t += (u % run) ? 1 : (long long)(ngrp - 1)*run + 1) {
     const int q = A.xl_list[t];
     const double x[3] = {A.dst.X(0, q), A.dst.X(1, q), A.dst.X(2, q)};
     const int lev = A.plev[kTags*A.dst.ORIG(q)];
@@ -2684,12 +2688,12 @@ __global__ void __launch_bounds__(kBlock) k_fxl_predictor(KArgs A, dk::CloudGeo 
     dk::CoopCells<false>(cl, lf, x, lane,
         [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
           const double wv = w*A.B[L.b].ivol;
-          const long long i0 = Idx(g, L.b, 4, 0, k + g.ks, j + g.js, i + g.is);
-          if (A.rate_dep) unsafeAtomicAdd(&qdep[i0], static_cast<float>(wv*mrate));
-          for (int d=0; d<3; ++d)
-            unsafeAtomicAdd(&qdep[i0 + (1 + d)*g.ncb], static_cast<float>(wv*gi[d]));
+          sum.Take(qdep, g.ncb, from, 4, Idx(g, L.b, 4, 0, k + g.ks, j + g.js, i + g.is));
+          sum.v[0] += wv*mrate;
+          for (int d=0; d<3; ++d) sum.v[1 + d] += wv*gi[d];
         });
   }
+  sum.Flush(qdep, g.ncb, from, 4);
 }
 
 // CloudAdvanceT (src/dust/dust_cloud3d.cpp:1449-1536) with CloudPC2Push (:118-158): the gather
@@ -2703,7 +2707,10 @@ __global__ void __launch_bounds__(kBlock) k_fxl_advance(KArgs A, dk::CloudGeo cg
   const int grp = threadIdx.x/kCoop, lane = threadIdx.x & (kCoop - 1);
   dk::CoopLeaf *lf = leaves[grp];
   const float hf = static_cast<float>(0.5*A.dt);
-  for (int t = blockIdx.x*(kBlock/kCoop) + grp; t < n; t += gridDim.x*(kBlock/kCoop)) {
+  dk::CoopHeld<3, double> sum;
+  const int run = dk::CoopRun(n), ngrp = gridDim.x*(kBlock/kCoop);
+  for (long long u = 0, t = (long long)(blockIdx.x*(kBlock/kCoop) + grp)*run; t < n;
+       ++u, t += (u % run) ? 1 : (long long)(ngrp - 1)*run + 1) {
     const int q = A.xl_list[t];
     double x[3] = {A.dst.X(0, q), A.dst.X(1, q), A.dst.X(2, q)};
     float v[3] = {A.dst.V(0, q), A.dst.V(1, q), A.dst.V(2, q)};
@@ -2736,10 +2743,11 @@ __global__ void __launch_bounds__(kBlock) k_fxl_advance(KArgs A, dk::CloudGeo cg
     dk::CoopCells<false>(cl, lf, xh, lane,
         [&](const dk::CoopLeaf &L, int k, int j, int i, double w) {
           const double wv = fac*w*A.B[L.b].ivol;
-          const long long i0 = Idx(g, L.b, 3, 0, k + g.ks, j + g.js, i + g.is);
-          for (int d=0; d<3; ++d) unsafeAtomicAdd(&dmom[i0 + d*g.ncb], wv*dv[d]);
+          sum.Take(dmom, g.ncb, 0, 3, Idx(g, L.b, 3, 0, k + g.ks, j + g.js, i + g.is));
+          for (int d=0; d<3; ++d) sum.v[d] += wv*dv[d];
         });
   }
+  sum.Flush(dmom, g.ncb, 0, 3);
 }
 
 // the centre masses of a tile's later parts added in part order (thread per cell of the tiles
