@@ -1009,7 +1009,7 @@ __device__ inline void CloudGather(const Tiles &Tl, const float *pk, int rb, con
 
 // The tile scratch holds the regions row by row: one row of the scratch is the x1 rows (RX
 // values each) of the regions of all tiles of a block that share (tz, ty, component, rz, ry), in
-// tx order, so that the combine reads consecutive cells of a padded row from consecutive words.
+// tx order, so that the fold reads consecutive cells of a padded row from consecutive words.
 __host__ __device__ inline long long ScrRow(const Tiles &T, int m, int tz, int ty, int nv, int v,
                                             int rz, int ry) {
   return ((((((long long)m*T.ntz + tz)*T.nty + ty)*nv + v)*T.RZ + rz)*T.RY + ry)*
@@ -2116,7 +2116,7 @@ k_p2(KArgs A, const float *us, float *scr, const DevBlock *__restrict__ Bk) {
 
 // P3: gather u*, kick, drag rate, and the deposit of the actual impulse (dust_pm.cpp:500-564).
 // The impulse is deposited in FP32; the tile's defect, the FP64 sum of its particles' impulses
-// minus the FP64 sum of its FP32 region, goes to the combine, which adds it to the tile's first
+// minus the FP64 sum of its FP32 region, goes to the fold, which adds it to the tile's first
 // cell: the FP64 field then holds exactly (to FP64 round-off) the particles' total impulse.
 // (REGS: the drag rate R is written, for a later stage; a template argument, as a run-time test
 // around the store costs the kernel registers)
@@ -2444,7 +2444,7 @@ k_pp(KArgs A, const float *uv, float *scr, const DevBlock *__restrict__ Bk) {
 // x = x0 + dt vh, and the deposit of the impulse -m (v - v0)/V at xh (dmom, dust_push.cpp:
 // 226-244).  v - v0 = dt (u* - vh)/t_s in exact arithmetic; the impulse and R take the exact
 // difference of the FP32 velocities, so that the gas receives the dust's actual change.  As P3:
-// the impulse is deposited in FP32 and every tile's FP64 defect goes to the combine.
+// the impulse is deposited in FP32 and every tile's FP64 defect goes to the fold.
 // (CLOUD: as k_pp, the linear gather from the 12-component pack us of u*)
 template <int S, bool OV, bool SPLIT = false, bool CLOUD = false>
 __global__ void __launch_bounds__(kCellThreads, CLOUD ? 4 : 6)

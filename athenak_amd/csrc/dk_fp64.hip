@@ -1,9 +1,11 @@
 // dk_fp64.hip -- context management and the plain FP64 form of the drag coupling.
 //
-// One kernel per reference kernel, thread per particle or per cell, deposits with hardware
-// FP64 atomics, operating in place on the caller's particle SoA and gas arrays.  This is the
-// baseline form the FP32 cell-sorted form is measured against.  Each kernel cites the
-// reference lambda it computes; the arithmetic is written in the reference's operation order.
+// One kernel per reference kernel, thread per particle or per cell, operating in place on the
+// caller's particle SoA and gas arrays; the particle-mesh passes run tile by tile (dk_tile64.hip),
+// or per particle with hardware FP64 atomics where the tiles do not pay or fit (T64Use,
+// T64Reserve).  This is the baseline form the FP32 cell-sorted form is measured against.  Each
+// kernel cites the reference lambda it computes; the arithmetic is written in the reference's
+// operation order.
 
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
