@@ -170,6 +170,15 @@ __device__ inline void Weights(int scheme, double d, double w[3]) {
   }
 }
 
+__device__ inline Stencil MakeW(const Geo &g, const Place &L) {
+  Stencil w;
+  w.ip = L.ic + g.is; w.jp = L.jc + g.js; w.kp = L.kc + g.ks;
+  Weights(g.deposit, L.dx, w.wx);
+  Weights(g.deposit, L.dy, w.wy);
+  Weights(g.deposit, L.dz, w.wz);
+  return w;
+}
+
 //----------------------------------------------------------------------------------------
 // the bins
 
@@ -267,8 +276,8 @@ __global__ void k_t64_place(const int *key, const int *rank, const int *start, l
 //----------------------------------------------------------------------------------------
 // the tile kernels
 
-// a particle whose centre cell lies outside the tile's cells: gathered from and deposited into
-// the padded fields directly (as the per-particle kernels)
+// a particle whose centre cell lies outside the tile's cells, or whose numbers are not finite:
+// gathered from and deposited into the padded fields directly (as the per-particle kernels)
 template <int NC>
 __device__ inline void FarDeposit(const Args64 &A, int m, const Stencil &w, const double val[NC]) {
   for (int c=0; c<3; ++c)
@@ -286,6 +295,7 @@ __device__ inline void FarDeposit(const Args64 &A, int m, const Stencil &w, cons
 template <int OP>
 __device__ inline void FarGather(const Args64 &A, int m, const Stencil &w, double u[3]) {
   constexpr int nv = (OP == kPredict) ? DK_NGAS : 3;
+  for (int d=0; d<3; ++d) u[d] = 0.0;
   for (int c=0; c<3; ++c)
     for (int bb=0; bb<3; ++bb) {
       const double wcb = w.wz[c]*w.wy[bb];
@@ -303,6 +313,18 @@ __device__ inline void FarGather(const Args64 &A, int m, const Stencil &w, doubl
     }
 }
 
+template <int N>
+__device__ inline bool Finite(const double x[N]) {
+  bool ok = true;
+#pragma unroll
+  for (int n=0; n<N; ++n) ok = ok && isfinite(x[n]);
+  return ok;
+}
+
+// fac x; a particle without mass (fac 0) gives nothing whatever its velocity, as the per-particle
+// kernels pass it over (the predictor's do not: its rate is no factor of the stencil's weights)
+__device__ inline double Share(double fac, double x) { return (fac == 0.0) ? 0.0 : fac*x; }
+
 // the particle's work of a pass: u, the gathered velocity; val, what it deposits per unit weight
 template <int OP>
 __device__ inline void Work(const Args64 &A, const DevBlock &b, long long p, const double u[3],
@@ -314,10 +336,10 @@ __device__ inline void Work(const Args64 &A, const DevBlock &b, long long p, con
   if constexpr (OP == kScatter) {
     const double muc = mass*(A.a_dt/(ts + A.a_dt))/vol;
     val[0] = muc;
-    for (int d=0; d<3; ++d) val[1 + d] = muc*r[(long long)(DK_IPVX + 2*d)*cap + p];
+    for (int d=0; d<3; ++d) val[1 + d] = Share(muc, r[(long long)(DK_IPVX + 2*d)*cap + p]);
   } else if constexpr (OP == kOper) {
     const double fac = mass*(A.a_dt/(ts + A.a_dt))/vol;
-    for (int d=0; d<3; ++d) val[d] = fac*u[d];
+    for (int d=0; d<3; ++d) val[d] = Share(fac, u[d]);
   } else if constexpr (OP == kKick) {
     const double cj = A.a_dt/(ts + A.a_dt), fac = -mass/vol;
     for (int d=0; d<3; ++d) {
@@ -325,7 +347,7 @@ __device__ inline void Work(const Args64 &A, const DevBlock &b, long long p, con
       const double dv = cj*(u[d] - v);
       v += dv;
       r[(long long)(DK_IPRX + d)*cap + p] = dv/A.a_dt;
-      val[d] = fac*dv;
+      val[d] = Share(fac, dv);
     }
   } else if constexpr (OP == kPredict) {
     const double rate = mass/(ts*vol);
@@ -364,7 +386,7 @@ __device__ inline void Work(const Args64 &A, const DevBlock &b, long long p, con
       r[(long long)(DK_IPX1 + 2*d)*cap + p] = xh[d];
       const double dv = dt*(u[d] - vh[d])/ts;
       r[(long long)(DK_IPRX + d)*cap + p] = dv;
-      val[d] = fac*dv;
+      val[d] = Share(fac, dv);
     }
   }
 }
@@ -485,47 +507,49 @@ __global__ void __launch_bounds__(kNT, 3) k_t64(Args64 A) {
       if (p[k] < 0) continue;
       double val[NC];
       double u[3] = {0.0, 0.0, 0.0};
-      if (cell[k] < 0) {
-        // outside the tile's cells: directly on the fields, inside the padded block only
-        Stencil w;
-        w.ip = L[k].ic + g.is; w.jp = L[k].jc + g.js; w.kp = L[k].kc + g.ks;
-        Weights(g.deposit, L[k].dx, w.wx);
-        Weights(g.deposit, L[k].dy, w.wy);
-        Weights(g.deposit, L[k].dz, w.wz);
+      const bool far = cell[k] < 0;
+      if (__builtin_expect(far, 0)) {
+        // outside the tile's cells: inside the padded block only
+        const Stencil w = MakeW(g, L[k]);
         if (!((OP == kScatter) ? dk::HaloOK(g, w) : dk::InPad(g, w))) {
           dk::RecordError(A.err, DK_EHALO, p[k]);
           continue;
         }
-        if constexpr (Gathers<OP>()) FarGather<OP>(A, m, w, u);
-        Work<OP>(A, b, p[k], u, val);
-        if (A.br) FarDeposit<NC>(A, m, w, val);
-        continue;
       }
       if constexpr (Gathers<OP>()) {
-        double wx[3], wy[3], wz[3];
-        Weights(g.deposit, L[k].dx, wx);
-        Weights(g.deposit, L[k].dy, wy);
-        Weights(g.deposit, L[k].dz, wz);
-        const int rb = ((L[k].kc - ck0)*T.RY + (L[k].jc - cj0 + T.SY))*T.RX + (L[k].ic - ci0);
+        if (!far) {
+          double wx[3], wy[3], wz[3];
+          Weights(g.deposit, L[k].dx, wx);
+          Weights(g.deposit, L[k].dy, wy);
+          Weights(g.deposit, L[k].dz, wz);
+          const int rb = ((L[k].kc - ck0)*T.RY + (L[k].jc - cj0 + T.SY))*T.RX + (L[k].ic - ci0);
 #pragma unroll
-        for (int c=0; c<3; ++c)
+          for (int c=0; c<3; ++c)
 #pragma unroll
-          for (int bb=0; bb<3; ++bb) {
-            const double wcb = wz[c]*wy[bb];
-            const int row = rb + (c*T.RY + bb)*T.RX;
+            for (int bb=0; bb<3; ++bb) {
+              const double wcb = wz[c]*wy[bb];
+              const int row = rb + (c*T.RY + bb)*T.RX;
 #pragma unroll
-            for (int a=0; a<3; ++a) {
-              const double ww = wcb*wx[a];
+              for (int a=0; a<3; ++a) {
+                const double ww = wcb*wx[a];
 #pragma unroll
-              for (int d=0; d<3; ++d) u[d] += ww*us[d*T.RN + row + a];
+                for (int d=0; d<3; ++d) u[d] += ww*us[d*T.RN + row + a];
+              }
             }
-          }
+        }
+        // The sums over the tile multiply the rows of weight zero too, which the per-particle
+        // kernels pass over: the same for finite numbers.  So a particle that gathers or gives
+        // what is not finite goes their way.
+        if (__builtin_expect(far || !Finite<3>(u), 0)) FarGather<OP>(A, m, MakeW(g, L[k]), u);
       }
       Work<OP>(A, b, p[k], u, val);
+      const bool direct = far || !Finite<NC>(val);
+      if (__builtin_expect(direct && A.br, 0)) FarDeposit<NC>(A, m, MakeW(g, L[k]), val);
+      if (far) continue;
       const int at = cst[cell[k]] + rk[k];
       rec[at] = L[k].dx; rec[kChunk + at] = L[k].dy; rec[2*kChunk + at] = L[k].dz;
 #pragma unroll
-      for (int v=0; v<NC; ++v) rec[(3 + v)*kChunk + at] = val[v];
+      for (int v=0; v<NC; ++v) rec[(3 + v)*kChunk + at] = direct ? 0.0 : val[v];
     }
     __syncthreads();
     // 4. the runs' sums, per slab, into the region
