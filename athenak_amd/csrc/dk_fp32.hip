@@ -4333,14 +4333,13 @@ int FastExport(dk_ctx *c) {
 // RefreshStoppingTimeMaximum over the store (dust_newdt.cpp:34-98, as the plain form's
 // k_stop_partial): per workgroup the largest and smallest (FP32) stopping time, an invalid one
 // recorded
-__global__ void k_fstop(Store S, long long np, const int32_t *itag, double *partial,
-                        dk::ErrWord *err) {
+__global__ void k_fstop(Store S, long long np, const int32_t *itag, double *partial) {
   __shared__ double smax[kBlock], smin[kBlock];
   double mx = 0.0, mn = 3.4028234663852886e38;
   GRID_STRIDE(q, np) {
     const double ts = static_cast<double>(S.TS(q));
     const int sp = itag[kTags*S.ORIG(q) + DK_PSP - 1];
-    if (!isfinite(ts) || !(ts > 0.0) || sp < 0) {dk::RecordError(err, DK_ESTOP, q); continue;}
+    if (!isfinite(ts) || !(ts > 0.0) || sp < 0) {mn = -1.0; continue;}
     mx = fmax(mx, ts);
     mn = fmin(mn, ts);
   }
@@ -4358,7 +4357,8 @@ __global__ void k_fstop(Store S, long long np, const int32_t *itag, double *part
 
 // NewTimeStep over the store (dust_newdt.cpp:135-145, as the plain form's k_newdt): min over
 // particles of dx/max(|v|, 1e-30), the azimuthal velocity without the background shear in the
-// 3-D shearing box, every stopping time validated (dust_newdt.cpp:34-99).  The store is
+// 3-D shearing box, every stopping time validated (dust_newdt.cpp:34-99; -1 where one is invalid,
+// as the plain form).  The store is
 // block-major: a workgroup takes an even run of slots and goes through the blocks in it, so a
 // thread keeps the largest speeds of a block and divides once (a rounded quotient falls as its
 // divisor grows: the minimum's bits are the same).  Bound by the reads (16 to 24 bytes a
@@ -4366,7 +4366,7 @@ __global__ void k_fstop(Store S, long long np, const int32_t *itag, double *part
 // permutation and three FP64 divides a particle, 0.88).
 __global__ void __launch_bounds__(kBlock)
 k_fnewdt(const DevBlock *B, Store S, const int *start, long long keys_blk, int nmb, long long np,
-         double qo, double *partial, dk::ErrWord *err) {
+         double qo, double *partial) {
   __shared__ double sh[kBlock];
   double dtmin = 3.4028234663852886e38;   // the largest float, the reference's start value
   const long long q0 = np*blockIdx.x/gridDim.x, q1 = np*(blockIdx.x + 1LL)/gridDim.x;
@@ -4381,11 +4381,10 @@ k_fnewdt(const DevBlock *B, Store S, const int *start, long long keys_blk, int n
     const long long e = min(q1, static_cast<long long>(start[(m + 1)*keys_blk]));
     double sx = 1.0e-30, sy = 1.0e-30, sz = 1.0e-30;
     bool any = false;
-    long long bad = -1;
 #pragma unroll 4
     for (long long q = a + threadIdx.x; q < e; q += kBlock) {
       const float ts = S.TS(q);
-      if (!isfinite(ts) || !(ts > 0.0f)) bad = q;
+      if (!isfinite(ts) || !(ts > 0.0f)) dtmin = -1.0;
       double vy = static_cast<double>(S.V(1, q));
       if (qo != 0.0) vy -= qo*S.X(0, q);
       sx = fmax(sx, fabs(static_cast<double>(S.V(0, q))));
@@ -4393,7 +4392,6 @@ k_fnewdt(const DevBlock *B, Store S, const int *start, long long keys_blk, int n
       sz = fmax(sz, fabs(static_cast<double>(S.V(2, q))));
       any = true;
     }
-    if (bad >= 0) dk::RecordError(err, DK_ESTOP, bad);
     if (any) dtmin = fmin(fmin(dtmin, B[m].dx1/sx), fmin(B[m].dx2/sy, B[m].dx3/sz));
     a = max(a, e);
   }
@@ -4411,7 +4409,7 @@ k_fnewdt(const DevBlock *B, Store S, const int *start, long long keys_blk, int n
 int FastStoppingTimes(dk_ctx *c, double *partial, int nb) {
   Fast *f = c->fast;
   if (f == nullptr) return DK_ESTATE;
-  k_fstop<<<nb, kBlock, 0, c->stream>>>(f->s[f->cur], f->np, f->itag, partial, c->d_err);
+  k_fstop<<<nb, kBlock, 0, c->stream>>>(f->s[f->cur], f->np, f->itag, partial);
   return dk::Check(hipGetLastError());
 }
 
@@ -4422,7 +4420,7 @@ int FastNewDt(dk_ctx *c, double qo, double *partial, int nb) {
   if ((e = Flush(c))) return e;
   TIMED("newdt", (k_fnewdt<<<nb, kBlock, 0, c->stream>>>(
       c->d_blocks, f->s[f->cur], f->start, (long long)f->T.ntb*f->T.TC, c->g.nmb, f->np, qo,
-      partial, c->d_err)));
+      partial)));
   return dk::Check(hipGetLastError());
 }
 

@@ -538,14 +538,15 @@ __global__ void __launch_bounds__(64) k_stiff_record(const double *partial, int 
 }
 
 // RefreshStoppingTimeMaximum (dust_newdt.cpp:34-98): per workgroup the largest and smallest
-// stopping time, an invalid one (not finite, not positive, species index negative) recorded
+// stopping time; -1 for the smallest where one is invalid (not finite, not positive, species index
+// negative), which leaves the error word to what it may hold already
 __global__ void k_stop_partial(const double *r, const int32_t *iv, long long cap, long long np,
-                               double *partial, dk::ErrWord *err) {
+                               double *partial) {
   __shared__ double smax[kBlock], smin[kBlock];
   double mx = 0.0, mn = 3.4028234663852886e38;
   GRID_STRIDE(p, np) {
     const double ts = PR(DK_IPTS,p);
-    if (!isfinite(ts) || !(ts > 0.0) || PI(DK_PSP,p) < 0) {dk::RecordError(err, DK_ESTOP, p); continue;}
+    if (!isfinite(ts) || !(ts > 0.0) || PI(DK_PSP,p) < 0) {mn = -1.0; continue;}
     mx = fmax(mx, ts);
     mn = fmin(mn, ts);
   }
@@ -963,15 +964,15 @@ __global__ void k_reduce_partials(const double *partial, int nblk, int ncomp, do
 
 // dust_newdt.cpp:135-145: min over particles of dx/max(|v|, 1e-30), the azimuthal transport
 // velocity with the background shear in a 3-D shearing box; stopping times validated
-// (dust_newdt.cpp:34-99)
+// (dust_newdt.cpp:34-99): -1 where one is invalid
 __global__ void k_newdt(const DevBlock *B, const double *r, const int32_t *iv, long long cap,
-                        long long np, double qo, double *partial, dk::ErrWord *err) {
+                        long long np, double qo, double *partial) {
   __shared__ double sh[kBlock];
   double dtmin = 3.4028234663852886e38;   // the largest float, the reference's start value
   GRID_STRIDE(p, np) {
     const int m = PI(DK_PGID,p);
     const double ts = PR(DK_IPTS,p);
-    if (!isfinite(ts) || !(ts > 0.0)) dk::RecordError(err, DK_ESTOP, p);
+    if (!isfinite(ts) || !(ts > 0.0)) dtmin = -1.0;
     const double vy = PR(DK_IPVY,p) - qo*PR(DK_IPX,p);
     dtmin = fmin(B[m].dx1/fmax(fabs(PR(DK_IPVX,p)), 1.0e-30), dtmin);
     dtmin = fmin(B[m].dx2/fmax(fabs(vy), 1.0e-30), dtmin);
@@ -986,10 +987,8 @@ __global__ void k_newdt(const DevBlock *B, const double *r, const int32_t *iv, l
   if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
 }
 
-// the smallest of n partial minima and the error word (cleared when set, as dk_error does) into
-// host memory
-__global__ void __launch_bounds__(kBlock) k_newdt_out(const double *partial, int n, dk::ErrWord *err,
-                                                      dk::HostOut *out) {
+// the smallest of n partial minima into host memory
+__global__ void __launch_bounds__(kBlock) k_newdt_out(const double *partial, int n, double *out) {
   __shared__ double sh[kBlock];
   double m = 3.4028234663852886e38;
   for (int i = threadIdx.x; i < n; i += kBlock) m = fmin(m, partial[i]);
@@ -999,10 +998,7 @@ __global__ void __launch_bounds__(kBlock) k_newdt_out(const double *partial, int
     if (threadIdx.x < s) sh[threadIdx.x] = fmin(sh[threadIdx.x], sh[threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x != 0) return;
-  out->value = sh[0];
-  out->err = *err;
-  if (out->err.code != 0) {err->code = 0; err->pad = 0; err->particle = 0;}
+  if (threadIdx.x == 0) *out = sh[0];
 }
 
 // cell sort (dust_cloud_device.cpp:1903-1950): key = block*ncell + cell of the position
@@ -1586,7 +1582,7 @@ int dk_create(const dk_mesh *mesh, const dk_block *blocks, const dk_physics *phy
   alloc((void**)&c->d_err, sizeof(dk::ErrWord));
   alloc((void**)&c->d_partial, sizeof(double)*9*4096);
   alloc((void**)&c->d_scalar, sizeof(double)*16);
-  if (!e && hipHostMalloc((void**)&c->h_out, sizeof(dk::HostOut)) != hipSuccess) {
+  if (!e && hipHostMalloc((void**)&c->h_out, sizeof(double)) != hipSuccess) {
     c->h_out = nullptr;
     e = DK_ENOMEM;
   }
@@ -2357,15 +2353,15 @@ int dk_new_time_step(dk_ctx *c, double dt_cfl, double *dt_out) {
   } else {
     if ((e = Ready(c))) return e;
     k_newdt<<<nb, kBlock, 0, c->stream>>>(c->d_blocks, c->rdata, c->idata, (long long)c->cap,
-                                          (long long)c->np, qo, c->d_partial, c->d_err);
+                                          (long long)c->np, qo, c->d_partial);
   }
   // (one kernel writes what the host needs into its memory, one wait: two copies and two waits
   // before, 60 -> 24 us a call at 32^3 cells)
-  k_newdt_out<<<1, kBlock, 0, c->stream>>>(c->d_partial, nb, c->d_err, c->h_out);
+  k_newdt_out<<<1, kBlock, 0, c->stream>>>(c->d_partial, nb, c->h_out);
   if ((e = dk::Check(hipGetLastError()))) return e;
   if ((e = dk::Check(hipStreamSynchronize(c->stream)))) return e;
-  if (c->h_out->err.code == DK_ESTOP) return DK_ESTOP;
-  double dt = dt_cfl*c->h_out->value;
+  if (*c->h_out < 0.0) return DK_ESTOP;
+  double dt = dt_cfl**c->h_out;
   if (c->form == DK_FORM_FP32 && c->P.shearing_box) {
     // the FP32 form's shearing-box limit: a stage's orbital-advection frame shift
     // q Omega c dt |x1|max, with the stage abscissa c at most 1 + 1/sqrt(2) (imex2+), must stay
@@ -2411,20 +2407,16 @@ int dk_stopping_times(dk_ctx *c, double out[2]) {
   } else {
     if ((e = Ready(c))) return e;
     k_stop_partial<<<kDiagGrid, kBlock, 0, c->stream>>>(c->rdata, c->idata, (long long)c->cap,
-                                                        (long long)c->np, c->d_partial,
-                                                        c->d_err);
+                                                        (long long)c->np, c->d_partial);
     if ((e = dk::Check(hipGetLastError()))) return e;
   }
   std::vector<double> h(2*kDiagGrid);
   if ((e = dk::Check(hipMemcpyAsync(h.data(), c->d_partial, sizeof(double)*h.size(),
                                     hipMemcpyDeviceToHost, c->stream)))) return e;
   if ((e = dk::Check(hipStreamSynchronize(c->stream)))) return e;
-  int32_t code = 0;
-  int64_t part = -1;
-  if ((e = dk_error(c, &code, &part))) return e;
-  if (code == DK_ESTOP) return DK_ESTOP;
   double mx = 0.0, mn = 3.4028234663852886e38;
   for (int b=0; b<kDiagGrid; ++b) {mx = std::max(mx, h[2*b]); mn = std::min(mn, h[2*b + 1]);}
+  if (mn < 0.0) return DK_ESTOP;
   out[0] = mx;
   out[1] = mn;
   return DK_OK;

@@ -118,12 +118,6 @@ struct ErrWord {
   long long particle;
 };
 
-// what a call that ends with a result for the host writes into pinned host memory
-struct HostOut {
-  double value;
-  ErrWord err;
-};
-
 __device__ inline void RecordError(ErrWord *e, int code, long long p) {
   if (atomicCAS(&e->code, 0, code) == 0) e->particle = p;
 }
@@ -165,7 +159,7 @@ struct dk_ctx {
   dk::ErrWord *d_err = nullptr;
   double *d_partial = nullptr;     // reduction partials
   double *d_scalar = nullptr;
-  dk::HostOut *h_out = nullptr;    // pinned host memory (dk_new_time_step)
+  double *h_out = nullptr;         // pinned host memory (dk_new_time_step)
   // sort scratch (grown on demand)
   void *sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;

@@ -343,7 +343,9 @@ int dk_stiffness(dk_ctx *ctx, double out[3]);
  * (dust_newdt.cpp:160-173) compares with dt on the host.  The FP32 form reduces its FP32 copies.
  * Waits for the stream. */
 int dk_stopping_times(dk_ctx *ctx, double out[2]);
-/* The first device-side error (code, particle index); clears it. */
+/* The first device-side error (code, particle index); clears it.  Only this call does: an error that
+ * a kernel recorded stays until it is read here.  (The stopping times that dk_new_time_step and
+ * dk_stopping_times find invalid are their return value, DK_ESTOP, and not recorded.) */
 int dk_error(dk_ctx *ctx, int32_t *code, int64_t *particle);
 /* Device pointer to a work field: 0 qdep(5), 1 ustar(3), 2 dmom(3), 3 solver ap(3),
  * 4 imex residual(4); layout as the gas (nvar components).  NULL if absent. */
