@@ -2015,7 +2015,9 @@ int StageGraph(dk_ctx *c, const dk_stage *st, const dk_gas_src *src) {
   const int slot = std::min(std::max(st->stage, 1), 3) - 1 + (src ? 3 : 0);
   if (hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
     return DK_EHIP;
+  c->own_capture = 1;
   const int e = StageBody(c, st, src);
+  c->own_capture = 0;
   hipGraph_t g = nullptr;
   const hipError_t ce = hipStreamEndCapture(c->stream, &g);
   if (e || ce != hipSuccess || g == nullptr) {

@@ -179,6 +179,7 @@ struct dk_ctx {
   // the plain form's tile passes (dk_tile64.hip); null: the per-particle kernels
   struct Tile64 *t64 = nullptr;
   int graphs = 0;
+  int own_capture = 0;             // a stage is being captured into one of the library's graphs
   long long graph_launches = 0;    // stage graphs launched (dk_graph_launches)
   // RemoveOutflowParticles run totals (x3_outflow_mass, x3_outflow_count, dust.hpp); the ledger
   // since the last removal is d_scalar[12..13] (bvals_part.cpp:184-186)

@@ -672,15 +672,25 @@ __global__ void __launch_bounds__(kBlock) k_t64_combine(Geo g, Grid64 T, const d
 
 }  // namespace
 
-// the workspaces of a context's tile passes
+// the workspaces of the present particles: the items and every particle's tile, place and slot
+struct Bins64 {
+  int *item_tile = nullptr, *item_part = nullptr, *key = nullptr, *rank = nullptr, *perm = nullptr;
+  void *mem = nullptr;      // the one allocation that holds them
+  long long cap = 0;        // particles they hold
+  // A graph that the caller captured holds them: they stay until the context ends, also when more
+  // particles are bound, so that the graph may be replayed as before (its particles and the
+  // context's fields outlive a bind as well).  prev: the ones kept so.
+  bool captured = false;
+  Bins64 *prev = nullptr;
+};
+
+// the workspaces of a context's tile passes; those of the mesh are allocated once
 struct Tile64 {
   Grid64 T;
-  int *count = nullptr, *start = nullptr, *item_tile = nullptr, *item_part = nullptr;
-  int *nitem = nullptr;
-  int *key = nullptr, *rank = nullptr, *perm = nullptr;
+  int *count = nullptr, *start = nullptr, *nitem = nullptr;
   double *scr = nullptr;
   void *mem = nullptr;      // the one allocation that holds them
-  long long cap = -1;       // particles the arrays hold
+  Bins64 *b = nullptr;
   int bins = 0;             // the bins of the present positions are built (T64Hold)
 };
 
@@ -688,9 +698,22 @@ namespace dk {
 
 namespace {
 
-void Free(Tile64 *w) {
-  if (w->mem) (void)hipFree(w->mem);
-  delete w;
+// the caller is capturing the context's stream (the library's own stage graphs, which are captured
+// anew before every launch, apart)
+bool CallerCaptures(const dk_ctx *c) {
+  if (c->stream == nullptr || c->own_capture) return false;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// one allocation (null: short of device memory, and then the per-particle kernels run)
+void *Mem(size_t bytes) {
+  void *p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
 }
 
 Args64 MakeArgs(const dk_ctx *c, double sh, double a_dt, double dt) {
@@ -698,8 +721,8 @@ Args64 MakeArgs(const dk_ctx *c, double sh, double a_dt, double dt) {
   Args64 A{};
   A.g = c->g; A.T = w->T; A.B = c->d_blocks;
   A.r = c->rdata; A.iv = c->idata; A.cap = c->cap; A.np = c->np;
-  A.perm = w->perm; A.start = w->start; A.item_tile = w->item_tile; A.item_part = w->item_part;
-  A.nitem = w->nitem;
+  A.perm = w->b->perm; A.start = w->start; A.nitem = w->nitem;
+  A.item_tile = w->b->item_tile; A.item_part = w->b->item_part;
   A.sh = sh; A.a_dt = a_dt; A.dt = dt;
   A.br = 1;
   A.sbox = c->P.shearing_box; A.strat = c->P.stratified;
@@ -711,11 +734,13 @@ Args64 MakeArgs(const dk_ctx *c, double sh, double a_dt, double dt) {
 template <int OP>
 int Bin(dk_ctx *c, const Args64 &A) {
   Tile64 *w = c->t64;
+  Bins64 *b = w->b;
+  if (CallerCaptures(c)) b->captured = true;
   const int pt = ProfBegin(c, "bins");
-  k_t64_count<OP><<<Grid(c->np), kBlock, 0, c->stream>>>(A, w->key, w->rank, w->count);
-  k_t64_scan<<<1, kScanThreads, 0, c->stream>>>(w->T.nt, w->count, w->start, w->item_tile,
-                                                w->item_part, w->nitem);
-  k_t64_place<<<Grid(c->np), kBlock, 0, c->stream>>>(w->key, w->rank, w->start, c->np, w->perm);
+  k_t64_count<OP><<<Grid(c->np), kBlock, 0, c->stream>>>(A, b->key, b->rank, w->count);
+  k_t64_scan<<<1, kScanThreads, 0, c->stream>>>(w->T.nt, w->count, w->start, b->item_tile,
+                                                b->item_part, w->nitem);
+  k_t64_place<<<Grid(c->np), kBlock, 0, c->stream>>>(b->key, b->rank, w->start, c->np, b->perm);
   ProfEnd(c, pt);
   return Check(hipGetLastError());
 }
@@ -741,23 +766,10 @@ int Pass(dk_ctx *c, Args64 A, const char *label) {
   return Check(hipGetLastError());
 }
 
-}  // namespace
-
-int T64Reserve(dk_ctx *c) {
-  if (c->form != DK_FORM_FP64 || c->smr || c->P.clouds || c->g.ng < 2) return DK_OK;
-  if (c->t64 != nullptr && c->t64->cap >= c->np) return DK_OK;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(c->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return DK_OK;   // (no allocation inside the caller's capture: the per-particle kernels run)
-  }
-  if (c->t64 != nullptr) {
-    (void)hipStreamSynchronize(c->stream);
-    Free(c->t64);
-    c->t64 = nullptr;
-  }
-  Tile64 *w = new Tile64();
-  Grid64 &T = w->T;
+// the mesh's part of the workspaces (false: the per-particle kernels run)
+bool ReserveMesh(dk_ctx *c) {
+  if (c->t64 != nullptr) return true;
+  Grid64 T;
   const Geo &g = c->g;
   T.SY = c->P.shearing_box ? 1 : 0;
   T.ntx = (g.nx1 + kTX - 1)/kTX; T.nty = (g.nx2 + kTY - 1)/kTY; T.ntz = (g.nx3 + kTZ - 1)/kTZ;
@@ -766,42 +778,86 @@ int T64Reserve(dk_ctx *c) {
   T.RN = T.RX*T.RY*T.RZ;
   T.iRX = 1.0f/T.RX; T.iRY = 1.0f/T.RY; T.iRN = 1.0f/T.RN;
   const long long nt = (long long)T.ntb*g.nmb;
-  const long long items = nt + c->np/kItemMax + 1;
-  if (items >= (1LL << 30)) {   // (beyond 32-bit items: the per-particle kernels run)
-    Free(w);
-    return DK_OK;
-  }
+  if (nt >= (1LL << 29)) return false;   // (32-bit items)
   T.nt = static_cast<int>(nt);
   // the scratch, then the int arrays
-  const size_t nscr = 4*(size_t)T.RN*nt, np = static_cast<size_t>(std::max<long long>(c->np, 1));
-  const size_t nint = 2*(size_t)(nt + 1) + 2*(size_t)items + 1 + 3*np;
-  if (hipMalloc(&w->mem, sizeof(double)*nscr + sizeof(int)*nint) != hipSuccess) {
-    (void)hipGetLastError();   // (short of device memory: the per-particle kernels run)
-    w->mem = nullptr;
-    Free(w);
-    return DK_OK;
-  }
-  w->scr = static_cast<double*>(w->mem);
+  const size_t nscr = 4*(size_t)T.RN*nt;
+  void *mem = Mem(sizeof(double)*nscr + sizeof(int)*(2*(size_t)(nt + 1) + 1));
+  if (mem == nullptr) return false;
+  Tile64 *w = new Tile64();
+  w->T = T;
+  w->mem = mem;
+  w->scr = static_cast<double*>(mem);
   w->count = reinterpret_cast<int*>(w->scr + nscr);
   w->start = w->count + nt + 1;
-  w->item_tile = w->start + nt + 1;
-  w->item_part = w->item_tile + items;
-  w->nitem = w->item_part + items;
-  w->key = w->nitem + 1;
-  w->rank = w->key + np;
-  w->perm = w->rank + np;
-  const int e = Check(hipMemsetAsync(w->count, 0, sizeof(int)*(nt + 1), c->stream));
-  if (e) {
-    Free(w);
-    return e;
-  }
-  w->cap = c->np;
+  w->nitem = w->start + nt + 1;
   c->t64 = w;
+  return true;
+}
+
+// the particles' part, for n of them
+Bins64 *NewBins(const Grid64 &T, long long n) {
+  const size_t items = static_cast<size_t>(T.nt + n/kItemMax + 1);
+  void *mem = Mem(sizeof(int)*(2*items + 3*static_cast<size_t>(n)));
+  if (mem == nullptr) return nullptr;
+  Bins64 *b = new Bins64();
+  b->mem = mem;
+  b->item_tile = static_cast<int*>(mem);
+  b->item_part = b->item_tile + items;
+  b->key = b->item_part + items;
+  b->rank = b->key + n;
+  b->perm = b->rank + n;
+  b->cap = n;
+  return b;
+}
+
+}  // namespace
+
+int T64Reserve(dk_ctx *c) {
+  if (c->form != DK_FORM_FP64 || c->smr || c->P.clouds || c->g.ng < 2) return DK_OK;
+  Bins64 *old = (c->t64 != nullptr) ? c->t64->b : nullptr;
+  if (old != nullptr && old->cap >= c->np) return DK_OK;
+  if (CallerCaptures(c))
+    return DK_OK;   // (no allocation inside the caller's capture: the per-particle kernels run)
+  const bool first = c->t64 == nullptr;
+  if (!ReserveMesh(c)) return DK_OK;
+  Tile64 *w = c->t64;
+  if (first) {
+    const int e = Check(hipMemsetAsync(w->count, 0, sizeof(int)*(w->T.nt + 1), c->stream));
+    if (e) {
+      T64Destroy(c);
+      return e;
+    }
+  }
+  long long n = std::max<long long>(c->np, 1);
+  if (old != nullptr && old->captured) {
+    // (half as many again as the ones kept, so that what a growing count leaves behind stays below
+    // twice what it has)
+    n = std::max(n, old->cap + old->cap/2);
+  } else if (old != nullptr) {
+    (void)hipStreamSynchronize(c->stream);
+    w->b = old->prev;
+    (void)hipFree(old->mem);
+    delete old;
+  }
+  Bins64 *b = NewBins(w->T, n);
+  if (b == nullptr) return DK_OK;
+  b->prev = w->b;
+  w->b = b;
   return DK_OK;
 }
 
 void T64Destroy(dk_ctx *c) {
-  if (c->t64 != nullptr) Free(c->t64);
+  Tile64 *w = c->t64;
+  if (w == nullptr) return;
+  while (w->b != nullptr) {
+    Bins64 *b = w->b;
+    w->b = b->prev;
+    (void)hipFree(b->mem);
+    delete b;
+  }
+  (void)hipFree(w->mem);
+  delete w;
   c->t64 = nullptr;
 }
 
@@ -810,7 +866,7 @@ void T64Destroy(dk_ctx *c) {
 // 3.08 against 4.14 ms (imex2+) and 1.51 against 1.73 ms (pc2), at one per 32 cells 2.97 against
 // 2.47 and 1.47 against 1.01 ms (64^3 cells: 0.68 / 0.80 and 0.35 / 0.34 ms at 16).
 bool T64Use(const dk_ctx *c) {
-  if (c->t64 == nullptr || c->t64->cap < c->np) return false;
+  if (c->t64 == nullptr || c->t64->b == nullptr || c->t64->b->cap < c->np) return false;
   return c->np*16 >= (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3;
 }
 
