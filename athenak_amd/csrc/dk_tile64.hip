@@ -862,12 +862,19 @@ void T64Destroy(dk_ctx *c) {
 }
 
 // The tile passes cost every tile's region and the combine whatever the particles, the
-// per-particle kernels their atomics: at one particle per 16 cells a step of 128^3 cells takes
-// 3.08 against 4.14 ms (imex2+) and 1.51 against 1.73 ms (pc2), at one per 32 cells 2.97 against
-// 2.47 and 1.47 against 1.01 ms (64^3 cells: 0.68 / 0.80 and 0.35 / 0.34 ms at 16).
+// per-particle kernels their atomics.  A step (imex2+ / pc2), tile passes against per-particle
+// kernels: 128^3 cells at 8 particles a tile (one per 16 cells) 3.08 against 4.14 / 1.51 against 1.73
+// ms, at 4 a tile 2.97 against 2.47 / 1.47 against 1.01.  Where blocks leave tiles partly empty it
+// is the particles a tile that count: 4096 blocks of 4^3 cells at 4 a tile 1.07 against 1.05 / 0.46
+// against 0.41 ms, at 8 1.07 against 1.35 / 0.46 against 0.50; 343 blocks of 9^3 at 5 a tile 0.89
+// against 1.08 / 0.39 against 0.38; 2197 blocks of 5^3 at 4 1.41 against 1.39 / 0.62 against 0.50,
+// at 8 1.44 against 2.04 / 0.63 against 0.69; 32768 blocks of 2^3 at 2 6.95 against 5.41 / 2.94
+// against 2.18, at 8 7.19 against 9.11 / 2.99 against 3.31.
 bool T64Use(const dk_ctx *c) {
   if (c->t64 == nullptr || c->t64->b == nullptr || c->t64->b->cap < c->np) return false;
-  return c->np*16 >= (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3;
+  const long long a_tile = (c->P.coupling == DK_PC2) ? 6 : 5;
+  return c->np*16 >= (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3 &&
+         c->np >= a_tile*c->t64->T.nt;
 }
 
 int T64Hold(dk_ctx *c, double sh) {
