@@ -84,7 +84,7 @@ struct Args64 {
   long long cap, np;
   const int *perm, *start, *item_tile, *item_part, *nitem;
   double sh, a_dt, dt;
-  int rate_dep, br, sbox, strat;
+  int rate_dep, sbox, strat;
   double qs, om;
   const double *src;      // u* (3 components), or u1 (the gas) for the predictor
   double *out;            // the field deposited into: nvar components, the first at comp0
@@ -544,7 +544,7 @@ __global__ void __launch_bounds__(kNT, 3) k_t64(Args64 A) {
       }
       Work<OP>(A, b, p[k], u, val);
       const bool direct = far || !Finite<NC>(val);
-      if (__builtin_expect(direct && A.br, 0)) FarDeposit<NC>(A, m, MakeW(g, L[k]), val);
+      if (__builtin_expect(direct, 0)) FarDeposit<NC>(A, m, MakeW(g, L[k]), val);
       if (far) continue;
       const int at = cst[cell[k]] + rk[k];
       rec[at] = L[k].dx; rec[kChunk + at] = L[k].dy; rec[2*kChunk + at] = L[k].dz;
@@ -553,55 +553,52 @@ __global__ void __launch_bounds__(kNT, 3) k_t64(Args64 A) {
     }
     __syncthreads();
     // 4. the runs' sums, per slab, into the region
-    if (A.br) {
-      for (int task = tid; task < 3*nruns; task += kNT) {
-        const int slab = (task >= 2*nruns) ? 2 : ((task >= nruns) ? 1 : 0);
-        const int rn = runs[task - slab*nruns];
-        const int l = rn & 255, a0 = cst[l] + (rn >> 8)*kRun;
-        const int a1 = min(a0 + kRun, cst[l] + cnt[l]);
-        double acc[3][3][NC];
+    for (int task = tid; task < 3*nruns; task += kNT) {
+      const int slab = (task >= 2*nruns) ? 2 : ((task >= nruns) ? 1 : 0);
+      const int rn = runs[task - slab*nruns];
+      const int l = rn & 255, a0 = cst[l] + (rn >> 8)*kRun;
+      const int a1 = min(a0 + kRun, cst[l] + cnt[l]);
+      double acc[3][3][NC];
 #pragma unroll
-        for (int bb=0; bb<3; ++bb)
+      for (int bb=0; bb<3; ++bb)
 #pragma unroll
-          for (int a=0; a<3; ++a)
+        for (int a=0; a<3; ++a)
 #pragma unroll
-            for (int v=0; v<NC; ++v) acc[bb][a][v] = 0.0;
-        for (int at = a0; at < a1; ++at) {
-          double wx[3], wy[3], wz[3];
-          Weights(g.deposit, rec[at], wx);
-          Weights(g.deposit, rec[kChunk + at], wy);
-          Weights(g.deposit, rec[2*kChunk + at], wz);
-          const double ws = (slab == 0) ? wz[0] : ((slab == 1) ? wz[1] : wz[2]);
-          double val[NC];
+          for (int v=0; v<NC; ++v) acc[bb][a][v] = 0.0;
+      for (int at = a0; at < a1; ++at) {
+        double wx[3], wy[3], wz[3];
+        Weights(g.deposit, rec[at], wx);
+        Weights(g.deposit, rec[kChunk + at], wy);
+        Weights(g.deposit, rec[2*kChunk + at], wz);
+        const double ws = (slab == 0) ? wz[0] : ((slab == 1) ? wz[1] : wz[2]);
+        double val[NC];
 #pragma unroll
-          for (int v=0; v<NC; ++v) val[v] = rec[(3 + v)*kChunk + at];
+        for (int v=0; v<NC; ++v) val[v] = rec[(3 + v)*kChunk + at];
 #pragma unroll
-          for (int bb=0; bb<3; ++bb) {
-            const double wcb = ws*wy[bb];
+        for (int bb=0; bb<3; ++bb) {
+          const double wcb = ws*wy[bb];
 #pragma unroll
-            for (int a=0; a<3; ++a) {
-              const double ww = wcb*wx[a];
+          for (int a=0; a<3; ++a) {
+            const double ww = wcb*wx[a];
 #pragma unroll
-              for (int v=0; v<NC; ++v) acc[bb][a][v] += ww*val[v];
-            }
+            for (int v=0; v<NC; ++v) acc[bb][a][v] += ww*val[v];
           }
         }
-        const int lx = l & (kTX - 1), lr = l/kTX, lz = lr/NY, ly = lr - lz*NY;
-        const int rb = ((lz + slab)*T.RY + ly)*T.RX + lx;
-#pragma unroll
-        for (int bb=0; bb<3; ++bb)
-#pragma unroll
-          for (int a=0; a<3; ++a)
-#pragma unroll
-            for (int v=0; v<NC; ++v)
-              unsafeAtomicAdd(&reg[v*T.RN + rb + bb*T.RX + a], acc[bb][a][v]);
       }
+      const int lx = l & (kTX - 1), lr = l/kTX, lz = lr/NY, ly = lr - lz*NY;
+      const int rb = ((lz + slab)*T.RY + ly)*T.RX + lx;
+#pragma unroll
+      for (int bb=0; bb<3; ++bb)
+#pragma unroll
+        for (int a=0; a<3; ++a)
+#pragma unroll
+          for (int v=0; v<NC; ++v)
+            unsafeAtomicAdd(&reg[v*T.RN + rb + bb*T.RX + a], acc[bb][a][v]);
     }
     __syncthreads();
     if (tid < ncell) cnt[tid] = 0;
     __syncthreads();
   }
-  if (!A.br) return;
   // the region: the tile's first item to the scratch, row by row (the rows of the tiles of a block
   // that share ty and tz lie one after another), a later one straight into the field
   for (int rc = tid; rc < T.RN; rc += kNT) {
@@ -724,7 +721,6 @@ Args64 MakeArgs(const dk_ctx *c, double sh, double a_dt, double dt) {
   A.perm = w->b->perm; A.start = w->start; A.nitem = w->nitem;
   A.item_tile = w->b->item_tile; A.item_part = w->b->item_part;
   A.sh = sh; A.a_dt = a_dt; A.dt = dt;
-  A.br = 1;
   A.sbox = c->P.shearing_box; A.strat = c->P.stratified;
   A.qs = c->P.qshear; A.om = c->P.omega0;
   A.scr = w->scr; A.err = c->d_err;
@@ -757,12 +753,10 @@ int Pass(dk_ctx *c, Args64 A, const char *label) {
   {const int pt = ProfBegin(c, label);
    k_t64<OP><<<static_cast<unsigned>(items), kNT, Lds64<OP>(w->T.RN), c->stream>>>(A);
    ProfEnd(c, pt);}
-  if (A.br) {
-    const int pt = ProfBegin(c, "combine");
-    const dim3 gr(static_cast<unsigned>((c->g.ncb + kBlock - 1)/kBlock), c->g.nmb);
-    k_t64_combine<NC><<<gr, kBlock, 0, c->stream>>>(c->g, w->T, A.scr, A.out, A.nvar, A.comp0);
-    ProfEnd(c, pt);
-  }
+  {const int pt = ProfBegin(c, "combine");
+   const dim3 gr(static_cast<unsigned>((c->g.ncb + kBlock - 1)/kBlock), c->g.nmb);
+   k_t64_combine<NC><<<gr, kBlock, 0, c->stream>>>(c->g, w->T, A.scr, A.out, A.nvar, A.comp0);
+   ProfEnd(c, pt);}
   return Check(hipGetLastError());
 }
 
@@ -870,7 +864,14 @@ void T64Destroy(dk_ctx *c) {
 // against 1.08 / 0.39 against 0.38; 2197 blocks of 5^3 at 4 1.41 against 1.39 / 0.62 against 0.50,
 // at 8 1.44 against 2.04 / 0.63 against 0.69; 32768 blocks of 2^3 at 2 6.95 against 5.41 / 2.94
 // against 2.18, at 8 7.19 against 9.11 / 2.99 against 3.31.
+// Without back-reaction nothing is deposited, and the per-particle kernels gather alone: sorted
+// particles, kick or advance of a step on the tile passes (their bins, and sums that nobody reads)
+// against the per-particle kernel, 33 thousand 47 against 19 us, 2.1 million in clumps 0.35 against
+// 0.23 ms, 67 million 8.9 against 8.1, pc2 7.5 million in uneven blocks 0.78 against 0.61.  (In no order
+// within their blocks the tile passes' gather was the faster one for large even boxes, 67 million 43
+// against 83 ms, and the slower one for small boxes, clumps and uneven blocks.)
 bool T64Use(const dk_ctx *c) {
+  if (!c->P.back_reaction) return false;
   if (c->t64 == nullptr || c->t64->b == nullptr || c->t64->b->cap < c->np) return false;
   const long long a_tile = (c->P.coupling == DK_PC2) ? 6 : 5;
   return c->np*16 >= (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3 &&
@@ -905,7 +906,6 @@ int T64Oper(dk_ctx *c, const double *field, double *out, double a_dt, double sh)
 int T64Kick(dk_ctx *c, double a_dt, double sh) {
   Args64 A = MakeArgs(c, sh, a_dt, 0.0);
   A.src = c->ustar; A.out = c->dmom; A.nvar = 3; A.comp0 = 0;
-  A.br = c->P.back_reaction;
   return Pass<kKick>(c, A, "gather_kick");
 }
 
@@ -919,7 +919,6 @@ int T64Predictor(dk_ctx *c, double dt, int rate_dep) {
 int T64Advance(dk_ctx *c, double dt) {
   Args64 A = MakeArgs(c, 0.0, 0.0, dt);
   A.src = c->ustar; A.out = c->dmom; A.nvar = 3; A.comp0 = 0;
-  A.br = c->P.back_reaction;
   return Pass<kAdvance>(c, A, "pc2_advance");
 }
 
