@@ -760,20 +760,45 @@ int Pass(dk_ctx *c, Args64 A, const char *label) {
   return Check(hipGetLastError());
 }
 
-// the mesh's part of the workspaces (false: the per-particle kernels run)
-bool ReserveMesh(dk_ctx *c) {
-  if (c->t64 != nullptr) return true;
+Grid64 MakeGrid(const dk_ctx *c) {
   Grid64 T;
   const Geo &g = c->g;
   T.SY = c->P.shearing_box ? 1 : 0;
   T.ntx = (g.nx1 + kTX - 1)/kTX; T.nty = (g.nx2 + kTY - 1)/kTY; T.ntz = (g.nx3 + kTZ - 1)/kTZ;
   T.ntb = T.ntx*T.nty*T.ntz;
+  T.nt = static_cast<int>(std::min<long long>((long long)T.ntb*g.nmb, INT32_MAX));
   T.RX = kTX + 2; T.RY = kTY + 2 + 2*T.SY; T.RZ = kTZ + 2;
   T.RN = T.RX*T.RY*T.RZ;
   T.iRX = 1.0f/T.RX; T.iRY = 1.0f/T.RY; T.iRN = 1.0f/T.RN;
-  const long long nt = (long long)T.ntb*g.nmb;
+  return T;
+}
+
+// The tile passes cost every tile's region and the combine whatever the particles, the
+// per-particle kernels their atomics.  A step (imex2+ / pc2), tile passes against per-particle
+// kernels: 128^3 cells at 8 particles a tile (one per 16 cells) 3.08 against 4.14 / 1.51 against 1.73
+// ms, at 4 a tile 2.97 against 2.47 / 1.47 against 1.01.  Where blocks leave tiles partly empty it
+// is the particles a tile that count: 4096 blocks of 4^3 cells at 4 a tile 1.07 against 1.05 / 0.46
+// against 0.41 ms, at 8 1.07 against 1.35 / 0.46 against 0.50; 343 blocks of 9^3 at 5 a tile 0.89
+// against 1.08 / 0.39 against 0.38; 2197 blocks of 5^3 at 4 1.41 against 1.39 / 0.62 against 0.50,
+// at 8 1.44 against 2.04 / 0.63 against 0.69; 32768 blocks of 2^3 at 2 6.95 against 5.41 / 2.94
+// against 2.18, at 8 7.19 against 9.11 / 2.99 against 3.31.
+// Without back-reaction nothing is deposited, and the per-particle kernels gather alone: sorted
+// particles, kick or advance of a step on the tile passes (their bins, and sums that nobody reads)
+// against the per-particle kernel, 33 thousand 47 against 19 us, 2.1 million in clumps 0.35 against
+// 0.23 ms, 67 million 8.9 against 8.1, pc2 7.5 million in uneven blocks 0.78 against 0.61.  (In no order
+// within their blocks the tile passes' gather was the faster one for large even boxes, 67 million 43
+// against 83 ms, and the slower one for small boxes, clumps and uneven blocks.)
+bool Pays(const dk_ctx *c, const Grid64 &T) {
+  if (!c->P.back_reaction) return false;
+  const long long a_tile = (c->P.coupling == DK_PC2) ? 6 : 5;
+  return c->np*16 >= (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3 && c->np >= a_tile*T.nt;
+}
+
+// the mesh's part of the workspaces (false: the per-particle kernels run)
+bool ReserveMesh(dk_ctx *c, const Grid64 &T) {
+  if (c->t64 != nullptr) return true;
+  const long long nt = T.nt;
   if (nt >= (1LL << 29)) return false;   // (32-bit items)
-  T.nt = static_cast<int>(nt);
   // the scratch, then the int arrays
   const size_t nscr = 4*(size_t)T.RN*nt;
   void *mem = Mem(sizeof(double)*nscr + sizeof(int)*(2*(size_t)(nt + 1) + 1));
@@ -809,32 +834,37 @@ Bins64 *NewBins(const Grid64 &T, long long n) {
 
 int T64Reserve(dk_ctx *c) {
   if (c->form != DK_FORM_FP64 || c->smr || c->P.clouds || c->g.ng < 2) return DK_OK;
+  const Grid64 T = MakeGrid(c);
+  if (!Pays(c, T)) return DK_OK;
   Bins64 *old = (c->t64 != nullptr) ? c->t64->b : nullptr;
   if (old != nullptr && old->cap >= c->np) return DK_OK;
   if (CallerCaptures(c))
     return DK_OK;   // (no allocation inside the caller's capture: the per-particle kernels run)
   const bool first = c->t64 == nullptr;
-  if (!ReserveMesh(c)) return DK_OK;
+  if (!ReserveMesh(c, T)) return DK_OK;
   Tile64 *w = c->t64;
   if (first) {
-    const int e = Check(hipMemsetAsync(w->count, 0, sizeof(int)*(w->T.nt + 1), c->stream));
+    const int e = Check(hipMemsetAsync(w->count, 0, sizeof(int)*(T.nt + 1), c->stream));
     if (e) {
       T64Destroy(c);
       return e;
     }
   }
-  long long n = std::max<long long>(c->np, 1);
+  // for as many as the caller's arrays hold, so that a count that grows within them neither
+  // allocates nor waits (12 of their 156 bytes a particle)
+  long long n = std::min<long long>(c->cap, INT32_MAX);
   if (old != nullptr && old->captured) {
-    // (half as many again as the ones kept, so that what a growing count leaves behind stays below
-    // twice what it has)
-    n = std::max(n, old->cap + old->cap/2);
+    // (half as many again as the ones kept, so that what growing arrays leave behind stays below
+    // twice what they have)
+    n = std::max(n, std::min<long long>(old->cap + old->cap/2, INT32_MAX));
   } else if (old != nullptr) {
     (void)hipStreamSynchronize(c->stream);
     w->b = old->prev;
     (void)hipFree(old->mem);
     delete old;
   }
-  Bins64 *b = NewBins(w->T, n);
+  Bins64 *b = NewBins(T, n);
+  if (b == nullptr && n > c->np) b = NewBins(T, c->np);
   if (b == nullptr) return DK_OK;
   b->prev = w->b;
   w->b = b;
@@ -855,27 +885,8 @@ void T64Destroy(dk_ctx *c) {
   c->t64 = nullptr;
 }
 
-// The tile passes cost every tile's region and the combine whatever the particles, the
-// per-particle kernels their atomics.  A step (imex2+ / pc2), tile passes against per-particle
-// kernels: 128^3 cells at 8 particles a tile (one per 16 cells) 3.08 against 4.14 / 1.51 against 1.73
-// ms, at 4 a tile 2.97 against 2.47 / 1.47 against 1.01.  Where blocks leave tiles partly empty it
-// is the particles a tile that count: 4096 blocks of 4^3 cells at 4 a tile 1.07 against 1.05 / 0.46
-// against 0.41 ms, at 8 1.07 against 1.35 / 0.46 against 0.50; 343 blocks of 9^3 at 5 a tile 0.89
-// against 1.08 / 0.39 against 0.38; 2197 blocks of 5^3 at 4 1.41 against 1.39 / 0.62 against 0.50,
-// at 8 1.44 against 2.04 / 0.63 against 0.69; 32768 blocks of 2^3 at 2 6.95 against 5.41 / 2.94
-// against 2.18, at 8 7.19 against 9.11 / 2.99 against 3.31.
-// Without back-reaction nothing is deposited, and the per-particle kernels gather alone: sorted
-// particles, kick or advance of a step on the tile passes (their bins, and sums that nobody reads)
-// against the per-particle kernel, 33 thousand 47 against 19 us, 2.1 million in clumps 0.35 against
-// 0.23 ms, 67 million 8.9 against 8.1, pc2 7.5 million in uneven blocks 0.78 against 0.61.  (In no order
-// within their blocks the tile passes' gather was the faster one for large even boxes, 67 million 43
-// against 83 ms, and the slower one for small boxes, clumps and uneven blocks.)
 bool T64Use(const dk_ctx *c) {
-  if (!c->P.back_reaction) return false;
-  if (c->t64 == nullptr || c->t64->b == nullptr || c->t64->b->cap < c->np) return false;
-  const long long a_tile = (c->P.coupling == DK_PC2) ? 6 : 5;
-  return c->np*16 >= (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3 &&
-         c->np >= a_tile*c->t64->T.nt;
+  return c->t64 != nullptr && c->t64->b != nullptr && c->t64->b->cap >= c->np && Pays(c, c->t64->T);
 }
 
 int T64Hold(dk_ctx *c, double sh) {

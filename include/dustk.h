@@ -9,7 +9,7 @@
  * where dk_stage carries the numbers the task read from Driver and Mesh (stage, dt, time,
  * the RK/IMEX tableau of src/driver/driver.cpp:106-118,278-300).  Every function returns 0 on
  * success or a positive DK_E* code; none aborts.  Calls are asynchronous and ordered on the
- * context's HIP stream; only dk_diag_sums, dk_error and dk_new_time_step wait for the stream.
+ * context's HIP stream; those that return a result to the host wait for it (each says so below).
  *
  * Layouts are the reference's:
  *   particles  rdata[c*capacity + p], c < DK_NRDATA (double), idata[c*capacity + p],
@@ -179,7 +179,13 @@ int dk_destroy(dk_ctx *ctx);
  * (Hydro::u0/u1).  In DK_FORM_FP32 the particles are copied into the library's
  * mixed-precision cell-sorted store; dk_export_particles writes them back (in the store's
  * order; at a step boundary the stage registers x1, v1, R, which no stage reads before the
- * next stage 1 sets them, are written as x1 = x, v1 = v, R = 0). */
+ * next stage 1 sets them, are written as x1 = x, v1 = v, R = 0).
+ * In DK_FORM_FP64 a bind with back-reaction on and enough particles for the tile passes (one per 16
+ * cells) reserves their workspaces: once per context 90 bytes a cell (120 in the shearing box) and,
+ * whenever capacity exceeds every earlier one, 12 bytes a particle of capacity, for which it waits
+ * for the stream; other binds neither allocate nor wait.  Where device memory does not suffice the
+ * call succeeds and the stages run on per-particle kernels, 10 to 30 times as slow.  Graphs that
+ * the caller captured of this form's calls stay valid over later binds, until the context ends. */
 int dk_bind_particles(dk_ctx *ctx, double *rdata, int32_t *idata, int64_t capacity,
                       int64_t npart);
 int dk_bind_gas(dk_ctx *ctx, double *u0, double *u1);
@@ -255,7 +261,8 @@ int dk_x3_removed(dk_ctx *ctx, double out[2]);
  * (both forms; the FP32 form applies a pending correction first, from its FP32 velocities).
  * The FP32 form in the shearing box also caps dt_out where a stage's orbital-advection frame
  * shift q Omega c dt |x1|max (c <= 1 + 1/sqrt(2)) would reach half a cell in x2, the largest
- * shift its stages accept (DK_EUNSUPPORTED beyond); the reference has no such limit. */
+ * shift its stages accept (DK_EUNSUPPORTED beyond); the reference has no such limit.  Waits for the
+ * stream. */
 int dk_new_time_step(dk_ctx *ctx, double dt_cfl, double *dt_out);
 
 /* The strict drag solver (dk_physics.solver = DK_PCG or DK_ADAPTIVE, FP64 form): its
@@ -335,7 +342,7 @@ int dk_prof_read(dk_ctx *ctx, int32_t idx, char *label, int32_t label_len, doubl
  * pc2 cycle records chi = dt max_cells qdep[4]/rho before the predictor is applied; out[0] = chi
  * of the last cycle, out[1] = the running maximum, out[2] = the rate maximum max qdep[4]/rho
  * (NewTimeStep's stiff_thresh/stiff_rate_max limit, dust_newdt.cpp:114-119).  One rank: no
- * reduction over ranks.  Both forms. */
+ * reduction over ranks.  Both forms.  Waits for the stream. */
 int dk_stiffness(dk_ctx *ctx, double out[3]);
 /* RefreshStoppingTimeMaximum (src/dust/dust_newdt.cpp:34-98): validates every particle's
  * stopping time (finite, positive, species index not negative; DK_ESTOP otherwise) and returns
@@ -343,7 +350,7 @@ int dk_stiffness(dk_ctx *ctx, double out[3]);
  * (dust_newdt.cpp:160-173) compares with dt on the host.  The FP32 form reduces its FP32 copies.
  * Waits for the stream. */
 int dk_stopping_times(dk_ctx *ctx, double out[2]);
-/* The first device-side error (code, particle index); clears it.  Only this call does: an error that
+/* The first device-side error (code, particle index); clears it.  Waits for the stream.  Only this call does: an error that
  * a kernel recorded stays until it is read here.  (The stopping times that dk_new_time_step and
  * dk_stopping_times find invalid are their return value, DK_ESTOP, and not recorded.) */
 int dk_error(dk_ctx *ctx, int32_t *code, int64_t *particle);

@@ -122,3 +122,51 @@ def test_a_callers_graph_is_replayed_after_other_binds(coupling):
     assert all(bool((x == 7).all()) for x in guard)
     g.check_device_error()
     g.close()
+
+
+def free_bytes():
+    import torch
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def big(coupling=abi.DK_IMEX, back_reaction=1):
+    w = workloads.c1(n=64, nb=2, coupling=coupling,
+                     solver=abi.DK_DC1 if coupling == abi.DK_IMEX else abi.DK_LOCAL)
+    w.phys.back_reaction = back_reaction
+    return w
+
+
+@pytest.mark.parametrize("n,back_reaction", [(1000, 1), (1 << 20, 0)])
+def test_a_bind_takes_no_memory_for_passes_that_do_not_run(n, back_reaction):
+    import torch
+    w = big(back_reaction=back_reaction)
+    p = Particles(w, n, 1)
+    g = context(w, torch.zeros((8, 4, 36, 36, 36), dtype=torch.float64, device="cuda"))
+    before = free_bytes()
+    bind(g, p)                  # (with the tile passes: 23 MB for the mesh, 12 MB a million)
+    assert free_bytes() == before
+    g.close()
+
+
+def test_a_count_that_grows_within_the_arrays_allocates_once():
+    import torch
+    w = big()
+    cap = 3 << 20
+    p = Particles(w, cap, 2)
+    u = torch.zeros((8, 4, 36, 36, 36), dtype=torch.float64, device="cuda")
+    u[:, 0] = 1.0
+    g = context(w, u)
+    before = free_bytes()
+    bind(g, p, 1 << 18)
+    after = free_bytes()
+    assert before - after >= 12 * cap
+    for n in (1 << 19, 1000, 1 << 20, cap):
+        bind(g, p, n)
+        assert free_bytes() == after
+        d0 = g.diag()
+        g.step(1e-4, None)
+        d1 = g.diag()           # (every count exchanges momentum without loss)
+        assert np.abs((d1[0:3] + d1[3:6]) - (d0[0:3] + d0[3:6])).max() < 1e-13 * d0[8]
+    g.check_device_error()
+    g.close()
