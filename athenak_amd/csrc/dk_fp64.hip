@@ -1402,12 +1402,18 @@ int HydroSupported(const dk_ctx *c, const dk_gas_src *src) {
 // the flux divergence field (allocated once, outside any stream capture)
 int HydroField(dk_ctx *c) {
   if (c->hdivf != nullptr) return DK_OK;
-  if (hipMalloc(&c->hdivf, sizeof(double)*DK_NGAS*NCells(c)) != hipSuccess) {
+  return DeviceAlloc(c, (void**)&c->hdivf, sizeof(double)*DK_NGAS*NCells(c));
+}
+
+int DeviceAlloc(dk_ctx *c, void **p, size_t bytes) {
+  if (hipMalloc(p, bytes) == hipSuccess) return DK_OK;
+  (void)hipGetLastError();
+  if (T64Yield(c)) {
+    if (hipMalloc(p, bytes) == hipSuccess) return DK_OK;
     (void)hipGetLastError();
-    c->hdivf = nullptr;
-    return DK_ENOMEM;
   }
-  return DK_OK;
+  *p = nullptr;
+  return DK_ENOMEM;
 }
 
 int GasHook(dk_ctx *c, const dk_stage *st, const dk_gas_src *src, const double *dmom,
@@ -2091,6 +2097,7 @@ int64_t dk_graph_launches(const dk_ctx *c) { return c ? c->graph_launches : 0; }
 // keeps its store sorted by (block, tile, cell) every stage, so it has nothing to do here.
 namespace {
 int SortScratch(dk_ctx *c, long long n);
+int SortTmp(dk_ctx *c, size_t bytes);
 }  // namespace
 
 namespace {
@@ -2150,12 +2157,7 @@ int dk_sort_particles(dk_ctx *c) {
   if ((e = SortScratch(c, n))) return e;
   SortBufs b{c->sort_keys, c->sort_idx, c->sort_rbuf, c->sort_ibuf, nullptr, 0};
   size_t bytes = 0;
-  if ((e = SortTmpBytes(c, b, n, bytes))) return e;
-  if (bytes > c->sort_tmp_bytes) {
-    if (c->sort_tmp) (void)hipFree(c->sort_tmp);
-    if (hipMalloc(&c->sort_tmp, bytes) != hipSuccess) {c->sort_tmp = nullptr; return DK_ENOMEM;}
-    c->sort_tmp_bytes = bytes;
-  }
+  if ((e = SortTmpBytes(c, b, n, bytes)) || (e = SortTmp(c, bytes))) return e;
   b.tmp = c->sort_tmp;
   b.tmp_bytes = bytes;
   return SortInto(c, b, n, true);
@@ -2261,13 +2263,25 @@ int SortScratch(dk_ctx *c, long long n) {
     if (p) (void)hipFree(p);
   c->sort_keys = nullptr; c->sort_idx = nullptr; c->sort_rbuf = nullptr;
   c->sort_ibuf = nullptr;
-  if (hipMalloc((void**)&c->sort_keys, sizeof(unsigned long long)*2*n) != hipSuccess ||
-      hipMalloc((void**)&c->sort_idx, sizeof(int)*2*n) != hipSuccess ||
-      hipMalloc((void**)&c->sort_rbuf, sizeof(double)*DK_NRDATA*n) != hipSuccess ||
-      hipMalloc((void**)&c->sort_ibuf, sizeof(int32_t)*DK_NIDATA*n) != hipSuccess)
-    return DK_ENOMEM;
+  c->sort_cap = 0;
+  int e;
+  if ((e = dk::DeviceAlloc(c, (void**)&c->sort_keys, sizeof(unsigned long long)*2*n)) ||
+      (e = dk::DeviceAlloc(c, (void**)&c->sort_idx, sizeof(int)*2*n)) ||
+      (e = dk::DeviceAlloc(c, (void**)&c->sort_rbuf, sizeof(double)*DK_NRDATA*n)) ||
+      (e = dk::DeviceAlloc(c, (void**)&c->sort_ibuf, sizeof(int32_t)*DK_NIDATA*n)))
+    return e;
   c->sort_cap = n;
   return DK_OK;
+}
+
+// the temporary storage of the sort's and the compaction's library calls
+int SortTmp(dk_ctx *c, size_t bytes) {
+  if (bytes <= c->sort_tmp_bytes) return DK_OK;
+  if (c->sort_tmp) (void)hipFree(c->sort_tmp);
+  c->sort_tmp_bytes = 0;
+  const int e = dk::DeviceAlloc(c, &c->sort_tmp, bytes);
+  if (!e) c->sort_tmp_bytes = bytes;
+  return e;
 }
 
 // the caller's particle columns without the particles of zero mass, in order; c->np updated
@@ -2282,11 +2296,7 @@ int CompactMassless(dk_ctx *c) {
   if ((e = dk::Check(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, flag, pos, (int)n,
                                                       c->stream))))
     return e;
-  if (bytes > c->sort_tmp_bytes) {
-    if (c->sort_tmp) (void)hipFree(c->sort_tmp);
-    if (hipMalloc(&c->sort_tmp, bytes) != hipSuccess) {c->sort_tmp = nullptr; return DK_ENOMEM;}
-    c->sort_tmp_bytes = bytes;
-  }
+  if ((e = SortTmp(c, bytes))) return e;
   if ((e = dk::Check(hipcub::DeviceScan::ExclusiveSum(c->sort_tmp, bytes, flag, pos, (int)n,
                                                       c->stream))))
     return e;

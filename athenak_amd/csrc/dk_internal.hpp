@@ -194,6 +194,9 @@ namespace dk {
 int Check(hipError_t e);
 long long NCells(const dk_ctx *c);   // nmb * ncb
 int Zero(dk_ctx *c, double *a, long long n);
+// device memory for what a call needs after particles are bound: where it is short, the tile passes'
+// workspaces make room (*p null and DK_ENOMEM when that is not enough)
+int DeviceAlloc(dk_ctx *c, void **p, size_t bytes);
 
 // dk_mesh.hip: ghost fill (copy, shear remap, x3 values) and additive ghost fold
 template <typename T> int FillGhostsT(dk_ctx *c, T *a, int nvar, bool velocity, double t);
@@ -213,6 +216,8 @@ void ProfDestroy(dk_ctx *c);
 int T64Reserve(dk_ctx *c);
 void T64Destroy(dk_ctx *c);
 bool T64Use(const dk_ctx *c);
+// the workspaces given back (false: there are none, or a graph that the caller captured holds them)
+bool T64Yield(dk_ctx *c);
 int T64Hold(dk_ctx *c, double sh);
 bool T64Held(const dk_ctx *c);
 void T64Release(dk_ctx *c);

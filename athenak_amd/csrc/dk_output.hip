@@ -503,7 +503,7 @@ int dk_particle_history(dk_ctx *c, double time, double stiff_thresh, double row[
   double sums[kSums] = {0, 0, 0, 0, 0, 0, 0};
   if (nchunk > 0) {
     double *part = nullptr;
-    if ((e = Hip(hipMalloc(&part, sizeof(double)*kSums*nchunk)))) return e;
+    if ((e = dk::DeviceAlloc(c, (void**)&part, sizeof(double)*kSums*nchunk))) return e;
     k_phst_chunks<<<(nchunk + kThreads - 1)/kThreads, kThreads, 0, c->stream>>>(
         c->rdata, (long long)c->cap, np, nchunk, part);
     std::vector<double> ph((size_t)kSums*nchunk);
@@ -527,7 +527,7 @@ int dk_particle_history(dk_ctx *c, double time, double stiff_thresh, double row[
     double *f = nullptr, *part = nullptr;
     int *bad = nullptr;
     const int nblk = 1024;
-    if ((e = Hip(hipMalloc(&f, sizeof(double)*ntot)))) return e;
+    if ((e = dk::DeviceAlloc(c, (void**)&f, sizeof(double)*ntot))) return e;
     e = Hip(hipMalloc(&part, sizeof(double)*2*nblk));
     if (!e) e = Hip(hipMalloc(&bad, sizeof(int)));
     if (!e) e = Hip(hipMemsetAsync(f, 0, sizeof(double)*ntot, c->stream));

@@ -885,6 +885,15 @@ void T64Destroy(dk_ctx *c) {
   c->t64 = nullptr;
 }
 
+bool T64Yield(dk_ctx *c) {
+  if (c->t64 == nullptr || c->t64->bins || CallerCaptures(c)) return false;
+  for (const Bins64 *b = c->t64->b; b != nullptr; b = b->prev)
+    if (b->captured) return false;
+  (void)hipStreamSynchronize(c->stream);
+  T64Destroy(c);
+  return true;
+}
+
 bool T64Use(const dk_ctx *c) {
   return c->t64 != nullptr && c->t64->b != nullptr && c->t64->b->cap >= c->np && Pays(c, c->t64->T);
 }

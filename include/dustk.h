@@ -184,7 +184,9 @@ int dk_destroy(dk_ctx *ctx);
  * cells) reserves their workspaces: once per context 90 bytes a cell (120 in the shearing box) and,
  * whenever capacity exceeds every earlier one, 12 bytes a particle of capacity, for which it waits
  * for the stream; other binds neither allocate nor wait.  Where device memory does not suffice the
- * call succeeds and the stages run on per-particle kernels, 10 to 30 times as slow.  Graphs that
+ * call succeeds and the stages run on per-particle kernels, 10 to 30 times as slow; they do so too,
+ * up to the next bind, after a call (a sort, an output) that found no other memory than the
+ * workspaces'.  Graphs that
  * the caller captured of this form's calls stay valid over later binds, until the context ends. */
 int dk_bind_particles(dk_ctx *ctx, double *rdata, int32_t *idata, int64_t capacity,
                       int64_t npart);

@@ -170,3 +170,44 @@ def test_a_count_that_grows_within_the_arrays_allocates_once():
         assert np.abs((d1[0:3] + d1[3:6]) - (d0[0:3] + d0[3:6])).max() < 1e-13 * d0[8]
     g.check_device_error()
     g.close()
+
+
+def test_the_sort_takes_the_workspaces_where_memory_is_short():
+    # 128^3 cells and a million particles: the workspaces take 200 MB, the sort 180 MB and more;
+    # half of that is left over when it is called
+    import torch
+    w = workloads.c1(n=128, nb=2)
+    n = 1 << 20
+    p = Particles(w, n, 5)
+    u = torch.zeros((8, 4, 68, 68, 68), dtype=torch.float64, device="cuda")
+    u[:, 0] = 1.0
+    want = eager(w, u, p)
+    p.reset()
+    torch.cuda.empty_cache()
+    g = context(w, u)
+    bind(g, p)
+    g.prof(True)
+    filler = []
+    for _ in range(6):                  # (torch gives its cached blocks back when it runs short)
+        room = free_bytes() - 90 * n
+        if room > 1 << 20:
+            filler.append(torch.empty(room, dtype=torch.uint8, device="cuda"))
+    assert free_bytes() < 180 * n
+    g.sort()
+    g.step(w.dt, w.src)
+    torch.cuda.synchronize()
+    del filler
+    torch.cuda.empty_cache()
+    assert "bins" not in g.prof_read()
+    # every particle as the tile passes advance it, in the order of the start's blocks and cells
+    i0, r0 = p.i0.cpu().numpy(), p.r0.cpu().numpy()
+    c = [(r0[2 * d] * 128).astype(np.int64) % 64 for d in range(3)]
+    order = np.argsort((i0[abi.PGID] * 64 + c[2]) * 4096 + c[1] * 64 + c[0], kind="stable")
+    np.testing.assert_array_equal(p.i[abi.PTAG].cpu().numpy(), order)
+    o = torch.from_numpy(order).cuda()
+    agree((p.r, p.i, g.u0), (want[0][:, o], want[1][:, o], want[2]))
+    bind(g, p)                          # (the next bind reserves them again)
+    g.prof_reset()
+    g.step(w.dt, w.src)
+    assert "bins" in g.prof_read()
+    g.close()
