@@ -660,7 +660,9 @@ __global__ void __launch_bounds__(kBlock) k_center_mass(Geo g, const DevBlock *B
       }
     }
     // runs of lanes with one target: the first lane of this lane's run, its sum at the last one
-    const unsigned long long heads = __ballot(lane == 0 || __shfl_up(at, 1, 64) != at);
+    // (the shuffle on its own: behind the || lane 0 would be switched off, whose value lane 1 reads)
+    const long long before = __shfl_up(at, 1, 64);
+    const unsigned long long heads = __ballot(lane == 0 || before != at);
     const int first = 63 - __clzll(static_cast<long long>(heads & (~0ull >> (63 - lane))));
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
