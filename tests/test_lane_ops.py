@@ -15,14 +15,20 @@ EXCHANGE = re.compile(r"\b(__shfl\w*|__ballot|__any|__all|WaveScan|WaveInclScan|
                       r"__builtin_amdgcn_(ds_bpermute|readlane|readfirstlane|update_dpp|mov_dpp))\(")
 
 
+def open_part(text):
+    """text without its closed parentheses: what still encloses its end."""
+    while True:
+        cut = re.sub(r"\([^()]*\)", " ", text)
+        if cut == text:
+            return text
+        text = cut
+
+
 def offending(text):
     text = re.sub(r"//[^\n]*|/\*.*?\*/", " ", text, flags=re.S)
-    out = []
-    for statement in re.split(r"[;{}]", text):
-        if any(re.search(r"\|\||&&|\?", statement[:m.start()])
-               for m in EXCHANGE.finditer(statement)):
-            out.append(" ".join(statement.split()))
-    return out
+    return [" ".join(statement.split()) for statement in re.split(r"[;{}]", text)
+            if any(re.search(r"\|\||&&|\?", open_part(statement[:m.start()]))
+                   for m in EXCHANGE.finditer(statement))]
 
 
 @pytest.mark.parametrize("path", FILES, ids=os.path.basename)
@@ -35,3 +41,4 @@ def test_the_check_sees_one():
     assert offending("const bool head = lane == 0 || __shfl_up(at, 1, 64) != at;")
     assert offending("heads = __ballot(lane == 0 || __shfl_up(at, 1, 64) != at);")
     assert not offending("const long long prev = __shfl_up(at, 1, 64); f(lane == 0 || prev != at);")
+    assert not offending("const int a = WaveScan(on ? n : 0), e = WaveScan((on && n) ? 1 : 0);")
