@@ -12,6 +12,7 @@ SOURCES = ["dk_fp64.hip", "dk_fp32.hip", "dk_setup.hip", "dk_prof.hip", "dk_mesh
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # -ffp-contract=off: no fused multiply-adds, so that the FP64 form rounds as the oracle does
+# (dk_tile64.hip turns them off itself, except in its sums over particles)
 COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 PER_FILE = {"dk_fp64.hip": ["-ffp-contract=off"], "dk_setup.hip": ["-ffp-contract=off"],

@@ -18,6 +18,11 @@
 //
 // The order of a cell's additions is not fixed (as with the per-particle atomics).
 //
+// Fused multiply-adds only in the sums of the records (step 4, where they pay: without them the
+// passes take 10 % longer): what a particle gathers and what becomes of it is rounded as on the
+// per-particle kernels and in the reference's operation order, so that a particle's path does not
+// depend on which kernels its deposit runs on (3 % of the gathering passes).
+//
 // Measured, per launch, per-particle kernels -> tile kernels with their combine: 8.4 million
 // particles on 128^3 cells (shearing box), deposit of Q, P 33.5 -> 0.50 ms, operator 25.6 -> 0.55,
 // kick 25.8 -> 0.73, the bins of a stage 0.14 ms; 2.1 million, half of them in clumps, 11.7 ->
@@ -160,6 +165,7 @@ __device__ inline int TileOf(const Geo &g, const Grid64 &T, const Place &L) {
 }
 
 __device__ inline void Weights(int scheme, double d, double w[3]) {
+#pragma clang fp contract(off)
   if (scheme == 2) {
     const double h0 = 0.5 - d, h2 = 0.5 + d;
     w[0] = 0.5*h0*h0; w[1] = 0.75 - d*d; w[2] = 0.5*h2*h2;
@@ -294,6 +300,7 @@ __device__ inline void FarDeposit(const Args64 &A, int m, const Stencil &w, cons
 
 template <int OP>
 __device__ inline void FarGather(const Args64 &A, int m, const Stencil &w, double u[3]) {
+#pragma clang fp contract(off)
   constexpr int nv = (OP == kPredict) ? DK_NGAS : 3;
   for (int d=0; d<3; ++d) u[d] = 0.0;
   for (int c=0; c<3; ++c)
@@ -329,6 +336,7 @@ __device__ inline double Share(double fac, double x) { return (fac == 0.0) ? 0.0
 template <int OP>
 __device__ inline void Work(const Args64 &A, const DevBlock &b, long long p, const double u[3],
                             double *val) {
+#pragma clang fp contract(off)
   double *r = A.r;
   const long long cap = A.cap;
   const double ts = r[(long long)DK_IPTS*cap + p], mass = r[(long long)DK_IPM*cap + p];
@@ -363,12 +371,9 @@ __device__ inline void Work(const Args64 &A, const DevBlock &b, long long p, con
       v0[d] = r[(long long)(DK_IPVX1 + 2*d)*cap + p];
       rr[d] = v0[d] + lambda*u[d];
     }
-    {
-#pragma clang fp contract(off)
-      xh[0] = x0[0] + 0.5*dt*v0[0];
-      xh[1] = x0[1] + 0.5*dt*(v0[1] - (A.sbox ? A.qs*A.om*x0[0] : 0.0));
-      xh[2] = x0[2] + 0.5*dt*v0[2];
-    }
+    xh[0] = x0[0] + 0.5*dt*v0[0];
+    xh[1] = x0[1] + 0.5*dt*(v0[1] - (A.sbox ? A.qs*A.om*x0[0] : 0.0));
+    xh[2] = x0[2] + 0.5*dt*v0[2];
     if (A.sbox) {
       const double cxy = 2.0*h*A.om, cyx = h*(2.0 - A.qs)*A.om, det = aa*aa + cxy*cyx;
       vh[0] = (aa*rr[0] + cxy*rr[1])/det;
@@ -518,6 +523,7 @@ __global__ void __launch_bounds__(kNT, 3) k_t64(Args64 A) {
       }
       if constexpr (Gathers<OP>()) {
         if (!far) {
+#pragma clang fp contract(off)
           double wx[3], wy[3], wz[3];
           Weights(g.deposit, L[k].dx, wx);
           Weights(g.deposit, L[k].dy, wy);
