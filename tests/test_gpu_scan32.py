@@ -1,0 +1,73 @@
+"""The FP32 form's scans where a workgroup takes several rounds, the last one ragged: 272 x 264 x 240
+cells (17.2 million keys, 16.8 million being the most of one round) in tiles of 4 x 2 x 2 (1.1
+million tiles, 1.05 million being the most of one round of the item lists).  The first slots of all
+keys and the permutation against numpy, and the run against the FP64 form: velocities and gas
+momenta within 1e-5 of the largest (as in test_gpu_fp32.py)."""
+
+import os
+
+import numpy as np
+import pytest
+
+from athenak_amd import abi, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def test_scans_of_several_rounds():
+    import torch
+    from athenak_amd.lib import DustContext
+    nx, nb, n, dt, steps = (68, 66, 60), (4, 4, 4), 1500000, 8e-3, 2
+    mesh, blocks = abi.uniform_mesh(nx, nb, ((0.0, 1.0),) * 3, ng=2)
+    phys = workloads._phys()
+    rng = np.random.default_rng(4)
+    x = rng.random((3, n))
+    r = np.zeros((abi.DK_NRDATA, n))
+    iv = np.zeros((abi.DK_NIDATA, n), dtype=np.int32)
+    for d in range(3):
+        r[2 * d], r[2 * d + 1] = x[d], 0.2 * rng.standard_normal(n)
+    r[abi.IPTS], r[abi.IPM] = 10.0 ** rng.uniform(-2, 0, n), 0.5 / n
+    b = [(x[d] * nb[d]).astype(np.int32) for d in range(3)]
+    iv[abi.PGID] = b[0] + nb[0] * (b[1] + nb[1] * b[2])
+    iv[abi.PTAG] = np.arange(n)
+    out = {}
+    for form in (abi.DK_FORM_FP64, abi.DK_FORM_FP32):
+        os.environ["DK_TILE"] = "4x2x2"
+        try:
+            g = DustContext(mesh, blocks, phys, n, form=form)
+        finally:
+            del os.environ["DK_TILE"]
+        g.rdata.copy_(torch.from_numpy(r))
+        g.idata.copy_(torch.from_numpy(iv))
+        gen = torch.Generator(device="cuda").manual_seed(8)
+        g.u0[:, 1:] = 0.2 * torch.randn(g.u0[:, 1:].shape, dtype=torch.float64, device="cuda",
+                                        generator=gen)
+        g.u0[:, 0] = 1.0
+        g.u1.copy_(g.u0)
+        torch.cuda.synchronize()
+        g.bind_particles(n)
+        g.task("fill_gas_ghosts", abi.imex2p_stages(0.0, 0.0)[0])
+        for _ in range(steps):
+            g.step(dt)
+        if form == abi.DK_FORM_FP32:
+            key, perm, start = g.sort_state()
+            nk = start.size - 1
+            assert nk == 272 * 264 * 240
+            count = np.bincount(key, minlength=nk)
+            np.testing.assert_array_equal(start, np.concatenate([[0], np.cumsum(count)]))
+            np.testing.assert_array_equal(np.bincount(perm, minlength=n), 1)
+            assert (np.diff(key[perm]) >= 0).all()
+        g.export()
+        o = torch.argsort(g.idata[abi.PTAG])
+        v = g.rdata[[abi.IPVX, abi.IPVY, abi.IPVZ]][:, o].cpu()
+        p = g.rdata[[abi.IPX, abi.IPY, abi.IPZ]][:, o].cpu()
+        out[form] = v, p, g.u0[:, 1:, 2:-2, 2:-2, 2:-2].cpu()
+        g.check_device_error()
+        g.close()
+    a, c = out[abi.DK_FORM_FP64], out[abi.DK_FORM_FP32]
+    vmax = float(a[0].abs().max())
+    errs = (float((a[0] - c[0]).abs().max()) / vmax, float((a[2] - c[2]).abs().max() /
+                                                          a[2].abs().max()),
+            float((a[1] - c[1]).abs().max()) / (vmax * dt * steps))
+    print("[gpu-scan32] velocity %.2e, gas %.2e, position %.2e" % errs, flush=True)
+    assert max(errs) < 1e-5, errs
