@@ -305,12 +305,9 @@ __global__ void __launch_bounds__(kBlock) k_fold(Geo g, const DevBlock *B, const
   const int m = blockIdx.y;
   if (threadIdx.x < 26) sdir[threadIdx.x] = slot_dir[threadIdx.x];
   if (threadIdx.x < 27) {
-    // (on a refined mesh only same-level neighbours fold: no deposit of the FP32 tile kernels
-    // reaches a region of another level, whose clouds go to the leaf traversal)
     const int d = threadIdx.x, o1 = d % 3;
     const DevBlock &bm = B[m];
     int nb = bm.nghbr[d];
-    if (nb >= 0 && B[nb].level != bm.level) nb = -1;
     if (g.bc_x1 == DK_X1_SHEAR &&
         ((o1 == 0 && bm.lx1 == 0) || (o1 == 2 && bm.lx1 == g.nmbx1 - 1)))
       nb = -1;
@@ -506,6 +503,5 @@ int FoldT(dk_ctx *c, T *a, int nvar, double t) {
 template int FillGhostsT<double>(dk_ctx *, double *, int, bool, double);
 template int FillGhostsT<float>(dk_ctx *, float *, int, bool, double);
 template int FoldT<double>(dk_ctx *, double *, int, double);
-template int FoldT<float>(dk_ctx *, float *, int, double);
 
 }  // namespace dk

@@ -77,7 +77,7 @@ template <int OP> constexpr bool Gathers() { return OP != kScatter; }
 struct Grid64 {
   int ntx, nty, ntz, ntb, nt, SY;
   int RX, RY, RZ, RN;
-  float iRX, iRY, iRN;
+  float iRX, iRY;
 };
 
 struct Args64 {
@@ -775,7 +775,7 @@ Grid64 MakeGrid(const dk_ctx *c) {
   T.nt = static_cast<int>(std::min<long long>((long long)T.ntb*g.nmb, INT32_MAX));
   T.RX = kTX + 2; T.RY = kTY + 2 + 2*T.SY; T.RZ = kTZ + 2;
   T.RN = T.RX*T.RY*T.RZ;
-  T.iRX = 1.0f/T.RX; T.iRY = 1.0f/T.RY; T.iRN = 1.0f/T.RN;
+  T.iRX = 1.0f/T.RX; T.iRY = 1.0f/T.RY;
   return T;
 }
 
