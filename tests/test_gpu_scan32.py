@@ -2,7 +2,13 @@
 cells (17.2 million keys, 16.8 million being the most of one round) in tiles of 4 x 2 x 2 (1.1
 million tiles, 1.05 million being the most of one round of the item lists).  The first slots of all
 keys and the permutation against numpy, and the run against the FP64 form: velocities and gas
-momenta within 1e-5 of the largest (as in test_gpu_fp32.py)."""
+momenta within 1e-5 of the largest (as in test_gpu_fp32.py).
+
+The consistent split gives a particle the residual of the cell that holds it, which jumps at the
+cells' faces: a particle whose positions in the two forms, 1e-8 of a cell apart, lie on either side
+of a face takes another cell's residual (one of these 1.5 million does, 3e-10 and -7e-9 of a cell
+from an x2 face, and differs by 2.6e-3).  Such particles, at most 3, and the cells on either side of
+their faces are not compared."""
 
 import os
 
@@ -65,9 +71,19 @@ def test_scans_of_several_rounds():
         g.check_device_error()
         g.close()
     a, c = out[abi.DK_FORM_FP64], out[abi.DK_FORM_FP32]
+    N = torch.tensor([nx[d] * nb[d] for d in range(3)])[:, None]
+    ca, cc = (a[1] * N).floor().long(), (c[1] * N).floor().long()
+    split = (ca != cc).any(0)
+    assert int(split.sum()) <= 3
+    cells = torch.ones(a[2][:, 0].shape, dtype=torch.bool)
+    for q in torch.nonzero(split)[:, 0].tolist():
+        for x in (ca[:, q].tolist(), cc[:, q].tolist()):
+            m = x[0] // nx[0] + nb[0] * (x[1] // nx[1] + nb[1] * (x[2] // nx[2]))
+            cells[m, x[2] % nx[2], x[1] % nx[1], x[0] % nx[0]] = False
     vmax = float(a[0].abs().max())
-    errs = (float((a[0] - c[0]).abs().max()) / vmax, float((a[2] - c[2]).abs().max() /
-                                                          a[2].abs().max()),
+    errs = (float((a[0] - c[0])[:, ~split].abs().max()) / vmax,
+            float(((a[2] - c[2]).abs().amax(1) * cells).max() / a[2].abs().max()),
             float((a[1] - c[1]).abs().max()) / (vmax * dt * steps))
-    print("[gpu-scan32] velocity %.2e, gas %.2e, position %.2e" % errs, flush=True)
+    print("[gpu-scan32] velocity %.2e, gas %.2e, position %.2e; %d on a face" %
+          (errs + (int(split.sum()),)), flush=True)
     assert max(errs) < 1e-5, errs
