@@ -365,10 +365,12 @@ def cpu_baseline(name, budget_s):
 # known size) of the workload's FP32 run, committed under profiles/ as hbm_traffic_<name>_fp32.md.
 # A timer label covers one launch of every kernel of a group (a tile kernel is two launches: its
 # first items and its extra parts); labels with two groups (P3 with and without the stage-2 rate
-# store) take their mean.
+# store) take their mean.  (The key pass: its variants that push, not those of a pending correction
+# alone.)
 PROFILES = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles")
 TRAFFIC_KERNEL = {"p1_gather_deposit": [["k_p1<"]], "p2_operator": [["k_p2<"]],
-                  "p3_gather_kick": [["k_p3<"], ["k_p3n<"]], "key": [["k_key<"]]}
+                  "p3_gather_kick": [["k_p3<"], ["k_p3n<"]],
+                  "key": [["k_key<false, false, false, true>", "k_key<true, false, false, true>"]]}
 
 
 def measured_traffic(label, w, form):
