@@ -2631,11 +2631,10 @@ k_pa(KArgs A, const float *us, float *scr, double *defect, const DevBlock *__res
 // src/dust/dust_leaf3d.hpp:383-517, as the FP64 form walks them) with each leaf cell's own
 // volume; the arithmetic of the particle is the tile kernels'.  Their deposits are atomic
 // additions into the folded fields, so the order of these additions (and the last bits of the
-// cells they touch) is not fixed.  A launch has a thread per particle of the store (up to the
-// grid limit; the threads beyond the list's length exit at once): each cloud's walk is a chain
-// of dependent loads, which only many threads in flight hide.  The walk would take 336 registers
-// (one wavefront per SIMD); a bound of 3 wavefronts per SIMD spills some of them and runs
-// C4's cross-level clouds 12 % faster (2 and 4: 11 % and 8 %).
+// cells they touch) is not fixed.  kCoop lanes take a cloud's leaf cells and a group takes a run of
+// clouds (dk_cloudwalk.hpp says why and what both measured); the list's length is known on the
+// device only, so the grid is sized for all particles of the store, up to the grid limit, and the
+// groups beyond the list leave at once.
 
 // a group of lanes per cross-level cloud of the list (dk_cloudwalk.hpp)
 constexpr int kCoop = dk::kCoop;
@@ -3297,7 +3296,9 @@ __global__ void __launch_bounds__(kBlock) k_fold_cells(Regions R, Shell S, TO *o
 // The cells of the shear-periodic x1 faces: the ghost deposits beyond the opposite face, moved in
 // x2 by shc cells and split between the two cells they overlap (src/bvals/bvals_dep_general.cpp:
 // 100-160, as a gather over the source cells that can reach the target: the order and the shares
-// of the fold of a padded field, dk_mesh.hip), then the cell pass.
+// of the fold of a padded field, dk_mesh.hip), then the cell pass.  Each candidate's tile regions
+// are summed anew, which no padded field holds any more: 90 to 114 us a launch at 256^3 cells, where
+// the fold of a padded field took 33, against 10 % less for the folds and cell passes together.
 template <int NV, typename TO, class Op>
 __global__ void __launch_bounds__(kBlock) k_fold_shear_cells(Regions R, const TO *out, double shc,
                                                              Op op) {

@@ -24,10 +24,10 @@
 // depend on which kernels its deposit runs on (3 % of the gathering passes).
 //
 // Measured, per launch, per-particle kernels -> tile kernels with their combine: 8.4 million
-// particles on 128^3 cells (shearing box), deposit of Q, P 33.5 -> 0.50 ms, operator 25.6 -> 0.55,
-// kick 25.8 -> 0.73, the bins of a stage 0.14 ms; 2.1 million, half of them in clumps, 11.7 ->
-// 0.14, 8.8 -> 0.15, 8.9 -> 0.18 ms; pc2 predictor and advance of 1 million in uneven blocks
-// 5.5 -> 0.18 and 4.3 -> 0.14 ms.
+// particles on 128^3 cells (shearing box), deposit of Q, P 33.5 -> 0.51 ms, operator 25.6 -> 0.58,
+// kick 25.8 -> 0.69, the bins of a stage 0.12 ms; 2.1 million, half of them in clumps, 11.7 ->
+// 0.15, 8.8 -> 0.16, 8.9 -> 0.18 ms; pc2 predictor and advance of 1 million in uneven blocks
+// 5.5 -> 0.17 and 4.3 -> 0.15 ms.
 
 #include <hip/hip_runtime.h>
 
@@ -52,8 +52,9 @@ constexpr int kTX = 8, kTY = 4, kTZ = 4, kTC = kTX*kTY*kTZ;   // cells of a tile
 // 0.47, kick 0.84 -> 0.65 ms)
 constexpr int kNT = 256;
 // particles of a chunk: 512, the mean of a tile at 4 particles per cell, and three standard
-// deviations of a random filling, so that such a tile is one chunk; the records of 576 keep
-// three workgroups on a CU (52 KB of LDS each)
+// deviations of a random filling, so that such a tile is one chunk; with the records of 576 a
+// workgroup takes 45 to 47 KB of LDS (50 to 53 KB in the shearing box), three on a CU.  (The pc2
+// predictor, with a gathered field and four components, takes 55 and 62 KB: two.)
 constexpr int kChunk = 576;
 constexpr int kPer = (kChunk + kNT - 1)/kNT;
 constexpr int kItemMax = 2*kChunk;

@@ -55,8 +55,8 @@ enum { DK_X3_PERIODIC = 0, DK_X3_REFLECT = 1, DK_X3_OUTFLOW = 2 };
 
 /* execution forms of a context */
 enum {
-  DK_FORM_FP64 = 0,   /* plain FP64: one kernel per reference kernel, atomic deposits,
-                         operating directly on the caller's arrays */
+  DK_FORM_FP64 = 0,   /* plain FP64, operating directly on the caller's arrays: one pass per
+                         reference kernel, deposits summed tile by tile and added with atomics */
   DK_FORM_FP32 = 1    /* FP32 bulk, FP64 positions and sums: cell-sorted particles,
                          atomic-free deposits, fused stage passes (dk_stage_run only).
                          imex with local/dc1/dc2 on any mesh of the FP64 form; pc2 with
