@@ -705,12 +705,20 @@ namespace {
 // the caller is capturing the context's stream (the library's own stage graphs, which are captured
 // anew before every launch, apart)
 bool CallerCaptures(const dk_ctx *c) {
-  if (c->stream == nullptr || c->own_capture) return false;
+  if (c->own_capture) return false;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(c->stream, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
   (void)hipGetLastError();
   return true;
 }
+
+// While another stream is captured, in any mode but the relaxed one, this thread's allocations and
+// waits would be refused and end that capture; they are no part of it.
+struct Relaxed {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
 
 // one allocation (null: short of device memory, and then the per-particle kernels run)
 void *Mem(size_t bytes) {
@@ -738,7 +746,7 @@ template <int OP>
 int Bin(dk_ctx *c, const Args64 &A) {
   Tile64 *w = c->t64;
   Bins64 *b = w->b;
-  if (CallerCaptures(c)) b->captured = true;
+  if (c->stream != nullptr && CallerCaptures(c)) b->captured = true;
   const int pt = ProfBegin(c, "bins");
   k_t64_count<OP><<<Grid(c->np), kBlock, 0, c->stream>>>(A, b->key, b->rank, w->count);
   k_t64_scan<<<1, kScanThreads, 0, c->stream>>>(w->T.nt, w->count, w->start, b->item_tile,
@@ -847,6 +855,7 @@ int T64Reserve(dk_ctx *c) {
   if (old != nullptr && old->cap >= c->np) return DK_OK;
   if (CallerCaptures(c))
     return DK_OK;   // (no allocation inside the caller's capture: the per-particle kernels run)
+  const Relaxed relaxed;
   const bool first = c->t64 == nullptr;
   if (!ReserveMesh(c, T)) return DK_OK;
   Tile64 *w = c->t64;

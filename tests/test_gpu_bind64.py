@@ -211,3 +211,37 @@ def test_the_sort_takes_the_workspaces_where_memory_is_short():
     g.step(w.dt, w.src)
     assert "bins" in g.prof_read()
     g.close()
+
+
+@pytest.mark.parametrize("mode", ["global", "thread_local", "relaxed"])
+@pytest.mark.parametrize("own_stream", [True, False])
+def test_a_bind_while_another_stream_is_captured(mode, own_stream):
+    # a bind does no work of the captured program's: the capture goes on, and the bound particles
+    # have their tile passes
+    import torch
+    from athenak_amd.lib import DustContext
+    w, u = workload()
+    small, p = Particles(w, 2000, 6), Particles(w, 6000, 7)
+    want = eager(w, u, p)
+    p.reset()
+    g = context(w, u) if own_stream else DustContext(w.mesh, w.blocks, w.phys, 1)
+    g.u0.copy_(u)
+    g.u1.copy_(u)
+    torch.cuda.synchronize()
+    bind(g, small)
+    x = torch.zeros(1000, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(), capture_error_mode=mode):
+        x.add_(1.0)
+        bind(g, p)                      # (larger than the first: it needs other workspaces)
+        x.add_(1.0)
+    for _ in range(3):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert bool((x == 6.0).all())
+    g.prof(True)
+    g.step(w.dt, w.src)
+    torch.cuda.synchronize()
+    assert "bins" in g.prof_read()
+    agree((p.r, p.i, g.u0), want)
+    g.close()
