@@ -679,7 +679,7 @@ __global__ void __launch_bounds__(kBlock) k_t64_combine(Geo g, Grid64 T, const d
 // the workspaces of the present particles: the items and every particle's tile, place and slot
 struct Bins64 {
   int *item_tile = nullptr, *item_part = nullptr, *key = nullptr, *rank = nullptr, *perm = nullptr;
-  void *mem = nullptr;      // the one allocation that holds them
+  void *mem = nullptr;      // the one allocation that holds them (null: Tile64's, the first ones)
   long long cap = 0;        // particles they hold
   // A graph that the caller captured holds them: they stay until the context ends, also when more
   // particles are bound, so that the graph may be replayed as before (its particles and the
@@ -688,7 +688,8 @@ struct Bins64 {
   Bins64 *prev = nullptr;
 };
 
-// the workspaces of a context's tile passes; those of the mesh are allocated once
+// the workspaces of a context's tile passes; those of the mesh are allocated once, the first
+// particles' with them
 struct Tile64 {
   Grid64 T;
   int *count = nullptr, *start = nullptr, *nitem = nullptr;
@@ -809,34 +810,15 @@ bool Pays(const dk_ctx *c, const Grid64 &T) {
   return c->np*16 >= (long long)c->g.nmb*c->g.nx1*c->g.nx2*c->g.nx3 && c->np >= a_tile*T.nt;
 }
 
-// the mesh's part of the workspaces (false: the per-particle kernels run)
-bool ReserveMesh(dk_ctx *c, const Grid64 &T) {
-  if (c->t64 != nullptr) return true;
-  const long long nt = T.nt;
-  if (nt >= (1LL << 29)) return false;   // (32-bit items)
-  // the scratch, then the int arrays
-  const size_t nscr = 4*(size_t)T.RN*nt;
-  void *mem = Mem(sizeof(double)*nscr + sizeof(int)*(2*(size_t)(nt + 1) + 1));
-  if (mem == nullptr) return false;
-  Tile64 *w = new Tile64();
-  w->T = T;
-  w->mem = mem;
-  w->scr = static_cast<double*>(mem);
-  w->count = reinterpret_cast<int*>(w->scr + nscr);
-  w->start = w->count + nt + 1;
-  w->nitem = w->start + nt + 1;
-  c->t64 = w;
-  return true;
+// the particles' part of the workspaces, for n of them: its ints, and its place at p
+size_t BinsInts(const Grid64 &T, long long n) {
+  return 2*static_cast<size_t>(T.nt + n/kItemMax + 1) + 3*static_cast<size_t>(n);
 }
 
-// the particles' part, for n of them
-Bins64 *NewBins(const Grid64 &T, long long n) {
+Bins64 *MakeBins(const Grid64 &T, long long n, int *p) {
   const size_t items = static_cast<size_t>(T.nt + n/kItemMax + 1);
-  void *mem = Mem(sizeof(int)*(2*items + 3*static_cast<size_t>(n)));
-  if (mem == nullptr) return nullptr;
   Bins64 *b = new Bins64();
-  b->mem = mem;
-  b->item_tile = static_cast<int*>(mem);
+  b->item_tile = p;
   b->item_part = b->item_tile + items;
   b->key = b->item_part + items;
   b->rank = b->key + n;
@@ -845,43 +827,62 @@ Bins64 *NewBins(const Grid64 &T, long long n) {
   return b;
 }
 
+// the mesh's part with the first particles', for n of them, in one allocation (two take 0.3 ms more
+// of a small program's start); false: short of device memory
+bool First(dk_ctx *c, const Grid64 &T, long long n) {
+  const long long nt = T.nt;
+  // the scratch, then the int arrays
+  const size_t nscr = 4*(size_t)T.RN*nt, nmesh = 2*(size_t)(nt + 1) + 1;
+  void *mem = Mem(sizeof(double)*nscr + sizeof(int)*(nmesh + BinsInts(T, n)));
+  if (mem == nullptr) return false;
+  Tile64 *w = new Tile64();
+  w->T = T;
+  w->mem = mem;
+  w->scr = static_cast<double*>(mem);
+  w->count = reinterpret_cast<int*>(w->scr + nscr);
+  w->start = w->count + nt + 1;
+  w->nitem = w->start + nt + 1;
+  w->b = MakeBins(T, n, w->nitem + 1);
+  c->t64 = w;
+  return true;
+}
+
 }  // namespace
 
 int T64Reserve(dk_ctx *c) {
   if (c->form != DK_FORM_FP64 || c->smr || c->P.clouds || c->g.ng < 2) return DK_OK;
   const Grid64 T = MakeGrid(c);
-  if (!Pays(c, T)) return DK_OK;
-  Bins64 *old = (c->t64 != nullptr) ? c->t64->b : nullptr;
-  if (old != nullptr && old->cap >= c->np) return DK_OK;
+  if (!Pays(c, T) || T.nt >= (1 << 29)) return DK_OK;   // (32-bit items)
+  if (c->t64 != nullptr && c->t64->b->cap >= c->np) return DK_OK;
   if (CallerCaptures(c))
     return DK_OK;   // (no allocation inside the caller's capture: the per-particle kernels run)
   const Relaxed relaxed;
-  const bool first = c->t64 == nullptr;
-  if (!ReserveMesh(c, T)) return DK_OK;
-  Tile64 *w = c->t64;
-  if (first) {
-    const int e = Check(hipMemsetAsync(w->count, 0, sizeof(int)*(T.nt + 1), c->stream));
-    if (e) {
-      T64Destroy(c);
-      return e;
-    }
-  }
   // for as many as the caller's arrays hold, so that a count that grows within them neither
   // allocates nor waits (12 of their 156 bytes a particle)
   long long n = std::min<long long>(c->cap, INT32_MAX);
-  if (old != nullptr && old->captured) {
+  if (c->t64 == nullptr) {
+    if (!First(c, T, n) && !First(c, T, c->np)) return DK_OK;
+    const int e = Check(hipMemsetAsync(c->t64->count, 0, sizeof(int)*(T.nt + 1), c->stream));
+    if (e) T64Destroy(c);
+    return e;
+  }
+  Tile64 *w = c->t64;
+  Bins64 *old = w->b;
+  if (old->captured) {
     // (half as many again as the ones kept, so that what growing arrays leave behind stays below
     // twice what they have)
     n = std::max(n, std::min<long long>(old->cap + old->cap/2, INT32_MAX));
-  } else if (old != nullptr) {
+  } else if (old->mem != nullptr) {
     (void)hipStreamSynchronize(c->stream);
     w->b = old->prev;
     (void)hipFree(old->mem);
     delete old;
   }
-  Bins64 *b = NewBins(T, n);
-  if (b == nullptr && n > c->np) b = NewBins(T, c->np);
-  if (b == nullptr) return DK_OK;
+  void *mem = Mem(sizeof(int)*BinsInts(T, n));
+  if (mem == nullptr && n > c->np) mem = Mem(sizeof(int)*BinsInts(T, n = c->np));
+  if (mem == nullptr) return DK_OK;
+  Bins64 *b = MakeBins(T, n, static_cast<int*>(mem));
+  b->mem = mem;
   b->prev = w->b;
   w->b = b;
   return DK_OK;
@@ -893,7 +894,7 @@ void T64Destroy(dk_ctx *c) {
   while (w->b != nullptr) {
     Bins64 *b = w->b;
     w->b = b->prev;
-    (void)hipFree(b->mem);
+    if (b->mem != nullptr) (void)hipFree(b->mem);
     delete b;
   }
   (void)hipFree(w->mem);
@@ -911,7 +912,7 @@ bool T64Yield(dk_ctx *c) {
 }
 
 bool T64Use(const dk_ctx *c) {
-  return c->t64 != nullptr && c->t64->b != nullptr && c->t64->b->cap >= c->np && Pays(c, c->t64->T);
+  return c->t64 != nullptr && c->t64->b->cap >= c->np && Pays(c, c->t64->T);
 }
 
 int T64Hold(dk_ctx *c, double sh) {
